@@ -102,3 +102,45 @@ def test_training_fits_a_teacher():
     print(losses)
     assert losses[-1] < losses[0] / 20, losses
     L.spdk_mlp_destroy(net)
+
+
+# batches at the edges of the 64-row tiles and of the weight gradient's row
+# steps; the last two fill the chip with 128-wide tiles (layer 3: 19 column
+# tiles of 64, 10 of 128), one of them with a ragged last row tile
+@pytest.mark.parametrize("B", [1, 63, 64, 65, 257, 6656, 6701])
+def test_tiles_match_oracle(B):
+    dims = [70, 64, 128, 1210]
+    rng = np.random.default_rng(B)
+    p = op.mlp_init(dims, seed=9)
+    X, T = rng.standard_normal((B, dims[0])), rng.standard_normal((B, dims[3]))
+    net = make_net(dims, 6701, p)
+    L = spd_k_amd.lib()
+    ldy = dims[3] + 3  # rows longer than the outputs: the tail is left alone
+    Xd, Td, Yd = dev(X), dev(T), torch.full((B, ldy), 7.0, device="cuda:0")
+    spd_k_amd.check(L.spdk_mlp_forward(net, ctypes.c_void_p(Xd.data_ptr()), ctypes.c_long(dims[0]), B,
+                                       ctypes.c_void_p(Yd.data_ptr()), ctypes.c_long(ldy)), "forward")
+    torch.cuda.synchronize()
+    Y = Yd.cpu().double().numpy()
+    ref = op.orc_mlp_forward(dims, p, X, bf16=True)
+    # the bounds of test_forward_matches_oracle (BF16 rounding of the hidden layers)
+    assert np.abs(Y[:, :dims[3]] - ref).max() <= 1e-2 * np.abs(ref).max()
+    assert np.linalg.norm(Y[:, :dims[3]] - ref) <= 2e-3 * np.linalg.norm(ref)
+    assert np.all(Y[:, dims[3]:] == 7.0)
+    g = np.zeros(op.mlp_param_count(dims), dtype=np.float32)
+    loss = ctypes.c_float()
+    spd_k_amd.check(L.spdk_mlp_gradients(net, ctypes.c_void_p(Xd.data_ptr()), ctypes.c_long(dims[0]),
+                                         ctypes.c_void_p(Td.data_ptr()), ctypes.c_long(dims[3]), B,
+                                         g.ctypes.data_as(ctypes.c_void_p), ctypes.byref(loss)), "gradients")
+    ref, ref_loss = op.orc_mlp_grad(dims, p, X, T, bf16=True)
+    o = 0
+    assert abs(loss.value - ref_loss) <= 1e-3 * ref_loss
+    for l in range(3):  # every weight matrix and bias by itself
+        for n in (dims[l + 1] * dims[l], dims[l + 1]):
+            a, b = g[o:o + n].astype(np.float64), ref[o:o + n]
+            assert np.linalg.norm(a - b) <= 2e-2 * np.linalg.norm(b), (l, n)
+            o += n
+    assert L.spdk_mlp_forward(net, ctypes.c_void_p(Xd.data_ptr()), ctypes.c_long(dims[0]), B, None,
+                              ctypes.c_long(ldy)) != 0
+    assert L.spdk_mlp_forward(net, ctypes.c_void_p(Xd.data_ptr()), ctypes.c_long(dims[0]), B,
+                              ctypes.c_void_p(Yd.data_ptr()), ctypes.c_long(dims[3] - 1)) != 0
+    L.spdk_mlp_destroy(net)
