@@ -6,21 +6,23 @@
 // What crosses HBM between launches is the raw edge field E of each element
 // (compute_E's first variable, src/induction.cpp:139-208, before any face
 // solve), FP64, for all time slices. A sweep launch works on a tile of
-// consecutive elements (along x), slice by slice:
-//   A. the tile's raw E of the slice goes to LDS; every edge point gets its
-//      face-solved value from its own raw E and its neighbours' raw E at the
-//      shared faces (from LDS inside the tile, else HBM), upwinded along the
-//      first face axis and then the second, exactly as the in-place
+// consecutive elements (along x), all slices at once:
+//   A. every edge point's face-solved value goes from HBM to LDS: upwinded
+//      along the first face axis and then the second, exactly as the in-place
 //      E_riemann_solver calls do (src/induction.cpp:509-560,
-//      src/induction_ader.hpp:437-448); boundary ghosts are resolved by index
-//      (periodic wrap, gradfree mirror) as the SD trace fill makes them;
-//   B. dB/dt of the slice at every face-B point (the derivative sums of
+//      src/induction_ader.hpp:437-448). The upwind velocity is uniform, so the
+//      solved value is one element's raw value (or, along an axis of zero
+//      velocity, the mean of two) and the face solve is a choice of address;
+//      boundary ghosts are resolved by index (periodic wrap, gradfree mirror)
+//      as the SD trace fill makes them;
+//   B. dB/dt at every face-B point (the derivative sums of
 //      src/induction.cpp:331-356), kept in registers for all slices;
-// then either the corrector into B (last launch, update_B_solution) or, slice
-// by slice, the predictor slice in LDS (update_B_prediction) and its raw E,
-// written for the next launch.
+// then either the corrector into B (last launch, update_B_solution) or the
+// predictor slices in LDS (update_B_prediction) and their raw E, written for
+// the next launch.
 // The zero-order guess makes every slice equal, so the first launch only
-// computes the raw E of B once per point and writes it to every slice.
+// computes the raw E of B, once per point, and the first sweep reads that one
+// slice.
 //
 // The same kernels with R = float are the mixed-precision form: raw E, the
 // face solves, the sp->fp interpolations and the predictor slices in FP32
@@ -38,6 +40,7 @@
 #include <cstring>
 #include <type_traits>
 #include "ctx.hpp"
+#include "physics.hpp"
 
 // Element tiles of the induction sweep in XCD-contiguous order (0: launch order).
 #ifndef SPDK_ISWEEP_XCD
@@ -47,10 +50,6 @@
 using namespace spdk;
 
 namespace {
-
-constexpr int BS = 256;
-constexpr int kMaxT = 5;
-constexpr int kLdsBudget = 40 * 1024;  // bytes of element tiles per workgroup
 
 // Point counts of one configuration: N solution points per active axis; D = 3,
 // or D = 2 with z inactive (one point along z).
@@ -71,60 +70,19 @@ struct IG {
     __host__ __device__ static constexpr int eoff(int e) { return e == 0 ? 0 : (e == 1 ? epts(0) : epts(0) + epts(1)); }
 };
 
+// A workgroup's tile: as many whole elements as its threads cover with one
+// edge point of a component per thread, so that phases A and C run without a
+// loop over points and phase B keeps one face-B point per component and
+// thread (256 threads: 10 elements of 2-D p=3, 250 threads busy; the 100 edge
+// points of 3-D p=3 fit 3 times into 320).
 template <int N, int D, int T, class R>
 struct Tile {
     using G = IG<N, D>;
-    // per element: raw and face-solved E of every slice (one predictor slice
-    // reuses the raw buffer)
-    static constexpr int PER = 2 * T * G::EP;
-    // LDS bound, and at most two face-B points per thread (their dB/dt of
-    // every slice stay in registers)
-    static constexpr int EPB_LDS = kLdsBudget / (int)(PER * sizeof(R));
-    static constexpr int EPB_REG = 2 * BS / G::BP;
-    static constexpr int EPB_RAW = EPB_LDS < EPB_REG ? EPB_LDS : EPB_REG;
-    static constexpr int EPB = EPB_RAW < 1 ? 1 : (EPB_RAW > 16 ? 16 : EPB_RAW);
-    static constexpr int NB = (EPB * G::BP + BS - 1) / BS;  // face-B points per thread
+    static constexpr int EMAX = G::epts(0) > G::epts(2) ? G::epts(0) : G::epts(2);
+    static constexpr int THREADS = D == 3 && N == 4 ? 320 : 256;
+    static constexpr int EPB = THREADS / EMAX;
+    static_assert(EPB >= 1 && G::bpts(0) <= EMAX && G::bpts(2) <= EMAX, "one point per thread");
 };
-
-// Edge points of one element (all components) ordered by how many faces
-// they lie on (none, the first face axis only, the second only, both) and by
-// component, so that the lanes of a wave mostly take the same path in the
-// face solves.
-template <int N, int D>
-struct PermT {
-    int p[IG<N, D>::EP];
-    constexpr PermT() : p() {
-        using G = IG<N, D>;
-        int k = 0;
-        for (int key = 0; key < 12; key++) {
-            const int cc = key / 3, e = key % 3;
-            int ax[2] = {-1, -1}, nax = 0;
-            for (int c = 0; c < 3; c++)
-                if (c != e && c < D) ax[nax++] = c;
-            for (int lp = 0; lp < G::epts(e); lp++) {
-                const int pt[3] = {lp % G::ecnt(e, 0), (lp / G::ecnt(e, 0)) % G::ecnt(e, 1),
-                                   lp / (G::ecnt(e, 0) * G::ecnt(e, 1))};
-                int code = 0;
-                for (int i = 0; i < nax; i++)
-                    if (pt[ax[i]] == 0 || pt[ax[i]] == G::ecnt(e, ax[i]) - 1) code |= 1 << i;
-                if (code == cc) p[k++] = G::eoff(e) + lp;
-            }
-        }
-    }
-};
-template <int N, int D>
-__constant__ PermT<N, D> kPerm = PermT<N, D>();
-template <int N, int D>
-constexpr bool perm_is_permutation() {
-    constexpr int EP = IG<N, D>::EP;
-    PermT<N, D> P;
-    bool seen[EP] = {};
-    for (int i = 0; i < EP; i++) {
-        if (P.p[i] < 0 || P.p[i] >= EP || seen[P.p[i]]) return false;
-        seen[P.p[i]] = true;
-    }
-    return true;
-}
 
 struct IArgs {
     void* Eout;           // raw E written by this launch (T, 3 components, elements, points)
@@ -142,6 +100,8 @@ struct IArgs {
     int g[3];             // ghost elements per side (1 on active axes)
     int periodic[3];      // 1: periodic wrap, 0: gradfree mirror
     int nel;              // active elements
+    int tin;              // slices present in Ein (1: every slice is slice 0)
+    ConstDiv dh[3];       // division by h
 };
 
 template <class R>
@@ -158,71 +118,6 @@ __device__ __forceinline__ size_t eslab(int e, int nel) {
     size_t o = 0;
     for (int c = 0; c < e; c++) o += (size_t)T * nel * G::epts(c);
     return o;
-}
-
-// Element and point that hold the raw E seen at element el, point pt of
-// component e, where el may be one past either end of an active axis: that is
-// the ghost the SD trace fill (src/boundary.cpp:48-113) makes, i.e. periodic,
-// the element at the other end, same point; gradfree, the element itself with
-// the point mirrored across its face. Returns the linear element index.
-template <int N, int D>
-__device__ __forceinline__ int resolve(const IArgs& a, int e, const int el[3], int r[3]) {
-    using G = IG<N, D>;
-    int q[3] = {el[0], el[1], el[2]};
-#pragma unroll
-    for (int c = 0; c < D; c++) {
-        if (q[c] < 0) {
-            if (a.periodic[c]) q[c] = a.n[c] - 1;
-            else { q[c] = 0; r[c] = G::ecnt(e, c) - 1 - r[c]; }
-        } else if (q[c] >= a.n[c]) {
-            if (a.periodic[c]) q[c] = 0;
-            else { q[c] = a.n[c] - 1; r[c] = G::ecnt(e, c) - 1 - r[c]; }
-        }
-    }
-    return (q[2] * a.n[1] + q[1]) * a.n[0] + q[0];
-}
-
-// E after the face solve along axis `ax` only (or the raw value off that
-// axis's faces); raw(e, el, pt) reads a raw value.
-template <int N, int D, class R, class Raw>
-__device__ __forceinline__ R solved_1(const IArgs& a, int e, const int el[3], const int pt[3], int ax, Raw raw) {
-    using G = IG<N, D>;
-    const int last = G::ecnt(e, ax) - 1;
-    const R own = raw(e, el, pt);
-    if (pt[ax] != 0 && pt[ax] != last) return own;
-    int el2[3] = {el[0], el[1], el[2]}, pt2[3] = {pt[0], pt[1], pt[2]};
-    if (pt[ax] == 0) {
-        el2[ax] -= 1;
-        pt2[ax] = last;
-        return upwind<R>(raw(e, el2, pt2), own, a.vel[ax]);
-    }
-    el2[ax] += 1;
-    pt2[ax] = 0;
-    return upwind<R>(own, raw(e, el2, pt2), a.vel[ax]);
-}
-
-// Face-solved E of component e: along its first active face axis, then its
-// second (x before y before z, the order of the stage calls).
-template <int N, int D, class R, class Raw>
-__device__ __forceinline__ R solved(const IArgs& a, int e, const int el[3], const int pt[3], Raw raw) {
-    using G = IG<N, D>;
-    int ax[2] = {0, 0}, nax = 0;
-#pragma unroll
-    for (int c = 0; c < 3; c++)
-        if (c != e && c < D) ax[nax++] = c;
-    if (nax == 1) return solved_1<N, D, R>(a, e, el, pt, ax[0], raw);
-    const int b = ax[1], last = G::ecnt(e, b) - 1;
-    const R own = solved_1<N, D, R>(a, e, el, pt, ax[0], raw);
-    if (pt[b] != 0 && pt[b] != last) return own;
-    int el2[3] = {el[0], el[1], el[2]}, pt2[3] = {pt[0], pt[1], pt[2]};
-    if (pt[b] == 0) {
-        el2[b] -= 1;
-        pt2[b] = last;
-        return upwind<R>(solved_1<N, D, R>(a, e, el2, pt2, ax[0], raw), own, a.vel[b]);
-    }
-    el2[b] += 1;
-    pt2[b] = 0;
-    return upwind<R>(own, solved_1<N, D, R>(a, e, el2, pt2, ax[0], raw), a.vel[b]);
 }
 
 __device__ __forceinline__ void split_pt(int p, int nx, int ny, int pt[3]) {
@@ -261,222 +156,277 @@ __device__ __forceinline__ R edge_e(int e, const int pt[3], const R* S2F, const 
     return vel[a1] * b2 - vel[a2] * b1;
 }
 
-// Zero-order guess: the raw E of B, written to every slice.
+// Face-solved E of component e (src/induction.cpp:509-560) at point pt of an
+// element, for the slices: raw(off) reads raw values at an offset from the
+// element's own point. lo[c] and hi[c] are the offsets of the points that
+// share a lower / upper face point along c: the neighbour's opposite face
+// point, or 0 where the ghost mirrors the element itself (gradfree).
+// face(c) = -1 / +1 on a lower / upper face along c, else 0. dir[c] is the
+// sign of the velocity along c; AVG: some dir is 0, where the solve takes the
+// mean of both sides.
+template <int e, int D, bool AVG, class V, class Raw>
+__device__ __forceinline__ V edge_solved(const long lo[3], const long hi[3], const int dir[3], const int face[3],
+                                         Raw raw) {
+    constexpr int c1 = e == 0 ? 1 : 0, c2 = e == 2 ? 1 : 2;  // face axes, x before y before z
+    auto shift = [&](int c) -> long {
+        return c >= D ? 0 : (face[c] < 0 && dir[c] > 0 ? lo[c] : (face[c] > 0 && dir[c] < 0 ? hi[c] : 0));
+    };
+    if (!AVG) return raw(shift(c1) + shift(c2));
+    auto first = [&](long base) -> V {
+        if (c1 >= D || face[c1] == 0 || dir[c1] != 0) return raw(base + shift(c1));
+        return mean(raw(base + (face[c1] < 0 ? lo[c1] : 0)), raw(base + (face[c1] < 0 ? 0 : hi[c1])));
+    };
+    if (c2 >= D || face[c2] == 0 || dir[c2] != 0) return first(shift(c2));
+    return mean(first(face[c2] < 0 ? lo[c2] : 0), first(face[c2] < 0 ? 0 : hi[c2]));
+}
+
+// One point's value in every slice
+template <class R, int T>
+struct Slices {
+    R v[T];
+};
+template <class R, int T>
+__device__ __forceinline__ Slices<R, T> mean(const Slices<R, T>& l, const Slices<R, T>& r) {
+    Slices<R, T> m;
+#pragma unroll
+    for (int t = 0; t < T; t++) m.v[t] = R(0.5) * (l.v[t] + r.v[t]);
+    return m;
+}
+
+template <class F>
+__device__ __forceinline__ void for_each_component(F f) {
+    f(std::integral_constant<int, 0>{});
+    f(std::integral_constant<int, 1>{});
+    f(std::integral_constant<int, 2>{});
+}
+
+// Linear index of active element lin in the ghost-inclusive arrays
+__device__ __forceinline__ size_t ghosted(const IArgs& a, int lin) {
+    return ((size_t)(lin / (a.n[0] * a.n[1]) + a.g[2]) * a.G[1] + ((lin / a.n[0]) % a.n[1] + a.g[1])) * a.G[0] +
+           (lin % a.n[0] + a.g[0]);
+}
+
+// Zero-order guess: the raw E of B, slice 0. The sweep's tile with B read once
+// into LDS (reading each of the up to 8 B values of an edge point through the
+// caches, over all components in one index, took 0.69 ms at 1024^2 p=3).
 template <int N, int D, int T, class R>
-__global__ void __launch_bounds__(BS) k_istart(IArgs a) {
+__global__ void __launch_bounds__((Tile<N, D, T, R>::THREADS)) k_istart(IArgs a) {
     using G = IG<N, D>;
-    constexpr int M = G::M;
+    using TL = Tile<N, D, T, R>;
+    constexpr int EPB = TL::EPB, M = G::M;
+    __shared__ R sB[EPB * G::BP];
     __shared__ R sS2F[M * N];
-    for (int i = threadIdx.x; i < M * N; i += BS) sS2F[i] = (R)a.S2F[i];
+    const int e0 = blockIdx.x * EPB, tid = threadIdx.x, ne = min(EPB, a.nel - e0);
+    for (int i = tid; i < M * N; i += TL::THREADS) sS2F[i] = (R)a.S2F[i];
+    for_each_component([&](auto comp) {
+        constexpr int d = comp.value, BPT = G::bpts(d);
+        if (tid >= ne * BPT) return;
+        const int q = tid / BPT, p = tid % BPT;
+        sB[q * G::BP + G::boff(d) + p] = (R)a.B[d][ghosted(a, e0 + q) * BPT + p];
+    });
     __syncthreads();
     const R vel[3] = {(R)a.vel[0], (R)a.vel[1], (R)a.vel[2]};
-    R* out = (R*)a.Eout;
-    const size_t total = (size_t)a.nel * G::EP;
-    for (size_t idx = (size_t)blockIdx.x * BS + threadIdx.x; idx < total; idx += (size_t)gridDim.x * BS) {
-        int lin = (int)(idx / G::EP), p = (int)(idx % G::EP);
-        int e = p < G::eoff(1) ? 0 : (p < G::eoff(2) ? 1 : 2);
-        p -= G::eoff(e);
-        int el[3] = {lin % a.n[0], (lin / a.n[0]) % a.n[1], lin / (a.n[0] * a.n[1])};
+    for_each_component([&](auto comp) {
+        constexpr int e = comp.value, EPT = G::epts(e);
+        if (tid >= ne * EPT) return;
+        const int q = tid / EPT, p = tid % EPT;
         int pt[3];
         split_pt(p, G::ecnt(e, 0), G::ecnt(e, 1), pt);
-        size_t gb = ((size_t)(el[2] + a.g[2]) * a.G[1] + (el[1] + a.g[1])) * a.G[0] + (el[0] + a.g[0]);
-        auto bget = [&](int d, const int q[3]) -> R {
-            return (R)a.B[d][gb * G::bpts(d) + (q[2] * G::bcnt(d, 1) + q[1]) * G::bcnt(d, 0) + q[0]];
+        const R* Bs = sB + q * G::BP;
+        auto bget = [&](int d, const int r3[3]) -> R {
+            return Bs[G::boff(d) + (r3[2] * G::bcnt(d, 1) + r3[1]) * G::bcnt(d, 0) + r3[0]];
         };
-        R v = edge_e<N, D, R>(e, pt, sS2F, vel, bget);
-        size_t o = eslab<N, D, T>(e, a.nel) + (size_t)lin * G::epts(e) + p;
-        for (int t = 0; t < T; t++) out[o + (size_t)t * a.nel * G::epts(e)] = v;
-    }
+        ((R*)a.Eout)[eslab<N, D, T>(e, a.nel) + (size_t)(e0 + q) * EPT + p] = edge_e<N, D, R>(e, pt, sS2F, vel, bget);
+    });
 }
 
 // One Picard sweep (CORR = false: predictor slices and their raw E; CORR =
-// true: the corrector into B). The tile's raw E of every slice is staged in
-// LDS (face partners inside the tile are read there, others from HBM),
-// face-solved into a second LDS buffer and differentiated into the dB/dt of
-// the thread's face-B points, kept in registers for all slices; the
-// predictor slices then go through the raw buffer one at a time.
+// true: the corrector into B). The sweep moves each raw-E value of the tile
+// once in and once out (2-D p=3: 4.6 KB per element, 1.1 ms at 1024^2 at the
+// rate of a large copy); a thread owns one point of each component in every
+// phase, with the slices unrolled, so that T loads are in flight per point,
+// all index arithmetic is by compile-time constants and shared by the slices,
+// and the sweep needs three barriers. Measured (1024^2 p=3 step): staging the
+// raw E and solving faces LDS to LDS, with points in a runtime order, took
+// 5.8 ms per sweep; this form 1.30 ms (3-D mixed 40 x 37 x 43: 1.04 -> 0.29 ms).
 template <int N, int D, int T, bool CORR, class R>
-__global__ void __launch_bounds__(BS) k_isweep(IArgs a) {
+__global__ void __launch_bounds__((Tile<N, D, T, R>::THREADS)) k_isweep(IArgs a) {
     using G = IG<N, D>;
     using TL = Tile<N, D, T, R>;
     constexpr bool PLAIN = std::is_same<R, double>::value;
     using Acc = typename std::conditional<PLAIN || CORR, double, float>::type;  // dB/dt
-    constexpr int EPB = TL::EPB, M = G::M, NB = TL::NB, EPT = T * G::EP;
-    static_assert(G::BP <= EPT, "a predictor slice fits in the raw-E buffer");
-    __shared__ R sE[EPB * EPT], sS[EPB * EPT];  // (element, slice, point)
-    R* const sB = sE;                           // predictor slice, after the face solves
+    constexpr int EPB = TL::EPB, M = G::M, TH = TL::THREADS;
+    static_assert(G::BP <= G::EP, "the predictor slices fit in the edge buffer");
+    __shared__ R sE[EPB * T * G::EP];  // face-solved E (element, slice, point), then the predictor slices
     __shared__ R sS2F[M * N];
     __shared__ double sDm[N * M], sInv[T * T], sW[T];
     __shared__ Acc sDmH[PLAIN ? 1 : D][PLAIN ? 1 : N * M];  // dfp_to_sp / h_axis
     __shared__ float sP[PLAIN ? 1 : T * T];                  // invader * w * dt
-    __shared__ int sEl[EPB][3];
-    __shared__ int sPerm[G::EP];
     // workgroups go to the 8 XCDs in turn; XCD x takes the x-th contiguous
     // eighth of the element tiles, so a tile's y (and z) neighbours, whose
     // face traces it reads, were mostly written through the same L2. The grid
     // is a multiple of 8; tiles past the end exit (uniform per block).
     const int blk = SPDK_ISWEEP_XCD ? (int)((blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8) : (int)blockIdx.x;
-    if (blk * EPB >= a.nel) return;
-    for (int i = threadIdx.x; i < G::EP; i += BS) sPerm[i] = kPerm<N, D>.p[i];
-    for (int i = threadIdx.x; i < N * M; i += BS) {
+    const int e0 = blk * EPB;
+    if (e0 >= a.nel) return;
+    const int tid = threadIdx.x, ne = min(EPB, a.nel - e0);
+    for (int i = tid; i < N * M; i += TH) {
         sDm[i] = a.Dm[i];
         sS2F[i] = (R)a.S2F[i];
         if (!PLAIN)
             for (int c = 0; c < D; c++) sDmH[c][i] = (Acc)(a.Dm[i] / a.h[c]);
     }
-    if (threadIdx.x < T * T) {
-        sInv[threadIdx.x] = a.inv[threadIdx.x];
-        if (!PLAIN) sP[threadIdx.x] = (float)(a.inv[threadIdx.x] * a.w[threadIdx.x % T] * a.dt);
+    if (tid < T * T) {
+        sInv[tid] = a.inv[tid];
+        if (!PLAIN) sP[tid] = (float)(a.inv[tid] * a.w[tid % T] * a.dt);
     }
-    if (threadIdx.x < T) sW[threadIdx.x] = a.w[threadIdx.x];
-    const int e0 = blk * EPB;
-    const int ne = min(EPB, a.nel - e0);
-    if ((int)threadIdx.x < ne) {
-        int lin = e0 + threadIdx.x;
-        sEl[threadIdx.x][0] = lin % a.n[0];
-        sEl[threadIdx.x][1] = (lin / a.n[0]) % a.n[1];
-        sEl[threadIdx.x][2] = lin / (a.n[0] * a.n[1]);
-    }
-    const R* Ein = (const R*)a.Ein;
-
-    // A1. the tile's raw E of every slice (contiguous per component and slice)
+    if (tid < T) sW[tid] = a.w[tid];
+    const int dir[3] = {a.vel[0] == 0 ? 0 : (a.vel[0] > 0 ? 1 : -1), a.vel[1] == 0 ? 0 : (a.vel[1] > 0 ? 1 : -1),
+                        a.vel[2] == 0 ? 0 : (a.vel[2] > 0 ? 1 : -1)};
+    bool any_mean = false;
 #pragma unroll
-    for (int e = 0; e < 3; e++)
-        for (int t = 0; t < T; t++) {
-            const R* src = Ein + eslab<N, D, T>(e, a.nel) + ((size_t)t * a.nel + e0) * G::epts(e);
-            for (int i = threadIdx.x; i < ne * G::epts(e); i += BS) {
-                int q = i / G::epts(e), p = i % G::epts(e);
-                sE[(q * T + t) * G::EP + G::eoff(e) + p] = src[i];
-            }
-        }
-    __syncthreads();
-    // A2. face solves of every slice; items run point-major over the tile's
-    // elements, points in class order within a slice
-    for (int idx = threadIdx.x; idx < ne * EPT; idx += BS) {
-        int rank = idx / ne, q = idx - rank * ne;
-        int t = rank / G::EP;
-        int p = sPerm[rank - t * G::EP];
-        int e = p < G::eoff(1) ? 0 : (p < G::eoff(2) ? 1 : 2);
+    for (int c = 0; c < D; c++) any_mean = any_mean || dir[c] == 0;
+
+    // A. face-solved E of every slice
+    for_each_component([&](auto comp) {
+        constexpr int e = comp.value, EPT = G::epts(e);
+        if (tid >= ne * EPT) return;
+        const int q = tid / EPT, p = tid % EPT, lin = e0 + q;
         int pt[3];
-        split_pt(p - G::eoff(e), G::ecnt(e, 0), G::ecnt(e, 1), pt);
-        auto raw = [&](int ec, const int el[3], const int pc[3]) -> R {
-            int r[3] = {pc[0], pc[1], pc[2]};
-            int lin = resolve<N, D>(a, ec, el, r);
-            int pp = (r[2] * G::ecnt(ec, 1) + r[1]) * G::ecnt(ec, 0) + r[0];
-            int qq = lin - e0;
-            if (qq >= 0 && qq < ne) return sE[(qq * T + t) * G::EP + G::eoff(ec) + pp];
-            return Ein[eslab<N, D, T>(ec, a.nel) + ((size_t)t * a.nel + lin) * G::epts(ec) + pp];
+        split_pt(p, G::ecnt(e, 0), G::ecnt(e, 1), pt);
+        const int el[3] = {lin % a.n[0], (lin / a.n[0]) % a.n[1], lin / (a.n[0] * a.n[1])};
+        const int es[3] = {1, a.n[0], a.n[0] * a.n[1]};
+        constexpr int ps[3] = {1, G::ecnt(e, 0), G::ecnt(e, 0) * G::ecnt(e, 1)};
+        long lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
+        int face[3] = {0, 0, 0};
+#pragma unroll
+        for (int c = 0; c < D; c++) {
+            if (c == e) continue;
+            face[c] = pt[c] == 0 ? -1 : (pt[c] == M - 1 ? 1 : 0);
+            const bool first = el[c] == 0, last = el[c] == a.n[c] - 1;
+            const long across = (long)(M - 1) * ps[c];
+            lo[c] = first && !a.periodic[c] ? 0 : (long)(first ? a.n[c] - 1 : -1) * es[c] * EPT + across;
+            hi[c] = last && !a.periodic[c] ? 0 : (long)(last ? 1 - a.n[c] : 1) * es[c] * EPT - across;
+        }
+        const size_t ss = (size_t)a.nel * EPT;
+        const R* own = (const R*)a.Ein + eslab<N, D, T>(e, a.nel) + (size_t)lin * EPT + p;
+        const int tin = a.tin;
+        auto raw = [&](long off) {
+            Slices<R, T> r;
+#pragma unroll
+            for (int t = 0; t < T; t++) r.v[t] = t < tin ? own[off + (long)(t * ss)] : r.v[0];
+            return r;
         };
-        sS[(q * T + t) * G::EP + p] = solved<N, D, R>(a, e, sEl[q], pt, raw);
-    }
+        const Slices<R, T> v = any_mean ? edge_solved<e, D, true, Slices<R, T>>(lo, hi, dir, face, raw)
+                                        : edge_solved<e, D, false, Slices<R, T>>(lo, hi, dir, face, raw);
+#pragma unroll
+        for (int t = 0; t < T; t++)
+            if (t < tin) sE[(q * T + t) * G::EP + G::eoff(e) + p] = v.v[t];
+    });
     __syncthreads();
-    // B. dB/dt of every slice at the thread's face-B points
-    Acc dBdt[NB][T];
-#pragma unroll
-    for (int j = 0; j < NB; j++) {
-        int idx = threadIdx.x + j * BS;
-#pragma unroll
-        for (int t = 0; t < T; t++) dBdt[j][t] = 0;
-        if (idx < ne * G::BP) {
-            // point-major over the tile's elements: a wave's lanes share the
-            // component
-            int p = idx / ne, q = idx - p * ne;
-            int d = p < G::boff(1) ? 0 : (p < G::boff(2) ? 1 : 2);
-            int pt[3];
-            split_pt(p - G::boff(d), G::bcnt(d, 0), G::bcnt(d, 1), pt);
-            const int a1 = d == 2 ? 0 : d + 1, a2 = a1 == 2 ? 0 : a1 + 1;
-#pragma unroll
-            for (int t = 0; t < T; t++) {
-                // E1 = E_{d+1} differentiated along d+2, E2 = E_{d+2} along d+1
-                const R* E1 = sS + (q * T + t) * G::EP + G::eoff(a1);
-                const R* E2 = sS + (q * T + t) * G::EP + G::eoff(a2);
-                Acc dB = 0, E;
-                for (int l = 0; l < M; l++) {
-                    if (a2 < D) {
-                        int r[3] = {pt[0], pt[1], pt[2]};
-                        r[a2] = l;
-                        E = (Acc)E1[(r[2] * G::ecnt(a1, 1) + r[1]) * G::ecnt(a1, 0) + r[0]];
-                        if (PLAIN) dB += E * sDm[pt[a2] * M + l] / a.h[a2];
-                        else dB += E * sDmH[PLAIN ? 0 : a2][pt[a2] * M + l];
-                    }
-                    if (a1 < D) {
-                        int r[3] = {pt[0], pt[1], pt[2]};
-                        r[a1] = l;
-                        E = (Acc)E2[(r[2] * G::ecnt(a2, 1) + r[1]) * G::ecnt(a2, 0) + r[0]];
-                        if (PLAIN) dB -= E * sDm[pt[a1] * M + l] / a.h[a1];
-                        else dB -= E * sDmH[PLAIN ? 0 : a1][pt[a1] * M + l];
-                    }
-                }
-                dBdt[j][t] = dB;
-            }
-        }
-    }
 
-    // the thread's face-B points: old values, then the corrector or the
-    // predictor slices
-    double B_old[NB];
-    double* Bp[NB];
+    // B. dB/dt of every slice at the thread's face-B points
+    Acc dBdt[3][T];
+    for_each_component([&](auto comp) {
+        constexpr int d = comp.value, BPT = G::bpts(d);
+        constexpr int a1 = (d + 1) % 3, a2 = (d + 2) % 3;
 #pragma unroll
-    for (int j = 0; j < NB; j++) {
-        int idx = threadIdx.x + j * BS;
-        Bp[j] = nullptr;
-        B_old[j] = 0;
-        if (idx < ne * G::BP) {
-            int p = idx / ne, q = idx - p * ne;
-            int d = p < G::boff(1) ? 0 : (p < G::boff(2) ? 1 : 2);
-            size_t gb = ((size_t)(sEl[q][2] + a.g[2]) * a.G[1] + (sEl[q][1] + a.g[1])) * a.G[0] + (sEl[q][0] + a.g[0]);
-            Bp[j] = a.B[d] + gb * G::bpts(d) + (p - G::boff(d));
-            B_old[j] = *Bp[j];
+        for (int t = 0; t < T; t++) dBdt[d][t] = 0;
+        if (tid >= ne * BPT) return;
+        const int q = tid / BPT, p = tid % BPT;
+        int pt[3];
+        split_pt(p, G::bcnt(d, 0), G::bcnt(d, 1), pt);
+        // E1 = E_{d+1} differentiated along d+2, E2 = E_{d+2} along d+1
+        constexpr int s1[3] = {1, G::ecnt(a1, 0), G::ecnt(a1, 0) * G::ecnt(a1, 1)};
+        constexpr int s2[3] = {1, G::ecnt(a2, 0), G::ecnt(a2, 0) * G::ecnt(a2, 1)};
+        const R* E1 = sE + q * T * G::EP + G::eoff(a1) + (pt[0] * s1[0] + pt[1] * s1[1] + pt[2] * s1[2] - pt[a2] * s1[a2]);
+        const R* E2 = sE + q * T * G::EP + G::eoff(a2) + (pt[0] * s2[0] + pt[1] * s2[1] + pt[2] * s2[2] - pt[a1] * s2[a1]);
+        Acc D1[M], D2[M];
+#pragma unroll
+        for (int l = 0; l < M; l++) {
+            D1[l] = a2 < D ? (PLAIN ? (Acc)sDm[pt[a2] * M + l] : sDmH[PLAIN || a2 >= D ? 0 : a2][PLAIN ? 0 : pt[a2] * M + l]) : (Acc)0;
+            D2[l] = a1 < D ? (PLAIN ? (Acc)sDm[pt[a1] * M + l] : sDmH[PLAIN || a1 >= D ? 0 : a1][PLAIN ? 0 : pt[a1] * M + l]) : (Acc)0;
         }
-    }
-    if (CORR) {
+        const int tin = a.tin;
 #pragma unroll
-        for (int j = 0; j < NB; j++) {
-            if (!Bp[j]) continue;
+        for (int t = 0; t < T; t++) {
+            if (t >= tin) {
+                dBdt[d][t] = dBdt[d][0];
+                continue;
+            }
+            Acc dB = 0;
+#pragma unroll
+            for (int l = 0; l < M; l++) {
+                if (a2 < D) {
+                    const Acc x = (Acc)E1[t * G::EP + l * s1[a2]] * D1[l];
+                    dB += PLAIN ? (Acc)div_fast((double)x, a.dh[a2]) : x;
+                }
+                if (a1 < D) {
+                    const Acc x = (Acc)E2[t * G::EP + l * s2[a1]] * D2[l];
+                    dB -= PLAIN ? (Acc)div_fast((double)x, a.dh[a1]) : x;
+                }
+            }
+            if (PLAIN && div_recheck((double)dB)) {
+                dB = 0;
+#pragma unroll 1
+                for (int l = 0; l < M; l++) {
+                    if (a2 < D) dB += (Acc)E1[t * G::EP + l * s1[a2]] * (Acc)sDm[pt[a2] * M + l] / (Acc)a.h[a2];
+                    if (a1 < D) dB -= (Acc)E2[t * G::EP + l * s2[a1]] * (Acc)sDm[pt[a1] * M + l] / (Acc)a.h[a1];
+                }
+            }
+            dBdt[d][t] = dB;
+        }
+    });
+
+    // the corrector, or the predictor slices over the edge buffer
+    if (!CORR) __syncthreads();
+    for_each_component([&](auto comp) {
+        constexpr int d = comp.value, BPT = G::bpts(d);
+        if (tid >= ne * BPT) return;
+        const int q = tid / BPT, p = tid % BPT;
+        double* Bp = a.B[d] + ghosted(a, e0 + q) * BPT + p;
+        const double B_old = *Bp;
+        if (CORR) {
             double dB = 0;
 #pragma unroll
-            for (int t = 0; t < T; t++) dB += (double)dBdt[j][t] * sW[t] * a.dt;
-            *Bp[j] = B_old[j] - dB;
+            for (int t = 0; t < T; t++) dB += (double)dBdt[d][t] * sW[t] * a.dt;
+            *Bp = B_old - dB;
+            return;
         }
-        return;
-    }
-    R* Eout = (R*)a.Eout;
+#pragma unroll
+        for (int t = 0; t < T; t++) {
+            Acc dB = 0;
+            if (PLAIN) {
+#pragma unroll
+                for (int l = 0; l < T; l++) dB += dBdt[d][l] * sInv[t * T + l] * sW[l] * a.dt;
+            } else {
+#pragma unroll
+                for (int l = 0; l < T; l++) dB += dBdt[d][l] * (Acc)sP[t * T + l];
+            }
+            sE[(q * T + t) * G::BP + G::boff(d) + p] = (R)B_old - (R)dB;
+        }
+    });
+    if (CORR) return;
+    __syncthreads();
+    // C. the slices' raw E
     const R vel[3] = {(R)a.vel[0], (R)a.vel[1], (R)a.vel[2]};
-    for (int t = 0; t < T; t++) {
-        __syncthreads();  // the raw buffer is free (face solves done / previous slice's E written)
-        // C1. predictor slice t
+    for_each_component([&](auto comp) {
+        constexpr int e = comp.value, EPT = G::epts(e);
+        if (tid >= ne * EPT) return;
+        const int q = tid / EPT, p = tid % EPT;
+        int pt[3];
+        split_pt(p, G::ecnt(e, 0), G::ecnt(e, 1), pt);
+        R* dst = (R*)a.Eout + eslab<N, D, T>(e, a.nel) + (size_t)(e0 + q) * EPT + p;
+        const size_t ss = (size_t)a.nel * EPT;
 #pragma unroll
-        for (int j = 0; j < NB; j++) {
-            int idx = threadIdx.x + j * BS;
-            if (idx < ne * G::BP) {
-                Acc dB = 0;
-                if (PLAIN) {
-#pragma unroll
-                    for (int l = 0; l < T; l++) dB += dBdt[j][l] * sInv[t * T + l] * sW[l] * a.dt;
-                } else {
-#pragma unroll
-                    for (int l = 0; l < T; l++) dB += dBdt[j][l] * (Acc)sP[t * T + l];
-                }
-                sB[(idx - (idx / ne) * ne) * G::BP + idx / ne] = (R)B_old[j] - (R)dB;
-            }
+        for (int t = 0; t < T; t++) {
+            const R* Bs = sE + (q * T + t) * G::BP;
+            auto bget = [&](int d, const int r3[3]) -> R {
+                return Bs[G::boff(d) + (r3[2] * G::bcnt(d, 1) + r3[1]) * G::bcnt(d, 0) + r3[0]];
+            };
+            dst[t * ss] = edge_e<N, D, R>(e, pt, sS2F, vel, bget);
         }
-        __syncthreads();
-        // C2. its raw E
-#pragma unroll
-        for (int e = 0; e < 3; e++) {
-            R* dst = Eout + eslab<N, D, T>(e, a.nel) + ((size_t)t * a.nel + e0) * G::epts(e);
-            for (int i = threadIdx.x; i < ne * G::epts(e); i += BS) {
-                int q = i / G::epts(e), pe = i % G::epts(e);
-                int pt[3];
-                split_pt(pe, G::ecnt(e, 0), G::ecnt(e, 1), pt);
-                const R* Bs = sB + q * G::BP;
-                auto bget = [&](int d, const int r3[3]) -> R {
-                    return Bs[G::boff(d) + (r3[2] * G::bcnt(d, 1) + r3[1]) * G::bcnt(d, 0) + r3[0]];
-                };
-                dst[i] = edge_e<N, D, R>(e, pt, sS2F, vel, bget);
-            }
-        }
-    }
+    });
 }
 
 template <int N, int D, int T, class R>
@@ -487,23 +437,22 @@ size_t ws_bytes(int nel) {
 template <int N, int D, int T, class R>
 int run_step(spdk_ctx* c, IArgs a, void* ws) {
     using TL = Tile<N, D, T, R>;
-    static_assert(perm_is_permutation<N, D>(), "edge-point order must be a permutation");
     const size_t half = (size_t)T * a.nel * IG<N, D>::EP;
     R* buf[2] = {(R*)ws, (R*)ws + half};
-    unsigned nb = (unsigned)((a.nel + TL::EPB - 1) / TL::EPB);
-    if (SPDK_ISWEEP_XCD) nb = (nb + 7) / 8 * 8;
-    const unsigned nstart = (unsigned)std::min<size_t>(((size_t)a.nel * IG<N, D>::EP + BS - 1) / BS, 65536);
+    const unsigned nstart = (unsigned)((a.nel + TL::EPB - 1) / TL::EPB);
+    const unsigned nb = SPDK_ISWEEP_XCD ? (nstart + 7) / 8 * 8 : nstart;
     a.Eout = buf[0];
     a.Ein = nullptr;
-    hipLaunchKernelGGL((k_istart<N, D, T, R>), dim3(nstart), dim3(BS), 0, c->stream, a);
+    hipLaunchKernelGGL((k_istart<N, D, T, R>), dim3(nstart), dim3(TL::THREADS), 0, c->stream, a);
     SPDK_LAUNCH_CHECK("induction istart");
     for (int s = 0; s < T; s++) {
         a.Ein = buf[s & 1];
         a.Eout = buf[(s + 1) & 1];
+        a.tin = s == 0 ? 1 : T;
         bool rec = c->timing && c->ev_used < spdk_ctx::kEvPool;
         if (rec) SPDK_CHECK(hipEventRecord(c->evs[c->ev_used][0], c->stream));
-        if (s < T - 1) hipLaunchKernelGGL((k_isweep<N, D, T, false, R>), dim3(nb), dim3(BS), 0, c->stream, a);
-        else hipLaunchKernelGGL((k_isweep<N, D, T, true, R>), dim3(nb), dim3(BS), 0, c->stream, a);
+        if (s < T - 1) hipLaunchKernelGGL((k_isweep<N, D, T, false, R>), dim3(nb), dim3(TL::THREADS), 0, c->stream, a);
+        else hipLaunchKernelGGL((k_isweep<N, D, T, true, R>), dim3(nb), dim3(TL::THREADS), 0, c->stream, a);
         SPDK_LAUNCH_CHECK("induction isweep");
         if (rec) SPDK_CHECK(hipEventRecord(c->evs[c->ev_used++][1], c->stream));
     }
@@ -595,6 +544,7 @@ int step(spdk_ctx* c, double* Bx, spdk_sd_shape sx, double* By, spdk_sd_shape sy
     for (int d = 0; d < 3; d++) {
         a.vel[d] = c->prm.vel[d];
         a.h[d] = c->prm.h[d];
+        a.dh[d] = const_div(c->prm.h[d]);
         a.G[d] = Gd[d];
         a.g[d] = c->ngh[d];
         a.n[d] = Gd[d] - 2 * c->ngh[d];

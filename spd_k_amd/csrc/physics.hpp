@@ -18,6 +18,29 @@ constexpr int NVP = 5; // physical variables
 __host__ __device__ __forceinline__ double smax(double a, double b) { return (a < b) ? b : a; }
 __host__ __device__ __forceinline__ double smin(double a, double b) { return (b < a) ? b : a; }
 
+// Division by a value known before the launch (an element or cell width).
+// With z = 1/h rounded to nearest, q = x z, then q - (q h - x) z with two
+// fused multiply-adds, is x / h rounded to nearest, the bits of the division
+// (Markstein 1990; Brisebarre, Muller, Raina 2004), in 3 instructions instead
+// of the 11 of the general division. It holds while no step leaves the normal
+// range: div_recheck(s) is true for a sum s of such quotients that may hold an
+// inexact one (a term below 2^-969 can only matter to a sum that small; an
+// infinite or NaN term makes the sum NaN), which the caller then forms again
+// with divisions. h must be positive, finite and well inside the normal
+// range; otherwise z is NaN and every sum is formed again.
+struct ConstDiv {
+    double h, z;
+};
+__host__ inline ConstDiv const_div(double h) {
+    const bool ok = h > 0x1p-100 && h < 0x1p100;
+    return {h, ok ? 1.0 / h : __builtin_nan("")};
+}
+__device__ __forceinline__ double div_fast(double x, const ConstDiv& c) {
+    const double q = x * c.z;
+    return __builtin_fma(-__builtin_fma(q, c.h, -x), c.z, q);
+}
+__device__ __forceinline__ bool div_recheck(double s) { return s != 0.0 && !(fabs(s) >= 0x1p-900); }
+
 // src/hydro.cpp:27-32
 __device__ __forceinline__ double sound_speed(double rho, double p, double gm) {
     double c2 = gm * p / rho;
