@@ -1,8 +1,8 @@
 // Fused element-tile path for the hydro SD step (plain FP64).
 //
 // One Picard sweep of ADER_step / one RK stage (src/hydro_ader.hpp:291-325)
-// is one kernel over element tiles. A workgroup owns EPB whole elements and
-// keeps their state, flux-point values and fluxes in LDS; the only data that
+// is one kernel over element tiles. A workgroup owns whole (element, time
+// slice) units and keeps their flux-point fluxes in LDS; the only data that
 // crosses elements are the face traces (the solution interpolated to the
 // first and last flux point of every pencil), which each sweep writes for the
 // next one. The Riemann flux of a face is evaluated by both elements that
@@ -17,6 +17,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include "ctx.hpp"
 #include "physics.hpp"
 
@@ -26,22 +27,50 @@ namespace {
 
 constexpr int kMaxT = 8;
 
+// Waves per SIMD the sweeps are compiled for.
+#ifndef SPDK_SWEEP_WAVES
+#define SPDK_SWEEP_WAVES 3
+#endif
+
 template <int N, int DIM>
 struct Tile {
     static constexpr int M = N + 1;                                // flux points per axis
     static constexpr int NT = DIM == 1 ? 1 : (DIM == 2 ? N : N * N);  // points per element face
     static constexpr int TPE = N * NT;                             // solution points per element
-    static constexpr int EPB = TPE >= 256 ? 1 : 256 / TPE;         // elements per workgroup
-    static constexpr int BLOCK = ((EPB * TPE + 63) / 64) * 64;
+    static constexpr int EPB = TPE >= 256 ? 1 : 256 / TPE;         // units (elements, if of one slice) per workgroup
+    static constexpr int BLOCK = 256;
     static constexpr int FSZ = M * NT;                             // flux points per axis per element
-    // LDS per element (doubles): state + fluxes of every axis
-    static constexpr int LDS_U = NVP * TPE;
-    static constexpr int LDS_F = DIM * NVP * FSZ;
-    // + 4 doubles: the element areas of a block start 8 banks apart (reads
-    // across elements at one in-element offset do not share a bank)
-    static constexpr int LDS_ELEM = LDS_U + LDS_F + 4;
-    static_assert(BLOCK == 256, "tile workgroups are 256 threads");
-    static_assert(LDS_F >= LDS_U, "cv ping-pong reuses the flux area");
+    static constexpr int LDS_U = NVP * TPE;                        // doubles: one state
+    static constexpr int LDS_F = DIM * NVP * FSZ;                  // doubles: fluxes of every axis
+    static_assert(EPB * TPE <= BLOCK && TPE <= BLOCK, "tile workgroups are 256 threads");
+};
+
+// What a sweep produces, and its units. PREDICT: the new predictor slices and
+// their traces; CORRECT: the solution after the step or stage; FACES: the
+// sub-cell face fluxes of the FV update; FLUXES: the flux-point fluxes.
+enum { PREDICT = 0, CORRECT = 1, FACES = 2, FLUXES = 3 };
+
+// S time slices of an element are units of one workgroup. S = T for the sweeps
+// whose slices differ: the workgroup then holds fewer elements (one at 3-D
+// p=3), every thread owns one point of one slice, and the slices meet once, in
+// LDS, for the time contraction. That keeps one slice's divergence per thread
+// in registers instead of T, makes the serial chain of a workgroup T times
+// shorter and gives T times the workgroups (a 32^2 mesh, 1156 elements, has
+// 289 for 256 CUs instead of 73). S = 1 where there is one slice: the first
+// sweep from the zero-order guess and an SSP-RK stage; and for FACES, whose
+// output rows run over elements, with a loop over the slices.
+template <int N, int DIM, int T, int S, int MODE>
+struct Unit {
+    using G = Tile<N, DIM>;
+    static constexpr int EL = G::EPB / S;  // elements per workgroup
+    // doubles per unit: the fluxes, over which the exchanges go (two states; S = 1 PREDICT: all T new slices);
+    // FACES: a scratch state ahead of them. + 4: the unit areas start 8 banks apart
+    static constexpr int SCR = MODE == FACES ? G::LDS_U : 0;
+    static constexpr int NEW = (S == 1 && MODE == PREDICT ? T : 2) * G::LDS_U;
+    static constexpr int AREA = SCR + (G::LDS_F > NEW ? G::LDS_F : NEW) + 4;
+    static constexpr int UNITS = EL * S;
+    static constexpr int DOUBLES = UNITS * AREA + N * G::M;  // + dfp_to_sp
+    static_assert(EL >= 1, "a workgroup holds every slice of an element");
 };
 
 struct SweepArgs {
@@ -65,6 +94,7 @@ struct SweepArgs {
     int act[3], bc[3];
     int E;
     double h[3];
+    ConstDiv dh[3];       // division by h
     double dt, gm, cfl, rk_a;
     int tin_slices;       // slices present in tr_in (1 or T)
     int in_nv;            // variables per slice of U_in
@@ -72,9 +102,7 @@ struct SweepArgs {
     double* Ffv[kMaxT][3];  // flux-only sweep: sub-cell face fluxes of slice t along axis d (FV layout)
     int fvn[3];           // FV cells per axis incl. ghost layers (an axis' face array has one more along it)
     int fgh[3];           // FV ghost layers per axis
-    int flux_only;        // write the flux-point fluxes of every slice and axis; no divergence
     int in_ader;          // state from U_in (else U_sp broadcast to every slice)
-    int out_pred;         // write predictor U_out + tr_out, else corrector
     int rk_first;         // RK: write U0 = U_sp
     int want_dt;          // corrector: compute cv primitives and dt partials
     double g[3];          // constant gravity (hydro/g1..g3)
@@ -118,7 +146,7 @@ __device__ __forceinline__ int face_sweep_block() {
     return (int)((blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8);
 }
 
-template <int N, int DIM>
+template <int N, int DIM, int AREA>
 __device__ __forceinline__ void fv_faces(const SweepArgs& a, double* scr, const double* Fs, int t, int s, bool live,
                                          int ei, int ej, int ek) {
     using G = Tile<N, DIM>;
@@ -189,7 +217,7 @@ __device__ __forceinline__ void fv_faces(const SweepArgs& a, double* scr, const 
                         const int I2 = ox + a.fgh[0] + (ec2[0] - 1) * N, J2 = oy + a.fgh[1] + (ec2[1] - 1) * N;
                         const int K2 = oz + a.fgh[2] + (ec2[2] - 1) * N;
                         double* out2 = a.Ffv[t][d] + ((size_t)K2 * ny + J2) * nx + I2;
-                        const double* sc2 = scr + (long)(e2l - el_of(threadIdx.x, TPE)) * G::LDS_ELEM;
+                        const double* sc2 = scr + (long)(e2l - el_of(threadIdx.x, TPE)) * AREA;
 #pragma unroll
                         for (int v = 0; v < NVP; v++) out2[(size_t)v * vstride] = sc2[v * TPE + ox + N * (oy + N * oz)];
                     }
@@ -226,27 +254,134 @@ __device__ __forceinline__ void fv_faces(const SweepArgs& a, double* scr, const 
     }
 }
 
-// FVF: the flux-only sweep that also forms the face integrals (fv_faces),
-// compiled apart so that the predictor and corrector sweeps keep their
-// register budget (2 waves per SIMD at 3-D p=3).
-template <int N, int DIM, int T, bool FVF>
-__global__ void __launch_bounds__(256) k_sweep(SweepArgs a) {
+// One pencil of axis D: state U (variables slabE apart) of element e, pencil q.
+// Writes the fluxes at its M flux points to Fd (the fidx layout): interpolation
+// to the flux points, Euler fluxes, and the LLF flux at the element faces
+// (src/hydro.cpp:167-206, :368-418). ts: slice of the traces. The neighbours'
+// face values are loaded first, with the ghost fill (src/boundary.cpp:48-113)
+// as a choice of source: n0 is the value left of the lower face, or, in the
+// left ghost, the fill that replaces its own upper face value; n1 likewise on
+// the right. The outer face of a ghost has no neighbour: its own flux.
+// lower_only: the upper face is not needed.
+template <int N, int DIM, int D>
+__device__ __forceinline__ void pencil(const SweepArgs& a, const double* U, size_t slabE, double* Fd, int q, size_t e,
+                                       int ed, int ts, bool lower_only) {
     using G = Tile<N, DIM>;
-    constexpr int M = G::M, NT = G::NT, TPE = G::TPE, EPB = G::EPB;
+    constexpr int M = G::M, NT = G::NT, TPE = G::TPE;
+    const int Nd = a.Ne[D], type = a.bc[D];
+    const bool per = type == SPDK_BC_PERIODIC;
+    const size_t E = (size_t)a.E;
+    const size_t stride = D == 0 ? 1 : (D == 1 ? (size_t)a.Ne[0] : (size_t)a.Ne[0] * a.Ne[1]);
+    const size_t line = e - (size_t)ed * stride;  // element with ed = 0 on this line
+    const bool lo = ed <= 1, hi = ed >= Nd - 2;
+    const size_t el0 = line + (size_t)(lo ? (per ? Nd - 2 : 1) : ed - 1) * stride;
+    const size_t el1 = line + (size_t)(hi ? (per ? 1 : Nd - 2) : ed + 1) * stride;
+    const double* t0 = a.tr_in[D] + ((size_t)ts * NVP * E + el0) * 2 * NT + (lo && !per ? 0 : NT) + q;
+    const double* t1 = a.tr_in[D] + ((size_t)ts * NVP * E + el1) * 2 * NT + (hi && !per ? NT : 0) + q;
+    double n0[NVP], n1[NVP], p[NVP][N];
+#pragma unroll
+    for (int v = 0; v < NVP; v++) {
+        n0[v] = t0[(size_t)v * E * 2 * NT];
+        n1[v] = t1[(size_t)v * E * 2 * NT];
+    }
+    if (type == SPDK_BC_REFLECTIVE) {
+        if (lo) n0[1 + D] = -1.0 * n0[1 + D];
+        if (hi) n1[1 + D] = -1.0 * n1[1 + D];
+    }
+#pragma unroll
+    for (int v = 0; v < NVP; v++)
+#pragma unroll
+        for (int l = 0; l < N; l++) p[v][l] = U[(size_t)v * slabE + e * TPE + spidx<N, DIM>(D, l, q)];
+    auto at = [&](int f, double* u) {
+#pragma unroll
+        for (int v = 0; v < NVP; v++) {
+            double x = 0;
+#pragma unroll
+            for (int l = 0; l < N; l++) x += p[v][l] * a.S2F[f * N + l];
+            u[v] = x;
+        }
+    };
+    auto put = [&](int f, const double* fl) {
+#pragma unroll
+        for (int v = 0; v < NVP; v++) Fd[v * G::FSZ + fidx(D, f, q, N, NT, M)] = fl[v];
+    };
+#pragma unroll
+    for (int f = 1; f < M - 1; f++) {
+        double u[NVP], fl[NVP];
+        at(f, u);
+        state_flux<D>(u, fl, a.gm);
+        put(f, fl);
+    }
+    const bool ghost0 = ed == 0, ghost1 = ed == Nd - 1;
+    {
+        double own[NVP], L[NVP], R[NVP], fl[NVP];
+        at(0, own);
+#pragma unroll
+        for (int v = 0; v < NVP; v++) {
+            L[v] = ghost0 ? own[v] : n0[v];
+            R[v] = ghost1 ? n1[v] : own[v];
+        }
+        riemann_llf<D>(L, R, fl, a.gm, ghost0);
+        put(0, fl);
+    }
+    if (lower_only) return;
+    double own[NVP], L[NVP], R[NVP], fl[NVP];
+    at(M - 1, own);
+#pragma unroll
+    for (int v = 0; v < NVP; v++) {
+        L[v] = ghost0 ? n0[v] : own[v];
+        R[v] = ghost1 ? own[v] : n1[v];
+    }
+    riemann_llf<D>(L, R, fl, a.gm, ghost1);
+    put(M - 1, fl);
+}
+
+// Flux divergence of variable v at solution point s (src/transforms.cpp:301-307),
+// with exact divisions: where a fast one may have been inexact.
+template <int N, int DIM>
+__device__ __forceinline__ double divergence_slow(const SweepArgs& a, const double* Fs, const double* sD, int v, int ii,
+                                                  int jj, int kk) {
+    using G = Tile<N, DIM>;
+    constexpr int M = G::M, NT = G::NT;
+    double acc = 0;
+#pragma unroll 1
+    for (int l = 0; l < M; l++) {
+        acc += Fs[v * G::FSZ + fidx(0, l, DIM == 3 ? kk * N + jj : jj, N, NT, M)] * sD[ii * M + l] / a.h[0];
+        if (DIM >= 2) acc += Fs[(NVP + v) * G::FSZ + fidx(1, l, DIM == 3 ? kk * N + ii : ii, N, NT, M)] * sD[jj * M + l] / a.h[1];
+        if (DIM == 3) acc += Fs[(2 * NVP + v) * G::FSZ + fidx(2, l, jj * N + ii, N, NT, M)] * sD[kk * M + l] / a.h[2];
+    }
+    return acc;
+}
+
+// One sweep (see Unit). Three dependent phases, a barrier between each: the
+// pencils' fluxes into LDS, the divergence at every point, and the output.
+// Pencils are dealt to threads axis by axis over all units, so that a wave
+// mostly works on one axis with all lanes (3-D p=3: 64 pencils per axis and
+// workgroup; the fourth wave has none, and it is another wave in every
+// workgroup and slice). What bounds it (3-D p=3, 64^3): FP64 issue, of which
+// the divergence's divisions by h were 41% before they became three
+// instructions each, and the latency of the phases. With the state read from
+// memory by the pencils and one slice per thread the predictor needs 38.5 KB
+// LDS and fits 4 workgroups per CU.
+template <int N, int DIM, int T, int S, int MODE>
+__global__ void __launch_bounds__(256, MODE == FACES ? 2 : SPDK_SWEEP_WAVES) k_sweep(SweepArgs a) {
+    using G = Tile<N, DIM>;
+    using X = Unit<N, DIM, T, S, MODE>;
+    constexpr int M = G::M, NT = G::NT, TPE = G::TPE, EL = X::EL;
     extern __shared__ double lds[];
+    double* const sD = lds + X::UNITS * X::AREA;
     const int tid = threadIdx.x;
-    const int el = tid / TPE;      // element slot in the tile
-    const int s = tid % TPE;       // solution point within the element
-    const int bx = FVF ? face_sweep_block() : (int)blockIdx.x;
-    if (FVF && bx * EPB >= a.E) return;  // padding of the XCD-ordered grid (uniform per block)
-    const int e = bx * EPB + el;
-    const bool live = el < EPB && e < a.E;
-    double* us = lds + (el < EPB ? el : 0) * G::LDS_ELEM;
-    double* Fs = us + G::LDS_U;
+    const int bx = MODE == FACES ? face_sweep_block() : (int)blockIdx.x;
+    if (MODE == FACES && bx * EL >= a.E) return;  // padding of the XCD-ordered grid (uniform per block)
+    const int unit = tid / TPE, s = tid % TPE;    // (element, slice) and solution point of this thread
+    const int el = unit / S, ut = unit % S;
+    const int e = bx * EL + el;
+    const bool live = unit < X::UNITS && e < a.E;
     const size_t E = (size_t)a.E;
     const size_t slabE = E * TPE;  // one (t,v) plane of a state array
+    double* const Fs = lds + (unit < X::UNITS ? unit : 0) * X::AREA + X::SCR;
+    for (int i = tid; i < N * M; i += G::BLOCK) sD[i] = a.Dm[i];
 
-    // element coordinates
     int ei = 0, ej = 0, ek = 0;
     if (live) {
         ei = e % a.Ne[0];
@@ -255,118 +390,31 @@ __global__ void __launch_bounds__(256) k_sweep(SweepArgs a) {
     }
     const int ii = s % N, jj = DIM >= 2 ? (s / N) % N : 0, kk = DIM == 3 ? s / (N * N) : 0;
 
-    // derivative rows of this solution point
-    double Dx[M], Dy[M], Dz[M];
-#pragma unroll
-    for (int l = 0; l < M; l++) {
-        Dx[l] = a.Dm[ii * M + l];
-        Dy[l] = DIM >= 2 ? a.Dm[jj * M + l] : 0.0;
-        Dz[l] = DIM == 3 ? a.Dm[kk * M + l] : 0.0;
-    }
-    double u_old[NVP];
-#pragma unroll
-    for (int v = 0; v < NVP; v++) u_old[v] = live && !a.flux_only ? a.U_sp[(size_t)v * slabE + (size_t)e * TPE + s] : 0.0;
-
-    double dudt[T][NVP];
-    const int nslices = a.in_ader ? T : 1;  // a broadcast state has identical slices
-
-#pragma unroll
-    for (int t = 0; t < T; t++) {
-        if (t >= nslices) break;
-        // ---- stage the slice in LDS
-        if (live) {
-#pragma unroll
-            for (int v = 0; v < NVP; v++)
-                us[v * TPE + s] = a.in_ader ? a.U_in[((size_t)t * a.in_nv + v) * slabE + (size_t)e * TPE + s] : u_old[v];
-        }
-        __syncthreads();
-        // ---- pencils: interpolation to flux points, fluxes, face Riemann solves
-        // (DIM * NT pencils; more than the element's points only for p = 1 in 3-D)
-        for (int task = s; live && task < DIM * NT; task += TPE) {
-            const int d = task / NT, q = task % NT;
-            const int ed = d == 0 ? ei : (d == 1 ? ej : ek);
-            const int Nd = a.Ne[d];
-            const size_t stride = d == 0 ? 1 : (d == 1 ? (size_t)a.Ne[0] : (size_t)a.Ne[0] * a.Ne[1]);
-            const size_t ebase = (size_t)e - (size_t)ed * stride;  // element with ed = 0 on this line
-            const int ts = a.tin_slices > 1 ? t : 0;
-            const double* tr = a.tr_in[d];
-            auto trace = [&](int ed_src, int side, int v) -> double {
-                size_t src = ebase + (size_t)ed_src * stride;
-                return tr[((((size_t)ts * NVP + v) * E + src) * 2 + side) * NT + q];
-            };
-            double uf[M][NVP];
-#pragma unroll
-            for (int v = 0; v < NVP; v++) {
-                double p[N];
-#pragma unroll
-                for (int l = 0; l < N; l++) p[l] = us[v * TPE + spidx<N, DIM>(d, l, q)];
-#pragma unroll
-                for (int f = 0; f < M; f++) {
-                    double x = 0;
-#pragma unroll
-                    for (int l = 0; l < N; l++) x += p[l] * a.S2F[f * N + l];
-                    uf[f][v] = x;
-                }
-            }
-            double* Fd = Fs + d * NVP * G::FSZ;
-            // interior flux points
-#pragma unroll
-            for (int f = 1; f < M - 1; f++) {
-                double fl[NVP];
-                if (d == 0) state_flux<0>(uf[f], fl, a.gm);
-                else if (d == 1) state_flux<1>(uf[f], fl, a.gm);
-                else state_flux<2>(uf[f], fl, a.gm);
-#pragma unroll
-                for (int v = 0; v < NVP; v++) Fd[v * G::FSZ + fidx(d, f, q, N, NT, M)] = fl[v];
-            }
-            // the two faces: ghost values follow src/boundary.cpp:48-113
-            const int type = a.bc[d];
-            double bl[NVP], br[NVP];  // values the trace fill writes at (0, M-1) and (Nd-1, 0)
-#pragma unroll
-            for (int v = 0; v < NVP; v++) {
-                double sg = (type == SPDK_BC_REFLECTIVE && v == 1 + d) ? -1.0 : 1.0;
-                if (type == SPDK_BC_PERIODIC) {
-                    bl[v] = (ed == 1 || ed == 0) ? trace(Nd - 2, 1, v) : 0.0;
-                    br[v] = (ed == Nd - 2 || ed == Nd - 1) ? trace(1, 0, v) : 0.0;
-                } else {
-                    bl[v] = (ed == 1 || ed == 0) ? sg * trace(1, 0, v) : 0.0;
-                    br[v] = (ed == Nd - 2 || ed == Nd - 1) ? sg * trace(Nd - 2, 1, v) : 0.0;
-                }
-            }
+    constexpr int LOOP = MODE == FACES ? T : 1;  // slices one after the other
+    double dudt[NVP] = {0, 0, 0, 0, 0};
+#pragma unroll 1
+    for (int tl = 0; tl < LOOP; tl++) {
+        // ---- pencils
+        for (int i = (tid + 64 * ((bx + tl) % 4)) % G::BLOCK; i < DIM * X::UNITS * NT; i += G::BLOCK) {
+            const int d = i / (X::UNITS * NT), pu = i / NT % X::UNITS, q = i % NT;
+            const int pe = bx * EL + pu / S, pt = MODE == FACES ? tl : pu % S;
+            if (pe >= a.E) continue;
+            const double* U = a.in_ader ? a.U_in + (size_t)pt * a.in_nv * slabE : a.U_sp;
+            const int ts = a.tin_slices > 1 ? pt : 0;
+            double* F = lds + pu * X::AREA + X::SCR;
+            const int px = pe % a.Ne[0], py = (pe / a.Ne[0]) % a.Ne[1], pz = pe / (a.Ne[0] * a.Ne[1]);
             // the face integrals read faces 0..M-2 only: the upper face's
             // flux is formed when the flux-point array is written as well
-            const int nsides = (FVF && !a.F_out[d]) ? 1 : 2;
-            for (int side = 0; side < nsides; side++) {
-                double fl[NVP];
-                const int f = side ? M - 1 : 0;
-                bool raw = side ? (ed == Nd - 1) : (ed == 0);
-                if (raw) {
-                    if (d == 0) state_flux<0>(uf[f], fl, a.gm);
-                    else if (d == 1) state_flux<1>(uf[f], fl, a.gm);
-                    else state_flux<2>(uf[f], fl, a.gm);
-                } else {
-                    double uL[NVP], uR[NVP];
-#pragma unroll
-                    for (int v = 0; v < NVP; v++) {
-                        if (side == 0) {
-                            uL[v] = (ed - 1 == 0) ? bl[v] : trace(ed - 1, 1, v);
-                            uR[v] = (ed == Nd - 1) ? br[v] : uf[0][v];
-                        } else {
-                            uL[v] = (ed == 0) ? bl[v] : uf[M - 1][v];
-                            uR[v] = (ed + 1 == Nd - 1) ? br[v] : trace(ed + 1, 0, v);
-                        }
-                    }
-                    if (d == 0) riemann_llf<0>(uL, uR, fl, a.gm);
-                    else if (d == 1) riemann_llf<1>(uL, uR, fl, a.gm);
-                    else riemann_llf<2>(uL, uR, fl, a.gm);
-                }
-#pragma unroll
-                for (int v = 0; v < NVP; v++) Fd[v * G::FSZ + fidx(d, f, q, N, NT, M)] = fl[v];
-            }
+            if (d == 0) pencil<N, DIM, 0>(a, U, slabE, F, q, pe, px, ts, MODE == FACES && !a.F_out[0]);
+            if (DIM >= 2 && d == 1)
+                pencil<N, DIM, 1>(a, U, slabE, F + NVP * G::FSZ, q, pe, py, ts, MODE == FACES && !a.F_out[1]);
+            if (DIM == 3 && d == 2)
+                pencil<N, DIM, 2>(a, U, slabE, F + 2 * NVP * G::FSZ, q, pe, pz, ts, MODE == FACES && !a.F_out[2]);
         }
         __syncthreads();
-        if (FVF || a.flux_only) {  // the fluxes of slice t in the stage flux-point layout (src/hydro_ader.hpp:278-289)
-            if (FVF) fv_faces<N, DIM>(a, us, Fs, t, s, live, ei, ej, ek);
+        if (MODE == FACES || MODE == FLUXES) {  // the stage flux-point layout (src/hydro_ader.hpp:278-289)
+            const int t = MODE == FACES ? tl : ut;
+            if (MODE == FACES) fv_faces<N, DIM, X::AREA>(a, Fs - X::SCR, Fs, t, s, live, ei, ej, ek);
             if (live) {
 #pragma unroll
                 for (int d = 0; d < DIM; d++)
@@ -377,141 +425,171 @@ __global__ void __launch_bounds__(256) k_sweep(SweepArgs a) {
                         for (int v = NVP; v < a.out_nv; v++) o[(size_t)v * E * G::FSZ] = 0.0;
                     }
             }
-            __syncthreads();
-            continue;
+            if (MODE == FACES) __syncthreads();
         }
-        // ---- flux divergence at the solution points (src/transforms.cpp:301-307)
-        if (live) {
-            const int qx = DIM == 3 ? kk * N + jj : jj;
-            const int qy = DIM == 3 ? kk * N + ii : ii;
-            const int qz = jj * N + ii;
+    }
+    if (MODE == FACES || MODE == FLUXES) return;
+
+    // ---- flux divergence at the solution points (src/transforms.cpp:301-307)
+    if (live) {
+        const int qx = DIM == 3 ? kk * N + jj : jj;
+        const int qy = DIM == 3 ? kk * N + ii : ii;
+        const int qz = jj * N + ii;
+        bool recheck = false;
 #pragma unroll
-            for (int v = 0; v < NVP; v++) {
-                double acc = 0;
-                const double* Fx = Fs + v * G::FSZ;
-                const double* Fy = Fs + (NVP + v) * G::FSZ;
-                const double* Fz = Fs + (2 * NVP + v) * G::FSZ;
+        for (int v = 0; v < NVP; v++) {
+            double acc = 0;
+            const double* Fx = Fs + v * G::FSZ;
+            const double* Fy = Fs + (NVP + v) * G::FSZ;
+            const double* Fz = Fs + (2 * NVP + v) * G::FSZ;
 #pragma unroll
-                for (int l = 0; l < M; l++) {
-                    acc += Fx[fidx(0, l, qx, N, NT, M)] * Dx[l] / a.h[0];
-                    if (DIM >= 2) acc += Fy[fidx(1, l, qy, N, NT, M)] * Dy[l] / a.h[1];
-                    if (DIM == 3) acc += Fz[fidx(2, l, qz, N, NT, M)] * Dz[l] / a.h[2];
-                }
-                dudt[t][v] = acc;
+            for (int l = 0; l < M; l++) {
+                acc += div_fast(Fx[fidx(0, l, qx, N, NT, M)] * sD[ii * M + l], a.dh[0]);
+                if (DIM >= 2) acc += div_fast(Fy[fidx(1, l, qy, N, NT, M)] * sD[jj * M + l], a.dh[1]);
+                if (DIM == 3) acc += div_fast(Fz[fidx(2, l, qz, N, NT, M)] * sD[kk * M + l], a.dh[2]);
             }
-            if (a.grav && !a.out_pred) {
-                // update_solution's gravity source (src/transforms.cpp:17-27,
-                // :364-367) from the ADER slice staged in LDS: rho g and m . g
-                const double rho = us[s], m1 = us[TPE + s], m2 = us[2 * TPE + s], m3 = us[3 * TPE + s];
-                dudt[t][1] -= rho * a.g[0];
-                dudt[t][2] -= rho * a.g[1];
-                dudt[t][3] -= rho * a.g[2];
-                dudt[t][4] -= m1 * a.g[0] + m2 * a.g[1] + m3 * a.g[2];
-            }
-            if (a.F_x && !a.out_pred) {  // x flux-point fluxes of the final sweep (outputs)
-                for (int idx = s; idx < G::FSZ; idx += TPE) {
-                    size_t o = (((size_t)t * NV) * E + e) * G::FSZ + idx;
+            dudt[v] = acc;
+            recheck = recheck || div_recheck(acc);
+        }
+        if (recheck)
 #pragma unroll
-                    for (int v = 0; v < NVP; v++) a.F_x[o + (size_t)v * E * G::FSZ] = Fs[v * G::FSZ + idx];
-                    a.F_x[o + (size_t)NVP * E * G::FSZ] = 0.0;
-                }
+            for (int v = 0; v < NVP; v++) dudt[v] = divergence_slow<N, DIM>(a, Fs, sD, v, ii, jj, kk);
+        if (a.grav && MODE == CORRECT) {
+            // update_solution's gravity source (src/transforms.cpp:17-27,
+            // :364-367) from the ADER slice: rho g and m . g
+            const double* U = (a.in_ader ? a.U_in + (size_t)ut * a.in_nv * slabE : a.U_sp) + (size_t)e * TPE + s;
+            const double rho = U[0], m1 = U[slabE], m2 = U[2 * slabE], m3 = U[3 * slabE];
+            dudt[1] -= rho * a.g[0];
+            dudt[2] -= rho * a.g[1];
+            dudt[3] -= rho * a.g[2];
+            dudt[4] -= m1 * a.g[0] + m2 * a.g[1] + m3 * a.g[2];
+        }
+        if (MODE == CORRECT && a.F_x) {  // x flux-point fluxes of the final sweep (outputs)
+            for (int idx = s; idx < G::FSZ; idx += TPE) {
+                size_t o = (((size_t)ut * NV) * E + e) * G::FSZ + idx;
+#pragma unroll
+                for (int v = 0; v < NVP; v++) a.F_x[o + (size_t)v * E * G::FSZ] = Fs[v * G::FSZ + idx];
+                a.F_x[o + (size_t)NVP * E * G::FSZ] = 0.0;
+            }
+        }
+    }
+    double u_old[NVP];
+#pragma unroll
+    for (int v = 0; v < NVP; v++) u_old[v] = live ? a.U_sp[(size_t)v * slabE + (size_t)e * TPE + s] : 0.0;
+    __syncthreads();  // the fluxes have been read
+
+    // ---- the slices' divergences meet in the flux area of each element's units
+    double* const mine = Fs;                    // this unit's divergence, then its exchange area
+    const double* const own0 = Fs - ut * X::AREA;  // the element's unit of slice 0
+    if (S > 1) {
+        if (live)
+#pragma unroll
+            for (int v = 0; v < NVP; v++) mine[v * TPE + s] = dudt[v];
+        __syncthreads();
+    }
+    auto rate = [&](int l, int v) -> double { return S > 1 ? own0[l * X::AREA + v * TPE + s] : dudt[v]; };
+
+    if (MODE == PREDICT) {
+        // ---- predictor (src/transforms.cpp:316-322): slices ut + k S of this thread
+        constexpr int OWN = T / S;  // slices this thread forms
+        constexpr int UO = S > 1 ? G::LDS_U : 0;  // new slices in LDS, behind the divergences
+        auto slice_at = [&](int t) -> double* {   // area of new slice t of this element
+            return S > 1 ? const_cast<double*>(own0) + t * X::AREA + UO : Fs + t * G::LDS_U;
+        };
+        if (!a.grav) {
+#pragma unroll
+            for (int k = 0; k < OWN; k++) {
+                const int t = S > 1 ? ut : k;
+                if (live)
+#pragma unroll
+                    for (int v = 0; v < NVP; v++) {
+                        double du = 0;
+#pragma unroll
+                        for (int l = 0; l < T; l++) du += rate(l, v) * a.inv[t * T + l] * a.w[l] * a.dt;
+                        const double un = u_old[v] - du;
+                        a.U_out[((size_t)t * NVP + v) * slabE + (size_t)e * TPE + s] = un;
+                        slice_at(t)[v * TPE + s] = un;
+                    }
+            }
+        } else {
+            // With gravity (src/transforms.cpp:17-27, :309-313) update_prediction
+            // writes U_ader variable by variable and its source reads U_ader
+            // back: the momenta's source takes the density just written, the
+            // energy's the momenta just written. Each group goes through LDS.
+#pragma unroll 1
+            for (int grp = 0; grp < 3; grp++) {
+                const int v0 = grp == 0 ? 0 : (grp == 1 ? 1 : 4), v1 = grp == 0 ? 1 : (grp == 1 ? 4 : 5);
+                if (live)
+#pragma unroll
+                    for (int k = 0; k < OWN; k++) {
+                        const int t = S > 1 ? ut : k;
+#pragma unroll
+                        for (int v = 0; v < NVP; v++) {
+                            if (v < v0 || v >= v1) continue;
+                            double du = 0;
+#pragma unroll
+                            for (int l = 0; l < T; l++) {
+                                const double* n = slice_at(l) + s;
+                                double r = rate(l, v);
+                                if (v >= 1 && v <= 3) r -= n[0] * a.g[v - 1];
+                                if (v == 4) r -= n[TPE] * a.g[0] + n[2 * TPE] * a.g[1] + n[3 * TPE] * a.g[2];
+                                du += r * a.inv[t * T + l] * a.w[l] * a.dt;
+                            }
+                            const double un = u_old[v] - du;
+                            a.U_out[((size_t)t * NVP + v) * slabE + (size_t)e * TPE + s] = un;
+                            slice_at(t)[v * TPE + s] = un;
+                        }
+                    }
+                __syncthreads();
             }
         }
         __syncthreads();
-    }
-    if (FVF || a.flux_only) return;
-    if (!a.in_ader) {
+        // ---- traces of the new slices, axis by axis over (slice, element)
+        for (int i = tid; i < DIM * T * EL * NT; i += G::BLOCK) {
+            const int d = i / (T * EL * NT), t = i / (EL * NT) % T, pl = i / NT % EL, q = i % NT;
+            const int pe = bx * EL + pl;
+            if (pe >= a.E) continue;
+            const double* un = S > 1 ? lds + (pl * S + t) * X::AREA + UO : lds + pl * X::AREA + t * G::LDS_U;
+            const int l0 = d == 0 ? spidx<N, DIM>(0, 0, q) : (d == 1 ? spidx<N, DIM>(1, 0, q) : spidx<N, DIM>(2, 0, q));
+            const int ls = d == 0 ? 1 : (d == 1 ? N : N * N);
+            double* tr = d == 0 ? a.tr_out[0] : (d == 1 ? a.tr_out[1] : a.tr_out[2]);
 #pragma unroll
-        for (int t = 1; t < T; t++)
+            for (int v = 0; v < NVP; v++) {
+                double p[N];
 #pragma unroll
-            for (int v = 0; v < NVP; v++) dudt[t][v] = dudt[0][v];
-    }
-
-    if (a.out_pred && a.grav && live) {
-        // update_prediction's gravity source (src/transforms.cpp:17-27,
-        // :309-313). That kernel writes U_ader variable by variable, and the
-        // source reads U_ader back: the momenta's source takes the density
-        // just written, the energy's the momenta just written. Those values
-        // are formed here exactly as the predictor below forms them.
-        double rn[T];
+                for (int l = 0; l < N; l++) p[l] = un[v * TPE + l0 + l * ls];
+                double x0 = 0, x1 = 0;
 #pragma unroll
-        for (int t = 0; t < T; t++) {
-            double du = 0;
+                for (int l = 0; l < N; l++) x0 += p[l] * a.S2F[l];
 #pragma unroll
-            for (int l = 0; l < T; l++) du += dudt[l][0] * a.inv[t * T + l] * a.w[l] * a.dt;
-            rn[t] = u_old[0] - du;
-        }
-        double mn[T][3];
-#pragma unroll
-        for (int v = 1; v <= 3; v++) {
-#pragma unroll
-            for (int t = 0; t < T; t++) dudt[t][v] -= rn[t] * a.g[v - 1];
-#pragma unroll
-            for (int t = 0; t < T; t++) {
-                double du = 0;
-#pragma unroll
-                for (int l = 0; l < T; l++) du += dudt[l][v] * a.inv[t * T + l] * a.w[l] * a.dt;
-                mn[t][v - 1] = u_old[v] - du;
+                for (int l = 0; l < N; l++) x1 += p[l] * a.S2F[(M - 1) * N + l];
+                double* to = tr + (((size_t)t * NVP + v) * E + pe) * 2 * NT + q;
+                to[0] = x0;
+                to[NT] = x1;
             }
-        }
-#pragma unroll
-        for (int t = 0; t < T; t++) dudt[t][4] -= mn[t][0] * a.g[0] + mn[t][1] * a.g[1] + mn[t][2] * a.g[2];
-    }
-    if (a.out_pred) {
-        // ---- predictor (src/transforms.cpp:316-322) and traces of the new slices
-#pragma unroll
-        for (int t = 0; t < T; t++) {
-            if (live) {
-#pragma unroll
-                for (int v = 0; v < NVP; v++) {
-                    double du = 0;
-#pragma unroll
-                    for (int l = 0; l < T; l++) du += dudt[l][v] * a.inv[t * T + l] * a.w[l] * a.dt;
-                    double un = u_old[v] - du;
-                    a.U_out[((size_t)t * NVP + v) * slabE + (size_t)e * TPE + s] = un;
-                    us[v * TPE + s] = un;
-                }
-            }
-            __syncthreads();
-            for (int task = s; live && task < DIM * NT; task += TPE) {
-                const int d = task / NT, q = task % NT;
-#pragma unroll
-                for (int v = 0; v < NVP; v++) {
-                    double p[N];
-#pragma unroll
-                    for (int l = 0; l < N; l++) p[l] = us[v * TPE + spidx<N, DIM>(d, l, q)];
-                    double x0 = 0, x1 = 0;
-#pragma unroll
-                    for (int l = 0; l < N; l++) x0 += p[l] * a.S2F[l];
-#pragma unroll
-                    for (int l = 0; l < N; l++) x1 += p[l] * a.S2F[(M - 1) * N + l];
-                    double* to = a.tr_out[d] + ((((size_t)t * NVP + v) * E + e) * 2) * NT + q;
-                    to[0] = x0;
-                    to[NT] = x1;
-                }
-            }
-            __syncthreads();
         }
         return;
     }
 
-    // ---- corrector (src/transforms.cpp:354-372), optional SSP combine
+    // ---- corrector (src/transforms.cpp:354-372), optional SSP combine: the
+    // element's slice-0 threads
+    const bool lead = live && ut == 0;
     double un[NVP];
-#pragma unroll
-    for (int v = 0; v < NVP; v++) {
-        double du = 0;
-#pragma unroll
-        for (int t = 0; t < T; t++) du += dudt[t][v] * a.w[t] * a.dt;
-        un[v] = u_old[v] - du;
-    }
-    if (a.rk_a != 0.0 && live) {  // combine_solution (src/transforms.cpp:252-261)
+    if (lead) {
 #pragma unroll
         for (int v = 0; v < NVP; v++) {
-            double u0 = a.U0[(size_t)v * slabE + (size_t)e * TPE + s];
-            un[v] = a.rk_a * u0 + (1.0 - a.rk_a) * un[v];
+            double du = 0;
+#pragma unroll
+            for (int t = 0; t < T; t++) du += rate(t, v) * a.w[t] * a.dt;
+            un[v] = u_old[v] - du;
         }
-    }
-    if (live) {
+        if (a.rk_a != 0.0) {  // combine_solution (src/transforms.cpp:252-261)
+#pragma unroll
+            for (int v = 0; v < NVP; v++) {
+                double u0 = a.U0[(size_t)v * slabE + (size_t)e * TPE + s];
+                un[v] = a.rk_a * u0 + (1.0 - a.rk_a) * un[v];
+            }
+        }
 #pragma unroll
         for (int v = 0; v < NVP; v++) {
             if (a.rk_first) a.U0[(size_t)v * slabE + (size_t)e * TPE + s] = u_old[v];
@@ -519,24 +597,22 @@ __global__ void __launch_bounds__(256) k_sweep(SweepArgs a) {
         }
     }
     if (!a.want_dt) return;
-    // ---- cv primitives: compute_primitives then sp->cv sweeps x, y, z
-    double* wa = us;  // ping (state area, free by now)
-    double* wb = Fs;  // pong
-    if (live) {
+    // ---- cv primitives: compute_primitives then sp->cv sweeps x, y, z, the
+    // variables shared out over the element's units
+    double* src = const_cast<double*>(own0) + G::LDS_U;  // clear of the divergences (slice 0's area)
+    double* dst = const_cast<double*>(own0);
+    if (lead) {
         double wv[NVP];
         prim(un, wv, a.gm);
 #pragma unroll
-        for (int v = 0; v < NVP; v++) wa[v * TPE + s] = wv[v];
+        for (int v = 0; v < NVP; v++) src[v * TPE + s] = wv[v];
     }
     __syncthreads();
-    double* src = wa;
-    double* dst = wb;
 #pragma unroll
     for (int d = 0; d < DIM; d++) {
         if (live) {
             const int id = d == 0 ? ii : (d == 1 ? jj : kk);
-#pragma unroll
-            for (int v = 0; v < NVP; v++) {
+            for (int v = ut; v < NVP; v += S) {
                 double x = 0;
 #pragma unroll
                 for (int l = 0; l < N; l++) {
@@ -553,7 +629,7 @@ __global__ void __launch_bounds__(256) k_sweep(SweepArgs a) {
     }
     // src now holds W_cv of the element
     double r = __builtin_inf();
-    if (live) {
+    if (lead) {
         double wc[NVP];
 #pragma unroll
         for (int v = 0; v < NVP; v++) wc[v] = src[v * TPE + s];
@@ -573,15 +649,12 @@ __global__ void __launch_bounds__(256) k_sweep(SweepArgs a) {
             r = a.cfl * dx_min / c_max / N;
         }
     }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) r = nan_min(r, __shfl_xor(r, o));
     __syncthreads();
-    double* red = lds;
-    red[tid] = r;
+    if (tid % 64 == 0) lds[tid / 64] = r;
     __syncthreads();
-    for (int wdt = G::BLOCK / 2; wdt > 0; wdt >>= 1) {
-        if (tid < wdt) red[tid] = nan_min(red[tid], red[tid + wdt]);
-        __syncthreads();
-    }
-    if (tid == 0) a.part[blockIdx.x] = red[0];
+    if (tid == 0) a.part[blockIdx.x] = nan_min(nan_min(lds[0], lds[1]), nan_min(lds[2], lds[3]));
 }
 
 // Face traces of slice blockIdx.y of U (in_nv variables per slice): of the
@@ -625,20 +698,23 @@ __global__ void __launch_bounds__(256) k_trace0(const double* __restrict__ U, in
     }
 }
 
-__global__ void k_partial_min(double* part, int n) {
-    __shared__ double red[1024];
+// Minimum of part[0, n) over the grid: out[blockIdx.x] per workgroup.
+__global__ void __launch_bounds__(1024) k_partial_min(const double* part, int n, double* out) {
+    __shared__ double red[16];
     double r = __builtin_inf();
-    for (int i = threadIdx.x; i < n; i += blockDim.x) r = nan_min(r, part[i]);
-    red[threadIdx.x] = r;
+    for (int i = blockIdx.x * 1024 + threadIdx.x; i < n; i += gridDim.x * 1024) r = nan_min(r, part[i]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) r = nan_min(r, __shfl_xor(r, o));
+    if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = r;
     __syncthreads();
-    for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] = nan_min(red[threadIdx.x], red[threadIdx.x + w]);
-        __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 16; w++) r = nan_min(r, red[w]);
+        out[blockIdx.x] = r;
     }
-    if (threadIdx.x == 0) part[0] = red[0];
 }
 
 // ---------------------------------------------------------------------------
+constexpr int kMinBlocks = 256;  // workgroups of the first of two dt reductions
 struct Layout {
     size_t E = 0, tpe = 0, nt = 0, T = 0, dim = 0;
     size_t off_uader = 0, off_trA = 0, off_trB = 0, off_u0 = 0, off_part = 0, total = 0;
@@ -655,7 +731,7 @@ Layout layout_for(size_t E, int T) {
     L.nt = G::NT;
     L.T = T;
     L.dim = DIM;
-    L.blocks = (unsigned)((E + G::EPB - 1) / G::EPB);
+    L.blocks = (unsigned)((E + G::EPB / T - 1) / (G::EPB / T));  // of a sweep with every slice (T = 1: one)
     size_t st = (size_t)T * NVP * E * G::TPE;
     L.tr_axis = (size_t)T * NVP * E * 2 * G::NT;
     size_t o = 0;
@@ -663,7 +739,7 @@ Layout layout_for(size_t E, int T) {
     L.off_trA = o; o += DIM * L.tr_axis;
     L.off_trB = o; o += DIM * L.tr_axis;
     L.off_u0 = o; o += (size_t)NVP * E * G::TPE;
-    L.off_part = o; o += L.blocks + 64;
+    L.off_part = o; o += L.blocks + kMinBlocks;
     L.total = o;
     return L;
 }
@@ -726,6 +802,7 @@ int run_step(spdk_ctx* c, double* U_sp, const int Ne[3], void* ws, double dt, do
         a.act[d] = c->prm.active[d];
         a.bc[d] = c->prm.bc[d];
         a.h[d] = c->prm.h[d];
+        a.dh[d] = const_div(c->prm.h[d]);
     }
     a.E = (int)E;
     a.in_nv = NVP;
@@ -734,19 +811,38 @@ int run_step(spdk_ctx* c, double* U_sp, const int Ne[3], void* ws, double dt, do
     a.cfl = c->prm.cfl;
     for (int d = 0; d < 3; d++) a.g[d] = c->prm.g[d];
     a.grav = (a.g[0] != 0.0 || a.g[1] != 0.0 || a.g[2] != 0.0);
-    size_t lds = sizeof(double) * (size_t)G::EPB * G::LDS_ELEM;
-    if (lds < sizeof(double) * G::BLOCK) lds = sizeof(double) * G::BLOCK;
-    dim3 grid(L.blocks), block(G::BLOCK);
+    const unsigned eblocks = (unsigned)((E + G::EPB - 1) / G::EPB);  // workgroups of whole elements, one slice
+    dim3 grid(eblocks), block(G::BLOCK);
     // timing: one event pair per sweep launch, harvested after the step's own sync
-    auto launch_sweep = [&](const SweepArgs& args) -> int {
+    auto launch_sweep = [&](auto mode_, const SweepArgs& args) -> int {
+        constexpr int mode = decltype(mode_)::value;
+        constexpr int ST = T > 1 ? T : 1;
         bool rec = c->timing && !x && c->ev_used < spdk_ctx::kEvPool;
         if (rec) SPDK_CHECK(hipEventRecord(c->evs[c->ev_used][0], c->stream));
-        if (args.Ffv[0][0])
-            hipLaunchKernelGGL((k_sweep<N, DIM, T, true>), dim3((L.blocks + 7) / 8 * 8), block, lds, c->stream, args);
-        else
-            hipLaunchKernelGGL((k_sweep<N, DIM, T, false>), grid, block, lds, c->stream, args);
+        auto go = [&](auto slices) {
+            constexpr int S = decltype(slices)::value;
+            using X = Unit<N, DIM, T, S, mode>;
+            unsigned nb = S == 1 ? eblocks : L.blocks;
+            if (mode == FACES) nb = (nb + 7) / 8 * 8;
+            hipLaunchKernelGGL((k_sweep<N, DIM, T, S, mode>), dim3(nb), block, sizeof(double) * X::DOUBLES, c->stream, args);
+        };
+        if constexpr (mode == FACES || ST == 1) go(std::integral_constant<int, 1>{});
+        else if constexpr (mode == PREDICT) {
+            if (args.in_ader) go(std::integral_constant<int, ST>{});
+            else go(std::integral_constant<int, 1>{});
+        } else go(std::integral_constant<int, ST>{});
         SPDK_LAUNCH_CHECK("k_sweep");
         if (rec) SPDK_CHECK(hipEventRecord(c->evs[c->ev_used++][1], c->stream));
+        return SPDK_OK;
+    };
+    constexpr std::integral_constant<int, PREDICT> predict{};
+    constexpr std::integral_constant<int, CORRECT> correct{};
+    // the flux evaluation of the slices: face integrals, or flux-point arrays alone
+    auto launch_fluxes = [&](const SweepArgs& args) -> int {
+        if constexpr (T > 1) {
+            if (args.Ffv[0][0]) return launch_sweep(std::integral_constant<int, FACES>{}, args);
+            return launch_sweep(std::integral_constant<int, FLUXES>{}, args);
+        }
         return SPDK_OK;
     };
     auto traces0 = [&]() -> int {
@@ -765,7 +861,7 @@ int run_step(spdk_ctx* c, double* U_sp, const int Ne[3], void* ws, double dt, do
     if (T > 1 && x && x->U_slices) {  // flux evaluation of given slices: their traces, then one flux sweep
         double* trS[3] = {nullptr, nullptr, nullptr};
         for (int d = 0; d < DIM; d++) trS[d] = W + (size_t)d * L.tr_axis;
-        hipLaunchKernelGGL((k_trace0<N, DIM>), dim3(L.blocks, T), block, 0, c->stream, x->U_slices, x->slices_nv, trS[0],
+        hipLaunchKernelGGL((k_trace0<N, DIM>), dim3(eblocks, T), block, 0, c->stream, x->U_slices, x->slices_nv, trS[0],
                            trS[1], trS[2], a.S2F, (int)E);
         SPDK_LAUNCH_CHECK("k_trace0");
         SweepArgs s = a;
@@ -776,10 +872,9 @@ int run_step(spdk_ctx* c, double* U_sp, const int Ne[3], void* ws, double dt, do
         s.in_ader = 1;
         s.U_in = x->U_slices;
         s.in_nv = x->slices_nv;
-        s.flux_only = 1;
         s.out_nv = x->out_nv;
         set_fv(s);
-        return launch_sweep(s);
+        return launch_fluxes(s);
     }
     if (T > 1) {  // ADER: K = T sweeps, the last one with the corrector (or the flux evaluation)
         if ((rc = traces0())) return rc;
@@ -794,7 +889,6 @@ int run_step(spdk_ctx* c, double* U_sp, const int Ne[3], void* ws, double dt, do
             s.in_ader = k > 0;
             s.U_in = W + L.off_uader;
             s.U_out = W + L.off_uader;
-            s.out_pred = !last;
             s.want_dt = last;
             s.W_cv = last ? W_cv : nullptr;
             s.F_x = last ? F_x : nullptr;
@@ -802,14 +896,15 @@ int run_step(spdk_ctx* c, double* U_sp, const int Ne[3], void* ws, double dt, do
                 s.want_dt = 0;
                 s.W_cv = nullptr;
                 s.F_x = nullptr;
-                s.flux_only = 1;
                 s.out_nv = x->out_nv;
                 for (int d = 0; d < 3; d++) s.F_out[d] = x->F_out[d];
                 set_fv(s);
+                return launch_fluxes(s);
             }
-            if ((rc = launch_sweep(s))) return rc;
+            if constexpr (T > 1) {
+                if ((rc = last ? launch_sweep(correct, s) : launch_sweep(predict, s))) return rc;
+            }
         }
-        if (flux_out) return SPDK_OK;
         if (pred_only) {
             const size_t slabE = E * G::TPE, total = (size_t)T * x->nv_export * slabE;
             hipLaunchKernelGGL(k_export_ader, dim3((unsigned)std::min<size_t>((total + 255) / 256, 65536)), dim3(256), 0,
@@ -828,19 +923,29 @@ int run_step(spdk_ctx* c, double* U_sp, const int Ne[3], void* ws, double dt, do
             for (int d = 0; d < 3; d++) { s.tr_in[d] = trA[d]; s.tr_out[d] = nullptr; }
             s.tin_slices = 1;
             s.in_ader = 0;
-            s.out_pred = 0;
             s.rk_a = rk[st];
             s.rk_first = st == 0 && order > 1;
             bool last = st == order - 1;
             s.want_dt = last;
             s.W_cv = last ? W_cv : nullptr;
             s.F_x = last ? F_x : nullptr;
-            if ((rc = launch_sweep(s))) return rc;
+            if constexpr (T == 1) {
+                if ((rc = launch_sweep(correct, s))) return rc;
+            }
         }
     }
-    hipLaunchKernelGGL(k_partial_min, dim3(1), dim3(1024), 0, c->stream, a.part, (int)L.blocks);
+    // one workgroup reads up to 16 k minima in about 5 us; more go through 256
+    // first (64^3: 36 us in one). The result is written to the host's page.
+    const double* mins = a.part;
+    int nmin = (int)L.blocks;
+    if (nmin > 16384) {
+        hipLaunchKernelGGL(k_partial_min, dim3(kMinBlocks), dim3(1024), 0, c->stream, mins, nmin, a.part + L.blocks);
+        SPDK_LAUNCH_CHECK("k_partial_min");
+        mins = a.part + L.blocks;
+        nmin = kMinBlocks;
+    }
+    hipLaunchKernelGGL(k_partial_min, dim3(1), dim3(1024), 0, c->stream, mins, nmin, c->red_host);
     SPDK_LAUNCH_CHECK("k_partial_min");
-    SPDK_CHECK(hipMemcpyAsync(c->red_host, a.part, sizeof(double), hipMemcpyDeviceToHost, c->stream));
     SPDK_CHECK(hipStreamSynchronize(c->stream));
     if (dt_next) *dt_next = c->red_host[0];
     for (int i = 0; i < c->ev_used; i++) {

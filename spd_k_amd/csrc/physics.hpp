@@ -97,8 +97,10 @@ __device__ __forceinline__ void state_flux(const double* u, double* f, double gm
 
 // Local Lax-Friedrichs flux (src/hydro.cpp:270-289) for the physical
 // variables; the slot flux is -0.5*c*(0-0) = +0 and is not carried.
+// own: the physical flux of the one state that both sides hold (the outer face
+// of a ghost element).
 template <int D>
-__device__ __forceinline__ void riemann_llf(const double* uL, const double* uR, double* F, double gm) {
+__device__ __forceinline__ void riemann_llf(const double* uL, const double* uR, double* F, double gm, bool own = false) {
     constexpr int V1 = 1 + D;
     double wL[NVP], wR[NVP], fL[NVP], fR[NVP];
     prim(uL, wL, gm);
@@ -109,7 +111,7 @@ __device__ __forceinline__ void riemann_llf(const double* uL, const double* uR, 
     double cR = sound_speed(wR[0], wR[4], gm) + fabs(wR[V1]);
     double c = smax(cL, cR);
 #pragma unroll
-    for (int v = 0; v < NVP; v++) F[v] = 0.5 * (fR[v] + fL[v]) - 0.5 * c * (uR[v] - uL[v]);
+    for (int v = 0; v < NVP; v++) F[v] = own ? fL[v] : 0.5 * (fR[v] + fL[v]) - 0.5 * c * (uR[v] - uL[v]);
 }
 
 // HLLC flux (src/hydro.cpp:291-363); the slot entry is zero.
