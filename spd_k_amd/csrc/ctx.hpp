@@ -5,6 +5,7 @@
 #include <string>
 #include <vector>
 #include "../../include/spdk.h"
+#include "physics.hpp"
 
 struct spdk_ctx {
     spdk_params prm;
@@ -21,6 +22,9 @@ struct spdk_ctx {
     double* fvf[3] = {};
     double* fvc[3] = {};
     int fvnf[3] = {}, fvn[3] = {};
+    // widths of the FV sub-grid with their divisions (spdk::ConstDiv), per axis: c[l+1] - c[l],
+    // c[l+1] - c[l-1] and f[l+1] - f[l] of centers c and faces f, at index l
+    spdk::ConstDiv *fvdc1[3] = {}, *fvdc2[3] = {}, *fvdf[3] = {};
     double* red = nullptr;       // reduction partials (device)
     double* red_host = nullptr;  // pinned host landing slot
     int red_blocks = 2048;

@@ -4,6 +4,7 @@
 // restates the reference function cited at its launcher.
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <type_traits>
 #include "ctx.hpp"
 #include "physics.hpp"
 
@@ -43,6 +44,8 @@ __device__ __forceinline__ uint32_t xcd_block() { return (blockIdx.x % kXcd) * (
 struct Geo {  // FV sub-grid coordinates per axis (device pointers)
     const double* f[3];
     const double* c[3];
+    // widths with their divisions: c[l+1] - c[l], c[l+1] - c[l-1], f[l+1] - f[l] at index l
+    const ConstDiv *dc1[3], *dc2[3], *df[3];
 };
 
 // ---------------------------------------------------------------------------
@@ -775,6 +778,40 @@ __device__ __forceinline__ double alpha_fn(double dv, double dUm, double dU, dou
     aR = (dv == 0.0 ? 1.0 : aR);
     return smin(aL, aR);
 }
+// alpha_fn(...) >= 1 without its divisions: for finite operands a rounded
+// quotient of two numbers of one sign is at least 1 exactly where the
+// numerator is at least as large, and with a NaN anywhere both forms are true
+// (smin(1, NaN) is 1).
+__device__ __forceinline__ bool alpha_ge1(double dv, double dUm, double dU, double dUp) {
+    const double vL = dU - dUm, vR = dUp - dU;
+    if (dv < 0.0) return !(smin(vL, 0.0) > dv) && !(smin(vR, 0.0) > dv);
+    return !(smax(vL, 0.0) < dv) && !(smax(vR, 0.0) < dv);
+}
+// The SED's difference quotients at a cell (src/trouble_detection.cpp:121-140)
+// from W_new at -2 .. +2 along an axis: central, upper and lower slope and the
+// second-derivative bound dv. h, hp, hm: distances of the centers -1 to +1, 0
+// to +2, -2 to 0; df: the cell's width.
+struct Sed {
+    double dU, dUp, dUm, dv;
+};
+// EXACT: by division; else in three instructions each, recheck set where a
+// quotient may be inexact.
+template <bool EXACT>
+__device__ __forceinline__ Sed sed_slopes(double wm2, double wm1, double u, double wp1, double wp2, const ConstDiv& h,
+                                          const ConstDiv& hp, const ConstDiv& hm, double df, bool& recheck) {
+    auto div = [&](double x, const ConstDiv& c) -> double {
+        if (EXACT) return x / c.h;
+        const double q = div_fast(x, c);
+        recheck = recheck || div_recheck(q);
+        return q;
+    };
+    Sed r;
+    r.dU = div(wp1 - wm1, h);
+    r.dUp = div(wp2 - u, hp);
+    r.dUm = div(u - wm2, hm);
+    r.dv = 0.5 * div(r.dUp - r.dUm, h) * df;
+    return r;
+}
 struct Det {
     int act[3];
     int moore, delta, use_sed, pad, mask;
@@ -844,24 +881,20 @@ __global__ void __launch_bounds__(BS) k_nad_sed(const double* __restrict__ Wn, c
 #pragma unroll
             for (int d = 0; d < 3; d++) {
                 if (!(d == 0 ? AX : (d == 1 ? AY : AZ))) continue;
-                const double* c = geo.c[d];
-                const double* f = geo.f[d];
                 const int l = d == 0 ? i : (d == 1 ? j : k);
                 const long st = d == 0 ? 1 : (d == 1 ? sy : sz);
-                double h = (c[l + 1] - c[l - 1]);
-                double hp = (c[l + 2] - c[l]);
-                double hm = (c[l] - c[l - 2]);
-                double du = (wn[st] - wn[-st]) / h;
-                double dup = (wn[2 * st] - u) / hp;
-                double dum = (u - wn[-2 * st]) / hm;
-                double d2u = (dup - dum) / (c[l + 1] - c[l - 1]);
-                double dv = 0.5 * d2u * (f[l + 1] - f[l]);
-                const double al_v = alpha_fn(dv, dum, du, dup);
+                const ConstDiv* c2 = geo.dc2[d];
+                bool recheck = false;
+                Sed q = sed_slopes<false>(wn[-2 * st], wn[-st], u, wn[st], wn[2 * st], c2[l], c2[l + 1], c2[l - 1],
+                                          geo.df[d][l].h, recheck);
+                if (recheck)
+                    q = sed_slopes<true>(wn[-2 * st], wn[-st], u, wn[st], wn[2 * st], c2[l], c2[l + 1], c2[l - 1],
+                                         geo.df[d][l].h, recheck);
                 if (BITS) {
-                    if (al_v >= 1.0) bits |= 1u << (v * 3 + d);
+                    if (alpha_ge1(q.dv, q.dUm, q.dU, q.dUp)) bits |= 1u << (v * 3 + d);
                 } else {
                     double* al = d == 0 ? alx : (d == 1 ? aly : alz);
-                    al[v * pl + c0] = al_v;
+                    al[v * pl + c0] = alpha_fn(q.dv, q.dUm, q.dU, q.dUp);
                 }
             }
         }
@@ -878,9 +911,11 @@ __global__ void __launch_bounds__(BS) k_nad_sed(const double* __restrict__ Wn, c
 // as in k_nad_sed, and the box's max and min by plane (each plane reduced
 // once, in (y, x) order, then the three planes): for finite values max and
 // min are exact in any grouping, so the flags are the same; a non-finite
-// state stops the run at the next dt anyway.
+// state stops the run at the next dt anyway. Without the SED's divisions (12
+// of a cell's 24 by grid widths, the others comparisons) a call at 62 x 66 x 61
+// elements p=3 takes 0.59 ms instead of 0.81; 0.2 ms would be its bytes.
 template <int KC>
-__global__ void __launch_bounds__(BS) k_nad_sed_z(const double* __restrict__ Wn, const double* __restrict__ Wo,
+__global__ void __launch_bounds__(BS, 4) k_nad_sed_z(const double* __restrict__ Wn, const double* __restrict__ Wo,
                                                   double* __restrict__ tr, uint16_t* __restrict__ abits, FV s, Det a,
                                                   Geo geo, uint32_t total) {
     uint32_t idx = xcd_block() * BS + threadIdx.x;
@@ -945,33 +980,26 @@ __global__ void __launch_bounds__(BS) k_nad_sed_z(const double* __restrict__ Wn,
                 tr[v * pl + ((size_t)k * s.Ny + j) * s.Nx + i] = (un > mx || un < mn) ? 1.0 : 0.0;
             }
             if (sed && k >= 2 && k <= s.Nz - 3) {
-                double u = Z[2];
+                // x and y neighbours are loaded before the first slope
+                const double wx[5] = {n[-2], n[-1], Z[2], n[1], n[2]};
+                const double wy[5] = {n[-2 * sy], n[-sy], Z[2], n[sy], n[2 * sy]};
+                uint32_t r = 0;
 #pragma unroll
                 for (int d = 0; d < 3; d++) {
-                    const double* c = geo.c[d];
-                    const double* f = geo.f[d];
                     const int l = d == 0 ? i : (d == 1 ? j : k);
-                    double wm2, wm1, wp1, wp2;
-                    if (d == 2) {
-                        wm2 = Z[0]; wm1 = Z[1]; wp1 = Z[3]; wp2 = Z[4];
-                    } else {
-                        const long st = d == 0 ? 1 : sy;
-                        wm2 = n[-2 * st]; wm1 = n[-st]; wp1 = n[st]; wp2 = n[2 * st];
-                    }
-                    double h = (c[l + 1] - c[l - 1]);
-                    double hp = (c[l + 2] - c[l]);
-                    double hm = (c[l] - c[l - 2]);
-                    double du = (wp1 - wm1) / h;
-                    double dup = (wp2 - u) / hp;
-                    double dum = (u - wm2) / hm;
-                    double d2u = (dup - dum) / (c[l + 1] - c[l - 1]);
-                    double dv = 0.5 * d2u * (f[l + 1] - f[l]);
-                    if (alpha_fn(dv, dum, du, dup) >= 1.0) {
-                        const uint64_t bit = 1ull << (16 * (kk & 3) + v * 3 + d);
-                        if (kk < 4) bits[0] |= bit;
-                        else bits[1] |= bit;
-                    }
+                    const double* w = d == 0 ? wx : (d == 1 ? wy : Z);
+                    const ConstDiv* c2 = geo.dc2[d];
+                    bool recheck = false;
+                    Sed q = sed_slopes<false>(w[0], w[1], w[2], w[3], w[4], c2[l], c2[l + 1], c2[l - 1],
+                                              geo.df[d][l].h, recheck);
+                    if (recheck)
+                        q = sed_slopes<true>(w[0], w[1], w[2], w[3], w[4], c2[l], c2[l + 1], c2[l - 1],
+                                             geo.df[d][l].h, recheck);
+                    if (alpha_ge1(q.dv, q.dUm, q.dU, q.dUp)) r |= 1u << d;
                 }
+                const uint64_t word = (uint64_t)r << (16 * (kk & 3) + v * 3);
+                if (kk < 4) bits[0] |= word;
+                else bits[1] |= word;
             }
         }
     }
@@ -1085,70 +1113,153 @@ __global__ void __launch_bounds__(BS) k_ring(const double* __restrict__ ti, doub
                 if (tp[dk * sz + dj * sy + di] > 0) ring = 0.25;
     to[c0] = smax(t, ring);
 }
-// apply_blending then blending_ring (3-D) in one pass on 16 x 4 x 4 cell
-// tiles: the aggregate troubles of the tile and a two-cell halo are staged in
-// LDS, theta_tmp is formed on the tile and a one-cell halo (0 outside cells
-// 1..N-2, where apply_blending does not write it), then the ring. The
-// troubles are 0 or 1 and every theta_tmp is >= +0, so the maxima do not
-// depend on the visiting order; k_blend's order is kept anyway. theta_tmp is
-// not written.
+// apply_blending then blending_ring in one pass, active axes x, x-y or x-y-z.
+// The troubles are 0 or 1, so a row of cells is a bit mask and the blend of a
+// row is a few shifts and ORs of the masks around it: a cell's theta_tmp is 1,
+// 0.75, 0.5 or 0.375 for the nearest trouble within 0, 1, 2 or 3 axis steps of
+// its box, and the ring is 0.25 next to any of those. A workgroup covers rows
+// of 60 cells: each wave loads 64 cells of a row (the 60 and two on each side)
+// and its comparison with 1 is the row's mask; theta_tmp is formed as masks on
+// the tile and a one-cell halo (none outside cells 1..N-2, where
+// apply_blending does not write it; theta_tmp itself is not written). Staging
+// doubles and visiting 27 + 27 of them per cell took 1.08 ms at 96^3 p=3
+// against 0.2 ms for the bytes; 62 x 66 x 61: 0.31 -> 0.08 ms. Troubles that are neither 0 nor 1 (never
+// written by detect_troubles) take the formula cell by cell.
+template <int AY, int AZ>
 struct ThTile {
-    static constexpr int TX = 16, TY = 4, TZ = 4;
-    static constexpr int RX = TX + 4, RY = TY + 4, RZ = TZ + 4;  // troubles with the two-cell halo
-    static constexpr int PX = TX + 2, PY = TY + 2, PZ = TZ + 2;  // theta_tmp with the one-cell halo
-    static_assert(TX * TY * TZ == BS, "one cell per thread");
+    static constexpr int TX = 60, TY = AZ ? 8 : (AY ? 16 : 1), TZ = AZ ? 8 : 1;
+    static constexpr int RY = TY + 4 * AY, RZ = TZ + 4 * AZ;  // rows of troubles, two-row halo
+    static constexpr int PY = TY + 2 * AY, PZ = TZ + 2 * AZ;  // rows of theta_tmp, one-row halo
+    static_assert(PY * PZ <= BS && TY * TZ <= BS, "one row per thread");
 };
+// theta_tmp of cell (k, j, i) from the troubles tv (src/trouble_detection.cpp:191-210); 0 where it is not written
+template <int AY, int AZ>
+__device__ double theta_tmp_at(const double* tv, const FV& s, int k, int j, int i) {
+    if (i < 1 || i > s.Nx - 2 || (AY && (j < 1 || j > s.Ny - 2)) || (AZ && (k < 1 || k > s.Nz - 2))) return 0.0;
+    const double w[4] = {1.0, 0.75, 0.5, 0.375};
+    double t = 0;
+#pragma unroll 1
+    for (int dk = -AZ; dk <= AZ; dk++)
+#pragma unroll 1
+        for (int dj = -AY; dj <= AY; dj++)
+#pragma unroll 1
+            for (int di = -1; di <= 1; di++)
+                t = smax(t, w[(di != 0) + (dj != 0) + (dk != 0)] * tv[((size_t)(k + dk) * s.Ny + j + dj) * s.Nx + i + di]);
+    return t;
+}
+template <int AY, int AZ>
 __global__ void __launch_bounds__(BS) k_blend_ring_tile(const double* __restrict__ tr, double* __restrict__ th, FV s,
                                                         int bx, int by, int bz) {
-    using TT = ThTile;
-    constexpr int NR = TT::RX * TT::RY * TT::RZ, NP = TT::PX * TT::PY * TT::PZ;
-    __shared__ double st[NR];
-    __shared__ double sp[NP];
+    using TT = ThTile<AY, AZ>;
+    constexpr int TY = TT::TY, TZ = TT::TZ, RY = TT::RY, PY = TT::PY;
+    __shared__ uint64_t sM[RY * TT::RZ];      // troubles; bit b of a row: cell i0 - 2 + b
+    __shared__ uint64_t sP[PY * TT::PZ];      // theta_tmp > 0
+    __shared__ uint64_t sC[5][TY * TZ];       // theta_tmp = 1, >= 0.75, >= 0.5, >= 0.375; the ring
     const uint32_t b = xcd_block();
     if (b >= (uint32_t)bx * by * bz) return;  // padding blocks of the XCD grid (uniform per block)
     const int bi = (int)(b % bx), bj = (int)((b / bx) % by), bk = (int)(b / ((uint32_t)bx * by));
-    const int i0 = 1 + bi * TT::TX, j0 = 1 + bj * TT::TY, k0 = 1 + bk * TT::TZ;  // first output cell
-    const int tid = threadIdx.x;
+    const int i0 = 1 + bi * TT::TX, j0 = AY ? 1 + bj * TY : 0, k0 = AZ ? 1 + bk * TZ : 0;  // first output cell
+    const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
     const double* tv = tr + (size_t)(s.nv - 1) * s.plane();
-    for (int q = tid; q < NR; q += BS) {
-        const int gi = i0 - 2 + q % TT::RX, gj = j0 - 2 + (q / TT::RX) % TT::RY, gk = k0 - 2 + q / (TT::RX * TT::RY);
-        if (gi >= 0 && gi < s.Nx && gj >= 0 && gj < s.Ny && gk >= 0 && gk < s.Nz)
-            st[q] = tv[((size_t)gk * s.Ny + gj) * s.Nx + gi];
-    }
-    __syncthreads();
-    const double w[4] = {1.0, 0.75, 0.5, 0.375};
-    for (int q = tid; q < NP; q += BS) {
-        const int x = q % TT::PX, y = (q / TT::PX) % TT::PY, z = q / (TT::PX * TT::PY);
-        const int gi = i0 - 1 + x, gj = j0 - 1 + y, gk = k0 - 1 + z;
-        double t = 0;
-        if (gi >= 1 && gi <= s.Nx - 2 && gj >= 1 && gj <= s.Ny - 2 && gk >= 1 && gk <= s.Nz - 2) {
-            const double* c = st + ((z + 1) * TT::RY + (y + 1)) * TT::RX + (x + 1);
+    const int gi = i0 - 2 + lane;
+    int odd = 0;
+    constexpr int NR = RY * TT::RZ, W = BS / 64, UN = 4;  // rows, waves, loads in flight
+    for (int r0 = wave; r0 < NR; r0 += UN * W) {
+        double t[UN];
 #pragma unroll
-            for (int dk = -1; dk <= 1; dk++)
-#pragma unroll
-                for (int dj = -1; dj <= 1; dj++)
-#pragma unroll
-                    for (int di = -1; di <= 1; di++) {
-                        const int n0 = (di != 0) + (dj != 0) + (dk != 0);
-                        t = smax(t, w[n0] * c[(dk * TT::RY + dj) * TT::RX + di]);
-                    }
+        for (int u = 0; u < UN; u++) {
+            const int r = r0 + u * W, gj = j0 - 2 * AY + r % RY, gk = k0 - 2 * AZ + r / RY;
+            const bool in = r < NR && gi >= 0 && gi < s.Nx && gj >= 0 && gj < s.Ny && gk >= 0 && gk < s.Nz;
+            t[u] = in ? tv[((size_t)gk * s.Ny + gj) * s.Nx + gi] : 0.0;
         }
-        sp[q] = t;
+#pragma unroll
+        for (int u = 0; u < UN; u++) {
+            const uint64_t m = __ballot(t[u] == 1.0);
+            odd |= !(t[u] == 0.0 || t[u] == 1.0);
+            if (lane == 0 && r0 + u * W < NR) sM[r0 + u * W] = m;
+        }
+    }
+    if (__syncthreads_or(odd)) {
+#pragma unroll 1
+        for (int r = wave; r < TY * TZ; r += BS / 64) {
+            const int j = j0 + r % TY, k = k0 + r / TY;
+            if (lane < 2 || lane > 61 || gi > s.Nx - 2 || (AY && j > s.Ny - 2) || (AZ && k > s.Nz - 2)) continue;
+            double ring = 0;
+#pragma unroll 1
+            for (int dk = -AZ; dk <= AZ; dk++)
+#pragma unroll 1
+                for (int dj = -AY; dj <= AY; dj++)
+#pragma unroll 1
+                    for (int di = -1; di <= 1; di++)
+                        if (theta_tmp_at<AY, AZ>(tv, s, k + dk, j + dj, gi + di) > 0) ring = 0.25;
+            th[((size_t)k * s.Ny + j) * s.Nx + gi] = smax(theta_tmp_at<AY, AZ>(tv, s, k, j, gi), ring);
+        }
+        return;
+    }
+    if (tid < PY * TT::PZ) {
+        const int y = tid % PY, z = tid / PY;  // row of theta_tmp
+        const int gj = j0 - AY + y, gk = k0 - AZ + z;
+        uint64_t c0 = 0, c1 = 0, c2 = 0, c3 = 0;
+        if ((!AY || (gj >= 1 && gj <= s.Ny - 2)) && (!AZ || (gk >= 1 && gk <= s.Nz - 2))) {
+            const uint64_t* m = sM + (z + AZ) * RY + y + AY;
+            auto beside = [](uint64_t x) { return (x << 1) | (x >> 1); };
+            c0 = m[0];
+            c1 = beside(m[0]);
+            if (AY) {
+                const uint64_t n = m[-1] | m[1];
+                c1 |= n;
+                c2 |= beside(n);
+            }
+            if (AZ) {
+                const uint64_t n = m[-RY] | m[RY];
+                c1 |= n;
+                c2 |= beside(n);
+            }
+            if (AY && AZ) {
+                const uint64_t n = m[-RY - 1] | m[-RY + 1] | m[RY - 1] | m[RY + 1];
+                c2 |= n;
+                c3 |= beside(n);
+            }
+            c1 |= c0;
+            c2 |= c1;
+            c3 |= c2;
+            // cells 1..Nx-2 that have both neighbours in the row: bits lo..hi
+            const int lo = max(1, 3 - i0), hi = min(62, s.Nx - i0);
+            const uint64_t in = hi >= lo ? (~0ull >> (63 - (hi - lo))) << lo : 0;
+            c0 &= in;
+            c1 &= in;
+            c2 &= in;
+            c3 &= in;
+        }
+        sP[tid] = c3;
+        const int ty = y - AY, tz = z - AZ;
+        if (ty >= 0 && ty < TY && tz >= 0 && tz < TZ) {
+            const int o = tz * TY + ty;
+            sC[0][o] = c0;
+            sC[1][o] = c1;
+            sC[2][o] = c2;
+            sC[3][o] = c3;
+        }
     }
     __syncthreads();
-    const int tx = tid % TT::TX, ty = (tid / TT::TX) % TT::TY, tz = tid / (TT::TX * TT::TY);
-    const int i = i0 + tx, j = j0 + ty, k = k0 + tz;
-    if (i > s.Nx - 2 || j > s.Ny - 2 || k > s.Nz - 2) return;
-    const double* p = sp + ((tz + 1) * TT::PY + (ty + 1)) * TT::PX + (tx + 1);
-    double ring = 0;
+    if (tid < TY * TZ) {
+        const int y = tid % TY + AY, z = tid / TY + AZ;
+        uint64_t p = 0;
 #pragma unroll
-    for (int dk = -1; dk <= 1; dk++)
+        for (int dk = -AZ; dk <= AZ; dk++)
 #pragma unroll
-        for (int dj = -1; dj <= 1; dj++)
-#pragma unroll
-            for (int di = -1; di <= 1; di++)
-                if (p[(dk * TT::PY + dj) * TT::PX + di] > 0) ring = 0.25;
-    th[((size_t)k * s.Ny + j) * s.Nx + i] = smax(p[0], ring);
+            for (int dj = -AY; dj <= AY; dj++) p |= sP[(z + dk) * PY + y + dj];
+        sC[4][tid] = p | (p << 1) | (p >> 1);
+    }
+    __syncthreads();
+    if (lane < 2 || lane > 61 || gi > s.Nx - 2) return;
+    for (int r = wave; r < TY * TZ; r += BS / 64) {
+        const int j = j0 + r % TY, k = k0 + r / TY;
+        if ((AY && j > s.Ny - 2) || (AZ && k > s.Nz - 2)) continue;
+        auto bit = [&](int q) { return (sC[q][r] >> lane) & 1; };
+        th[((size_t)k * s.Ny + j) * s.Nx + gi] =
+            bit(0) ? 1.0 : (bit(1) ? 0.75 : (bit(2) ? 0.5 : (bit(3) ? 0.375 : (bit(4) ? 0.25 : 0.0))));
+    }
 }
 // theta_from_troubles (src/trouble_detection.cpp:213-221)
 __global__ void __launch_bounds__(BS) k_theta_raw(const double* __restrict__ tr, double* __restrict__ th, FV s, uint32_t total) {
@@ -1160,12 +1271,6 @@ __global__ void __launch_bounds__(BS) k_theta_raw(const double* __restrict__ tr,
 // ---------------------------------------------------------------------------
 // MUSCL-Hancock + HLLC fallback flux: src/muscl.hpp:2-13,
 // src/hydro.cpp:591-788
-__device__ __forceinline__ double minmod(double SL, double SR, double xL, double xR) {
-    double ratio = SR / SL;
-    ratio = smax(0.0, smin(ratio, 1.0));
-    double slope = ratio * SL;
-    return 0.5 * slope * (xR - xL);
-}
 // src/hydro.cpp:591-615
 __device__ __forceinline__ void corrector(const double* W, double* dWt, const double* dWx, const double* dWy,
                                           const double* dWz, double gm) {
@@ -1191,44 +1296,76 @@ __device__ __forceinline__ void corrector(const double* W, double* dWt, const do
 // (its primitive state, minmod slopes along the active axes and the Hancock
 // time derivative), which is the same for every face of the cell, and the
 // state at one of its faces along D. A cell's reconstruction is computed once
-// per thread and used for every face that needs it.
+// per thread and used for every face that needs it. The divisions by grid
+// widths (30 of a 3-D cell's slopes and 15 of its Hancock shifts) take three
+// instructions each; quotients that may be inexact are divided.
 struct Recon {
     double w[NVP], dw[3][NVP], dwt[NVP];
 };
-__device__ __forceinline__ void recon(const double* __restrict__ W, const FV& s, const Geo& g, int k, int j, int i,
-                                      int ay, int az, double gm, Recon& r) {
-    const double *xc = g.c[0], *xf = g.f[0], *yc = g.c[1], *yf = g.f[1], *zc = g.c[2], *zf = g.f[2];
+__device__ __forceinline__ double minmod(double SL, double SR, double df) {
+    double ratio = SR / SL;
+    ratio = smax(0.0, smin(ratio, 1.0));
+    double slope = ratio * SL;
+    return 0.5 * slope * df;
+}
+// W: the cell's first variable, variables pl apart, neighbours st[d] apart
+// along axis d; l: its FV cell index per axis.
+template <class P>
+__device__ __forceinline__ void recon(P W, size_t pl, const int (&st)[3], const Geo& g, const int (&l)[3], int ay, int az,
+                                      double gm, Recon& r) {
+    const int act[3] = {1, ay, az};
 #pragma unroll
-    for (int v = 0; v < NVP; v++) {
-        const double w = W[s.off(v, k, j, i)];
-        r.w[v] = w;
-        double wL = W[s.off(v, k, j, i - 1)], wR = W[s.off(v, k, j, i + 1)];
-        r.dw[0][v] = minmod((wR - w) / (xc[i + 1] - xc[i]), (w - wL) / (xc[i] - xc[i - 1]), xf[i], xf[i + 1]);
-        r.dw[1][v] = 0;
-        r.dw[2][v] = 0;
-        if (ay) {
-            wL = W[s.off(v, k, j - 1, i)];
-            wR = W[s.off(v, k, j + 1, i)];
-            r.dw[1][v] = minmod((wR - w) / (yc[j + 1] - yc[j]), (w - wL) / (yc[j] - yc[j - 1]), yf[j], yf[j + 1]);
+    for (int v = 0; v < NVP; v++) r.w[v] = W[v * pl];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        if (!act[d]) {
+#pragma unroll
+            for (int v = 0; v < NVP; v++) r.dw[d][v] = 0;
+            continue;
         }
-        if (az) {
-            wL = W[s.off(v, k - 1, j, i)];
-            wR = W[s.off(v, k + 1, j, i)];
-            r.dw[2][v] = minmod((wR - w) / (zc[k + 1] - zc[k]), (w - wL) / (zc[k] - zc[k - 1]), zf[k], zf[k + 1]);
+        const ConstDiv cd = g.dc1[d][l[d] - 1], cu = g.dc1[d][l[d]];
+        const double df = g.df[d][l[d]].h;
+        bool recheck = false;
+#pragma unroll
+        for (int v = 0; v < NVP; v++) {
+            const double SL = div_fast(W[v * pl + st[d]] - r.w[v], cu), SR = div_fast(r.w[v] - W[(long)(v * pl) - st[d]], cd);
+            recheck = recheck || div_recheck(SL) || div_recheck(SR);
+            r.dw[d][v] = minmod(SL, SR, df);
         }
+        if (recheck)
+#pragma unroll
+            for (int v = 0; v < NVP; v++)
+                r.dw[d][v] = minmod((W[v * pl + st[d]] - r.w[v]) / cu.h, (r.w[v] - W[(long)(v * pl) - st[d]]) / cd.h, df);
     }
     corrector(r.w, r.dwt, r.dw[0], r.dw[1], r.dw[2], gm);
 }
-// The reconstructed state at the cell's upper (WL of the reference) or lower
-// (WR) face along D.
+__device__ __forceinline__ void recon_at(const double* __restrict__ W, const FV& s, const Geo& g, int k, int j, int i,
+                                         int ay, int az, double gm, Recon& r) {
+    const int st[3] = {1, s.Nx, s.Nx * s.Ny}, l[3] = {i, j, k};
+    recon(W + s.off(0, k, j, i), s.plane(), st, g, l, ay, az, gm, r);
+}
+// Hancock shift of the cell's states at its faces along D: dwt dt / h.
 template <int D>
-__device__ __forceinline__ void face_state(const Recon& r, const Geo& g, int k, int j, int i, double dt, bool upper,
-                                           double* out) {
-    const double h = (D == 0 ? g.f[0][i + 1] - g.f[0][i] : (D == 1 ? g.f[1][j + 1] - g.f[1][j] : g.f[2][k + 1] - g.f[2][k]));
+__device__ __forceinline__ void hancock(const Recon& r, const Geo& g, int k, int j, int i, double dt, double* hs) {
+    const ConstDiv h = g.df[D][D == 0 ? i : (D == 1 ? j : k)];
+    bool recheck = false;
+#pragma unroll
+    for (int v = 0; v < NVP; v++) {
+        hs[v] = div_fast(r.dwt[v] * dt, h);
+        recheck = recheck || div_recheck(hs[v]);
+    }
+    if (recheck)
+#pragma unroll
+        for (int v = 0; v < NVP; v++) hs[v] = r.dwt[v] * dt / h.h;
+}
+// The reconstructed state at the cell's upper (WL of the reference) or lower
+// (WR) face along D, hs its Hancock shift.
+template <int D>
+__device__ __forceinline__ void face_state(const Recon& r, const double* hs, bool upper, double* out) {
 #pragma unroll
     for (int v = 0; v < NVP; v++) {
         const double dw = r.dw[D][v];
-        out[v] = upper ? r.w[v] + dw + r.dwt[v] * dt / h : r.w[v] - dw + r.dwt[v] * dt / h;
+        out[v] = upper ? r.w[v] + dw + hs[v] : r.w[v] - dw + hs[v];
     }
 }
 // compute_fluxes<D> (src/hydro.cpp:683-751) at the lower D face of cell
@@ -1242,8 +1379,10 @@ __device__ __forceinline__ void fb_face(const double* __restrict__ W, double* __
     double wL[NVP], uL[NVP], uR[NVP], fL[NVP];
     {
         Recon rn;
-        recon(W, s, g, kn, jn, in, ay, az, gm, rn);
-        face_state<D>(rn, g, kn, jn, in, dt, true, wL);
+        recon_at(W, s, g, kn, jn, in, ay, az, gm, rn);
+        double hs[NVP];
+        hancock<D>(rn, g, kn, jn, in, dt, hs);
+        face_state<D>(rn, hs, true, wL);
     }
     cons(wL, uL, gm);
     cons(wR, uR, gm);
@@ -1286,10 +1425,11 @@ __global__ void __launch_bounds__(BS) k_fallback(const double* __restrict__ W, c
     double wR[3][NVP];  // this cell's lower-face states
     {
         Recon rc;
-        recon(W, s, g, k, j, i, ay, az, gm, rc);
-        if (t0 != 0.0) face_state<0>(rc, g, k, j, i, dt, false, wR[0]);
-        if (t1 != 0.0) face_state<1>(rc, g, k, j, i, dt, false, wR[1]);
-        if (t2 != 0.0) face_state<2>(rc, g, k, j, i, dt, false, wR[2]);
+        recon_at(W, s, g, k, j, i, ay, az, gm, rc);
+        double hs[NVP];
+        if (t0 != 0.0) { hancock<0>(rc, g, k, j, i, dt, hs); face_state<0>(rc, hs, false, wR[0]); }
+        if (t1 != 0.0) { hancock<1>(rc, g, k, j, i, dt, hs); face_state<1>(rc, hs, false, wR[1]); }
+        if (t2 != 0.0) { hancock<2>(rc, g, k, j, i, dt, hs); face_state<2>(rc, hs, false, wR[2]); }
     }
     if (t0 != 0.0) fb_face<0>(W, Fx, sx, s, g, k, j, i, t0, wR[0], dt, ay, az, gm);
     if (t1 != 0.0) fb_face<1>(W, Fy, sy, s, g, k, j, i, t1, wR[1], dt, ay, az, gm);
@@ -1304,12 +1444,24 @@ __global__ void __launch_bounds__(BS) k_fallback(const double* __restrict__ W, c
 // face (the per-cell kernel above reconstructs a cell up to four times).
 // The arithmetic of each state and flux is the per-cell kernel's, so the
 // faces are the same bits. A tile with no nonzero theta in reach exits.
+// It is bound by latency (wave cycles 74% waiting), so the waits are few: the
+// tile's W with its halo (two cells below, one above) is staged in LDS in one
+// go (each value read once instead of once per stencil), the faces' old
+// fluxes are on the way while the upper states are exchanged, and the
+// exchange reuses the staged W's space, which keeps four workgroups per CU
+// (62 x 66 x 61 elements p=3: 1.60 -> 1.22 ms per call, 2-D 256^2 27 -> 22 us;
+// three-instruction divisions alone, with W from memory, cost 1.78 ms: their
+// rechecks kept the loads of one axis behind the slopes of the other).
 template <int AY, int AZ>
 struct FbTile {
     static constexpr int TX = AZ ? SPDK_FB_TX : (AY ? 16 : 256), TY = AZ ? BS / (SPDK_FB_TX * SPDK_FB_TZ) : (AY ? 16 : 1),
                          TZ = AZ ? SPDK_FB_TZ : 1;
     static constexpr int NC = TX * TY * TZ;          // = BS
     static constexpr int HX = TY * TZ, HY = AY ? TX * TZ : 0, HZ = AZ ? TX * TY : 0;  // halo cells per layer
+    static constexpr int DIM = 1 + AY + AZ;
+    static constexpr int RX = TX + 3, RY = AY ? TY + 3 : 1, RZ = AZ ? TZ + 3 : 1, NR = RX * RY * RZ;  // staged W
+    static constexpr int UP = DIM * NVP * NC, UPH = NVP * (HX + HY + HZ);  // upper-face states: tile, halo
+    static constexpr int LDS = NVP * NR > UP + UPH ? NVP * NR : UP + UPH;
     static_assert(NC == BS, "one cell per thread");
     static_assert(HX + HY + HZ <= BS, "one halo cell per thread");
 };
@@ -1319,9 +1471,10 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(SPDK_FB
                                                       double* __restrict__ Fz, FV s, FV fx, FV fy, FV fz, Geo g,
                                                       double dt, double gm, int bx, int by, int bz) {
     using TL = FbTile<AY, AZ>;
-    constexpr int TX = TL::TX, TY = TL::TY, TZ = TL::TZ;
-    __shared__ double up[3][NVP][TL::NC];                    // upper-face states of the tile cells, per axis
-    __shared__ double uph[NVP][TL::HX + TL::HY + TL::HZ];    // upper-face state of each halo cell (its one axis)
+    constexpr int TX = TL::TX, TY = TL::TY, TZ = TL::TZ, DIM = TL::DIM;
+    __shared__ double lds[TL::LDS];  // staged W [variable][z][y][x], then the upper-face states
+    double* const up = lds;              // [axis][variable][tile cell]
+    double* const uph = lds + TL::UP;    // [variable][halo cell], each at its one axis
     const int tid = threadIdx.x;
     const uint32_t b = xcd_block();
     if (b >= (uint32_t)bx * by * bz) return;  // padding blocks of the XCD grid (uniform per block)
@@ -1353,6 +1506,15 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(SPDK_FB
         if (AZ && tz + 1 < TZ && k + 1 <= s.Nz - 2) { thi[2] = th[c0 + sz]; upper = upper || smax(thi[2], tc) != 0.0; }
     }
     if (!__syncthreads_or(lower)) return;  // no blended face in the tile
+    const size_t pl = s.plane();
+    for (int q = tid; q < TL::NR; q += BS) {
+        const int gi = i0 - 2 + q % TL::RX, gj = AY ? j0 - 2 + (q / TL::RX) % TL::RY : 0;
+        const int gk = AZ ? k0 - 2 + q / (TL::RX * TL::RY) : 0;
+        if (gi >= s.Nx || gj >= s.Ny || gk >= s.Nz) continue;
+        const double* w = W + ((size_t)gk * s.Ny + gj) * s.Nx + gi;
+#pragma unroll
+        for (int v = 0; v < NVP; v++) lds[v * TL::NR + q] = w[v * pl];
+    }
     // halo cell of this thread: layer x (i0-1, j0+.., k0+..), then y, then z
     int hd = -1, hi = 0, hj = 0, hk = 0, hslot = tid;
     if (tid < TL::HX) {
@@ -1373,70 +1535,85 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(SPDK_FB
             hneed = smax(th[cu], th[ch]) != 0.0;
         }
     }
-    double wR[3][NVP];  // this cell's lower-face states
-    if (valid && (lower || upper)) {
-        Recon rc;
-        recon(W, s, g, k, j, i, AY, AZ, gm, rc);
-        if (tf[0] != 0.0) face_state<0>(rc, g, k, j, i, dt, false, wR[0]);
-        if (AY && tf[1] != 0.0) face_state<1>(rc, g, k, j, i, dt, false, wR[1]);
-        if (AZ && tf[2] != 0.0) face_state<2>(rc, g, k, j, i, dt, false, wR[2]);
-        if (upper) {
-            double wu[NVP];
-            face_state<0>(rc, g, k, j, i, dt, true, wu);
-#pragma unroll
-            for (int v = 0; v < NVP; v++) up[0][v][tid] = wu[v];
-            if (AY) {
-                face_state<1>(rc, g, k, j, i, dt, true, wu);
-#pragma unroll
-                for (int v = 0; v < NVP; v++) up[1][v][tid] = wu[v];
-            }
-            if (AZ) {
-                face_state<2>(rc, g, k, j, i, dt, true, wu);
-#pragma unroll
-                for (int v = 0; v < NVP; v++) up[2][v][tid] = wu[v];
-            }
-        }
-    }
+    __syncthreads();
+    constexpr int st[3] = {1, TL::RX, TL::RX * TL::RY};
+    auto staged = [&](int kk, int jj, int ii) -> const double* {
+        return lds + ((AZ ? kk - k0 + 2 : 0) * TL::RY + (AY ? jj - j0 + 2 : 0)) * TL::RX + ii - i0 + 2;
+    };
+    double wh[NVP];  // the halo cell's upper-face state
     if (hneed) {
         Recon rh;
-        recon(W, s, g, hk, hj, hi, AY, AZ, gm, rh);
-        double wu[NVP];
-        if (hd == 0) face_state<0>(rh, g, hk, hj, hi, dt, true, wu);
-        else if (hd == 1) face_state<1>(rh, g, hk, hj, hi, dt, true, wu);
-        else face_state<2>(rh, g, hk, hj, hi, dt, true, wu);
-#pragma unroll
-        for (int v = 0; v < NVP; v++) uph[v][hslot] = wu[v];
+        const int l[3] = {hi, hj, hk};
+        recon(staged(hk, hj, hi), TL::NR, st, g, l, AY, AZ, gm, rh);
+        double hs[NVP];
+        if (hd == 0) { hancock<0>(rh, g, hk, hj, hi, dt, hs); face_state<0>(rh, hs, true, wh); }
+        else if (AY && hd == 1) { hancock<1>(rh, g, hk, hj, hi, dt, hs); face_state<1>(rh, hs, true, wh); }
+        else if (AZ) { hancock<2>(rh, g, hk, hj, hi, dt, hs); face_state<2>(rh, hs, true, wh); }
     }
+    double wR[DIM][NVP], wU[DIM][NVP];  // this cell's lower- and upper-face states
+    const bool need = valid && (lower || upper);
+    if (need) {
+        Recon rc;
+        const int l[3] = {i, j, k};
+        recon(staged(k, j, i), TL::NR, st, g, l, AY, AZ, gm, rc);
+        double hs[NVP];
+        hancock<0>(rc, g, k, j, i, dt, hs);
+        face_state<0>(rc, hs, false, wR[0]);
+        face_state<0>(rc, hs, true, wU[0]);
+        if (AY) {
+            hancock<1>(rc, g, k, j, i, dt, hs);
+            face_state<1>(rc, hs, false, wR[DIM > 1 ? 1 : 0]);
+            face_state<1>(rc, hs, true, wU[DIM > 1 ? 1 : 0]);
+        }
+        if (AZ) {
+            hancock<2>(rc, g, k, j, i, dt, hs);
+            face_state<2>(rc, hs, false, wR[DIM > 2 ? 2 : 0]);
+            face_state<2>(rc, hs, true, wU[DIM > 2 ? 2 : 0]);
+        }
+    }
+    __syncthreads();  // the staged W has been read
+    if (need)
+#pragma unroll
+        for (int d = 0; d < DIM; d++)
+#pragma unroll
+            for (int v = 0; v < NVP; v++) up[(d * NVP + v) * TL::NC + tid] = wU[d][v];
+    if (hneed)
+#pragma unroll
+        for (int v = 0; v < NVP; v++) uph[v * (TL::HX + TL::HY + TL::HZ) + hslot] = wh[v];
+    double* const F[3] = {Fx, Fy, Fz};
+    const FV* const sF[3] = {&fx, &fy, &fz};
+    double fo[DIM][NVP];
+#pragma unroll
+    for (int d = 0; d < DIM; d++)
+#pragma unroll
+        for (int v = 0; v < NVP; v++) fo[d][v] = tf[d] != 0.0 ? F[d][sF[d]->off(v, k, j, i)] : 0.0;
     __syncthreads();
     if (!valid) return;
 #pragma unroll
-    for (int d = 0; d < 3; d++) {
-        if ((d == 1 && !AY) || (d == 2 && !AZ) || tf[d] == 0.0) continue;
+    for (int d = 0; d < DIM; d++) {
+        if (tf[d] == 0.0) continue;
         const int td = d == 0 ? tx : (d == 1 ? ty : tz);
         const int stride = d == 0 ? 1 : (d == 1 ? TX : TX * TY);
         const int hs = d == 0 ? ty + TY * tz : (d == 1 ? TL::HX + tx + TX * tz : TL::HX + TL::HY + tx + TX * ty);
         double wL[NVP], uL[NVP], uR[NVP], fL[NVP];
 #pragma unroll
-        for (int v = 0; v < NVP; v++) wL[v] = td > 0 ? up[d][v][tid - stride] : uph[v][hs];
+        for (int v = 0; v < NVP; v++)
+            wL[v] = td > 0 ? up[(d * NVP + v) * TL::NC + tid - stride] : uph[v * (TL::HX + TL::HY + TL::HZ) + hs];
         cons(wL, uL, gm);
         cons(wR[d], uR, gm);
         if (d == 0) riemann_hllc<0>(uL, uR, fL, gm);
         else if (d == 1) riemann_hllc<1>(uL, uR, fL, gm);
         else riemann_hllc<2>(uL, uR, fL, gm);
-        double* F = d == 0 ? Fx : (d == 1 ? Fy : Fz);
-        const FV& sF = d == 0 ? fx : (d == 1 ? fy : fz);
 #pragma unroll
         for (int v = 0; v < NVP; v++) {
-            size_t o = sF.off(v, k, j, i);
-            double f = F[o];
-            f = f + tf[d] * (fL[v] - f);
-            F[o] = f;
+            const double f = fo[d][v];
+            F[d][sF[d]->off(v, k, j, i)] = f + tf[d] * (fL[v] - f);
         }
-        for (int v = NVP; v < sF.nv; v++) {  // slot: HLLC slot taken as zero
-            size_t o = sF.off(v, k, j, i);
-            double f = F[o];
+        for (int v = NVP; v < sF[d]->nv; v++) {  // slot: HLLC slot taken as zero
+            const size_t o = sF[d]->off(v, k, j, i);
+            double f = F[d][o];
             f = f + tf[d] * (0.0 - f);
-            F[o] = f;
+            F[d][o] = f;
         }
     }
 }
@@ -1447,6 +1624,9 @@ static Geo geo_of(spdk_ctx* c) {
     for (int d = 0; d < 3; d++) {
         g.f[d] = c->fvf[d] ? c->fvf[d] : c->fvf[0];
         g.c[d] = c->fvc[d] ? c->fvc[d] : c->fvc[0];
+        g.dc1[d] = c->fvdc1[d];
+        g.dc2[d] = c->fvdc2[d];
+        g.df[d] = c->fvdf[d];
     }
     return g;
 }
@@ -1887,14 +2067,21 @@ int spdk_detect_troubles_bits(spdk_ctx* c, const double* Wn, const double* Wo, d
 
 int spdk_blend_theta(spdk_ctx* c, const double* tr, double* th_tmp, double* th, spdk_fv_shape s) {
     int ax = c->prm.active[0], ay = c->prm.active[1], az = c->prm.active[2];
-    if (c->prm.blending && ax && ay && az) {  // 3-D: both passes on cell tiles, theta_tmp not written
-        const int bx = (s.Nx - 2 + ThTile::TX - 1) / ThTile::TX, by = (s.Ny - 2 + ThTile::TY - 1) / ThTile::TY;
-        const int bz = (s.Nz - 2 + ThTile::TZ - 1) / ThTile::TZ;
-        const size_t nb = (size_t)bx * by * bz;
-        hipLaunchKernelGGL(k_blend_ring_tile, dim3((unsigned)((nb + kXcd - 1) / kXcd * kXcd)), dim3(BS), 0, c->stream,
-                           tr, th, FV(s), bx, by, bz);
+    if (c->prm.blending && ax && (ay || !az)) {  // both passes on bit-mask tiles, theta_tmp not written
+#define SPDK_THT(AY_, AZ_)                                                                                      \
+    do {                                                                                                        \
+        using TT = ThTile<AY_, AZ_>;                                                                            \
+        const int bx = (s.Nx - 2 + TT::TX - 1) / TT::TX, by = AY_ ? (s.Ny - 2 + TT::TY - 1) / TT::TY : 1;         \
+        const int bz = AZ_ ? (s.Nz - 2 + TT::TZ - 1) / TT::TZ : 1;                                               \
+        const size_t nb = (size_t)bx * by * bz;                                                                 \
+        hipLaunchKernelGGL((k_blend_ring_tile<AY_, AZ_>), dim3((unsigned)((nb + kXcd - 1) / kXcd * kXcd)), dim3(BS), 0, \
+                           c->stream, tr, th, FV(s), bx, by, bz);                                               \
+    } while (0)
+        if (az) SPDK_THT(1, 1);
+        else if (ay) SPDK_THT(1, 0);
+        else SPDK_THT(0, 0);
+#undef SPDK_THT
         SPDK_LAUNCH_CHECK("blend_ring");
-        (void)th_tmp;
     } else if (c->prm.blending) {
         uint32_t t2 = (uint32_t)((size_t)(s.Nz - 2 * az) * (s.Ny - 2 * ay) * (s.Nx - 2 * ax));
         const int a3[3] = {ax, ay, az};

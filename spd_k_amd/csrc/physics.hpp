@@ -131,14 +131,14 @@ __device__ __forceinline__ void riemann_hllc(const double* UL, const double* UR,
     double rcR = WR[0] * (sR - vR);
     double vs = (rcR * vR + rcL * vL + (WL[4] - WR[4])) / (rcR + rcL);
     double ps = (rcR * WL[4] + rcL * WR[4] + rcL * rcR * (vL - vR)) / (rcR + rcL);
-    double rsL = WL[0] * (sL - vL) / (sL - vs);
-    double esL = ((sL - vL) * UL[4] - WL[4] * vL + ps * vs) / (sL - vs);
-    double rsR = WR[0] * (sR - vR) / (sR - vs);
-    double esR = ((sR - vR) * UR[4] - WR[4] * vR + ps * vs) / (sR - vs);
+    // the star state of the side the face lies in (the other one is not used)
+    const bool left = vs > 0;
+    const double sK = left ? sL : sR, vK = left ? vL : vR, pK = left ? WL[4] : WR[4];
+    double rs = (left ? WL[0] : WR[0]) * (sK - vK) / (sK - vs);
+    double es = ((sK - vK) * (left ? UL[4] : UR[4]) - pK * vK + ps * vs) / (sK - vs);
     double rg, vg, pg, eg;
     if (sL > 0) { rg = WL[0]; vg = WL[V1]; pg = WL[4]; eg = UL[4]; }
-    else if (vs > 0) { rg = rsL; vg = vs; pg = ps; eg = esL; }
-    else if (sR > 0) { rg = rsR; vg = vs; pg = ps; eg = esR; }
+    else if (left || sR > 0) { rg = rs; vg = vs; pg = ps; eg = es; }
     else { rg = WR[0]; vg = WR[V1]; pg = WR[4]; eg = UR[4]; }
     F[0] = rg * vg;
     F[V1] = rg * vg * vg + pg;

@@ -586,6 +586,26 @@ int spdk_ctx_create(const spdk_params* prm, const spdk_operators* ops, void* str
             SPDK_CHECK(hipMemcpy(c->fvc[d], ops->fv_centers[d], sizeof(double) * c->fvn[d], hipMemcpyHostToDevice));
         }
     }
+    for (int d = 0; d < 3; d++) {
+        auto widths = [&](int n, auto width, ConstDiv** out) -> int {
+            if (n < 1) return SPDK_OK;
+            std::vector<ConstDiv> h(n);
+            for (int l = 0; l < n; l++) h[l] = const_div(width(l));
+            void* p = nullptr;
+            SPDK_CHECK(hipMalloc(&p, sizeof(ConstDiv) * n));
+            c->owned.push_back(p);
+            *out = (ConstDiv*)p;
+            SPDK_CHECK(hipMemcpy(p, h.data(), sizeof(ConstDiv) * n, hipMemcpyHostToDevice));
+            return SPDK_OK;
+        };
+        const double *x = ops->fv_centers[d], *f = ops->fv_faces[d];
+        int rc = SPDK_OK;
+        if (x) rc = widths(c->fvn[d] - 1, [&](int l) { return x[l + 1] - x[l]; }, &c->fvdc1[d]);
+        if (x && !rc)
+            rc = widths(c->fvn[d] - 1, [&](int l) { return l ? x[l + 1] - x[l - 1] : 0.0; }, &c->fvdc2[d]);
+        if (f && !rc) rc = widths(c->fvnf[d] - 1, [&](int l) { return f[l + 1] - f[l]; }, &c->fvdf[d]);
+        if (rc) return rc;
+    }
     SPDK_CHECK(hipMalloc(&c->red, sizeof(double) * (c->red_blocks + 8)));
     SPDK_CHECK(hipHostMalloc(&c->red_host, sizeof(double) * 8, hipHostMallocDefault));
     SPDK_CHECK(hipEventCreate(&c->ev0));
