@@ -76,12 +76,6 @@ constexpr int kGExtra = 6;       // extra features per element
 constexpr float kAmin = 1e-6f;   // floor of the element amplitude
 constexpr float kAgate = 1e-5f;  // amplitude at or below which the guess is the zero-order one
 
-// Minimum waves per SIMD the sweep kernel is compiled for (bounds its VGPRs);
-// the 3-D p=3 predictor is held at 3 (168 VGPRs), where it fits without spills.
-#ifndef SPDK_MSWEEP_WAVES
-#define SPDK_MSWEEP_WAVES 1
-#endif
-
 template <int N, int DIM>
 struct MT {
     static constexpr int T = N;  // ADER time nodes
@@ -98,12 +92,24 @@ struct MT {
     // + 32 bytes: the element areas of a block start 8 banks apart, so reads
     // that cross elements at one in-element offset do not share a bank
     static constexpr int ELEM_BYTES = ((LDS_X * 8 + (LDS_D + LDS_F) * 4) + 15) / 16 * 16 + 32;
-    static constexpr int EPB0 = TPE >= 256 ? 1 : 256 / TPE;
-    static constexpr int EPB_LDS = 61440 / ELEM_BYTES;
-    static constexpr int EPB = EPB0 < EPB_LDS ? EPB0 : EPB_LDS;
-    static constexpr int BLOCK = ((EPB * TPE + 63) / 64) * 64;
+    // Whole elements per wave (at most a quarter of the lanes idles): the
+    // phases of an element then need no block barrier (elem_sync).
+    static constexpr int EPW = 64 / TPE;
+    static constexpr int EPB_LDS = 61440 / ELEM_BYTES / EPW * EPW;
+    static constexpr int EPB = 4 * EPW < EPB_LDS ? 4 * EPW : EPB_LDS;
+    static constexpr int BLOCK = EPB / EPW * 64;
+    // element of the block (EPB: an idle lane) and solution point of a thread
+    static __device__ __forceinline__ int el_of(int tid) {
+        if (TPE == 64) return __builtin_amdgcn_readfirstlane(tid / 64);  // wave-uniform: scalar element addresses
+        const int j = (tid % 64) / TPE;
+        return j < EPW ? tid / 64 * EPW + j : EPB;
+    }
+    static __device__ __forceinline__ int pt_of(int tid) { return (tid % 64) % TPE; }
     static constexpr int LDS_BYTES = EPB * ELEM_BYTES > BLOCK * 8 ? EPB * ELEM_BYTES : BLOCK * 8;
-    static_assert(EPB >= 1 && BLOCK <= 256, "tile does not fit a workgroup");
+    // waves per SIMD the sweeps are compiled for: as many as the blocks' LDS lets in, at most 3 (168 VGPRs)
+    static constexpr int WAVES = 163840 / LDS_BYTES * BLOCK / 256 < 3 ? 163840 / LDS_BYTES * BLOCK / 256 : 3;
+    static_assert(TPE <= 64 && EPB >= 1 && BLOCK <= 256, "tile does not fit a workgroup");
+    static_assert(T * NT == TPE, "one pencil per thread and axis");
     static_assert((LDS_D + LDS_F) * 4 >= 2 * NVP * TPE * 8, "cv ping-pong needs two FP64 state planes");
     static constexpr int XRES = 4 * NVP;      // X slot: element residual
     static constexpr int XACT = 4 * NVP + 1;  // X slot: element active this sweep
@@ -118,7 +124,7 @@ struct MArgs {
     const double* mu;       // (5,E) element means of U_sp
     const float* d_old;     // (5,E,TPE) U_sp - mu
     float* D;               // (T,5,E,TPE) predictor state, read and rewritten in place
-    float* trb[2][3];       // two trace buffers per axis, (T,5,E,2,NT) (slice 0 only for the zero-order guess)
+    float* trb[2][3];       // two trace buffers per axis, (5,2,E,slices,NT) (see trace_at)
     int* ver;               // (2,E): sweep number of each element's last write to each buffer
     int cur;                // this sweep's number
     const unsigned char* big_in;  // per element: r_e >= tol in the previous sweep (null: every element active)
@@ -146,7 +152,7 @@ struct MArgs {
     int sweep;
     double g[3];    // constant gravity (hydro/g1..g3)
     int grav;       // any component nonzero
-    int path;       // 0: every slice is d_old (zero-order guess); 1: slices from D
+    int path;       // predictor: 0: every slice is d_old (zero-order guess); 1: slices from D
     int tin_slices; // slices present in the readable trace buffers (1 or T)
     int out_pred;   // predictor (else corrector)
     // FV face-flux sweep: sub-cell face fluxes of slice t along axis d (FV
@@ -158,6 +164,16 @@ struct MArgs {
     const float* SS;
     int fv_valu;
 };
+
+// p[i] of an array that the kernel's own writes cannot change: through the
+// constant address space, so that wave-uniform elements come by scalar loads
+// and the others may be loaded ahead of fences and stores. (a.ver is written
+// by the sweep, but the value that replaces an entry, the current sweep's
+// number, leads every reader to the same buffer as the entry it replaces.)
+template <typename V>
+__device__ __forceinline__ V cload(const V* p, size_t i) {
+    return ((const __attribute__((address_space(4))) V*)p)[i];
+}
 
 // ---- FP64 physics in the frame of the face normal: slot 1 is the normal
 // momentum, slots 2 and 3 the transverse ones (cyclic, as V1, V2, V3 of
@@ -297,10 +313,22 @@ __device__ __forceinline__ Geo geo(int d, int q) {
     return g;
 }
 
+// Offset of the trace of variable v, side sd, element e, slice t, line q in an
+// axis' buffer of ns slices (1: the zero-order guess). The slices of a face are
+// together, then the elements along x: one wave's access is T * NT contiguous
+// floats, and the 128-byte lines that a block reads of its y and z neighbours
+// hold nothing but the side it reads. With the two sides of an element side
+// by side (64 bytes each at 3-D p=3) every sweep fetched both: at 98^3
+// elements, p=3, a predictor sweep 19.5 GB against 13.6 GB.
+template <int NT>
+__device__ __forceinline__ size_t trace_at(size_t E, int ns, int v, int sd, size_t e, int t, int q) {
+    return (((size_t)(v * 2 + sd) * E + e) * ns + t) * NT + q;
+}
+
 // Trace buffer of axis d holding element el's newest traces written before
 // this sweep.
 __device__ __forceinline__ const float* read_buffer(const MArgs& a, int d, size_t el) {
-    const int v0 = a.ver[el], v1 = a.ver[(size_t)a.E + el];
+    const int v0 = cload(a.ver, el), v1 = cload(a.ver, (size_t)a.E + el);
     const int b = (v1 < a.cur && (v1 > v0 || v0 >= a.cur)) ? 1 : 0;
     const float* t0 = d == 0 ? a.trb[0][0] : (d == 1 ? a.trb[0][1] : a.trb[0][2]);
     const float* t1 = d == 0 ? a.trb[1][0] : (d == 1 ? a.trb[1][1] : a.trb[1][2]);
@@ -321,50 +349,71 @@ __device__ __forceinline__ void face_sources(const MArgs& a, int d, int ei, int 
     el1 = ebase + (size_t)(ed >= Nd - 2 ? (per ? 1 : Nd - 2) : ed + 1) * stride;
 }
 
+// Traces a pencil reads across its two faces: v0 is the value left of face 0
+// (or the ghost fill that replaces the own value at face M-1 of the left
+// ghost), v1 the value right of face M-1 (or the ghost fill at face 0 of the
+// right ghost), normal frame, without the neighbours' means.
+struct Nbr { float v0[NVP], v1[NVP]; };
+
+// Loads the traces pencil (d, slice ts of ns, q) of element e reads. Ghost fills: periodic
+// copies the opposite interior element, gradfree / reflective the adjacent one
+// (src/boundary.cpp:48-113). lower_face_only: v1 only where the lower face
+// takes it (the right ghost).
+template <int N, int DIM>
+__device__ __forceinline__ Nbr load_traces(const MArgs& a, int d, int ns, int ts, int q, int ei, int ej, int ek,
+                                           size_t e, bool lower_face_only = false) {
+    constexpr int NT = MT<N, DIM>::NT;
+    const int ed = d == 0 ? ei : (d == 1 ? ej : ek);
+    const int Nd = d == 0 ? a.Ne[0] : (d == 1 ? a.Ne[1] : a.Ne[2]);
+    const bool per = (d == 0 ? a.bc[0] : (d == 1 ? a.bc[1] : a.bc[2])) == SPDK_BC_PERIODIC;
+    size_t el0, el1;
+    face_sources(a, d, ei, ej, ek, e, el0, el1);
+    const int sid0 = ed <= 1 ? (per ? 1 : 0) : 1;
+    const int sid1 = ed >= Nd - 2 ? (per ? 0 : 1) : 0;
+    const float* t0 = read_buffer(a, d, el0);
+    const float* t1 = read_buffer(a, d, el1);
+    Nbr n;
+#pragma unroll
+    for (int v = 0; v < NVP; v++) {
+        n.v0[v] = t0[trace_at<NT>(a.E, ns, vperm(v, d), sid0, el0, ts, q)];
+        n.v1[v] = 0.f;
+    }
+    if (!lower_face_only || ed == Nd - 1)
+#pragma unroll
+        for (int v = 0; v < NVP; v++) n.v1[v] = t1[trace_at<NT>(a.E, ns, vperm(v, d), sid1, el1, ts, q)];
+    return n;
+}
+
 // One pencil task: slice Dsl of the LDS state (floats [v][PSZ]) along axis
-// d, pencil q. Writes F - F(mu) at the M flux points into the flux slot
-// (floats [v][FSZ]) and, when asked, adds bw * (F(1) - F(0)) of the
+// d, pencil q, neighbour traces nb. Writes F - F(mu) at the M flux points into
+// the flux slot (floats [v][FSZ]) and, when asked, adds bw * (F(1) - F(0)) of the
 // pencil to the face balance (want_bal). Face values follow src/boundary.cpp:48-113
 // (ghost traces) and src/hydro.cpp:368-418 (LLF at element faces).
 template <int N, int DIM>
-__device__ __forceinline__ void pencil(const MArgs& a, const float* Dsl, float* Fslot, const double* X, int d, int q,
-                                       int ts, int ei, int ej, int ek, size_t e, bool want_bal, double (&bal)[NVP],
-                                       double bw, bool lower_face_only = false) {
+__device__ __forceinline__ void pencil(const MArgs& a, const Nbr& nb, const float* Dsl, float* Fslot, const double* X,
+                                       int d, int q, int ei, int ej, int ek, size_t e, bool want_bal,
+                                       double (&bal)[NVP], double bw, bool lower_face_only = false) {
     using G = MT<N, DIM>;
-    constexpr int M = G::M, NT = G::NT;
+    constexpr int M = G::M;
     const size_t E = (size_t)a.E;
     const double gm1 = a.gm - 1.0;
     const Geo g = geo<N, DIM>(d, q);
     int pv[NVP];
 #pragma unroll
     for (int v = 0; v < NVP; v++) pv[v] = vperm(v, d);
-    // neighbour operands: n0 is the value left of face 0 (or the ghost fill
-    // that replaces the own value at face M-1 of the left ghost), n1 the value
-    // right of face M-1 (or the ghost fill at face 0 of the right ghost).
-    // Ghost fills: periodic copies the opposite interior element, gradfree /
-    // reflective the adjacent one (normal momentum negated). Issued first so
-    // the loads overlap the interpolation and the interior fluxes.
     const int ed = d == 0 ? ei : (d == 1 ? ej : ek);
     const int Nd = d == 0 ? a.Ne[0] : (d == 1 ? a.Ne[1] : a.Ne[2]);
     const int type = d == 0 ? a.bc[0] : (d == 1 ? a.bc[1] : a.bc[2]);
-    const size_t stride = d == 0 ? 1 : (d == 1 ? (size_t)a.Ne[0] : (size_t)a.Ne[0] * a.Ne[1]);
-    const size_t ebase = e - (size_t)ed * stride;
-    const bool per = type == SPDK_BC_PERIODIC;
-    const size_t el0 = ebase + (size_t)(ed <= 1 ? (per ? Nd - 2 : 1) : ed - 1) * stride;
-    const int sid0 = ed <= 1 ? (per ? 1 : 0) : 1;
-    const size_t el1 = ebase + (size_t)(ed >= Nd - 2 ? (per ? 1 : Nd - 2) : ed + 1) * stride;
-    const int sid1 = ed >= Nd - 2 ? (per ? 0 : 1) : 0;
+    // ghost fills of a reflective axis: normal momentum negated
     const bool flip0 = ed <= 1 && type == SPDK_BC_REFLECTIVE;
     const bool flip1 = ed >= Nd - 2 && type == SPDK_BC_REFLECTIVE;
-    const float* tr0 = read_buffer(a, d, el0);
-    const float* tr1 = read_buffer(a, d, el1);
+    size_t el0, el1;
+    face_sources(a, d, ei, ej, ek, e, el0, el1);
     double n0[NVP], n1[NVP];
 #pragma unroll
     for (int v = 0; v < NVP; v++) {
-        const size_t pvE = (size_t)pv[v] * E;
-        const size_t tb = ((size_t)ts * NVP + pv[v]) * E;
-        n0[v] = a.mu[pvE + el0] + (double)tr0[((tb + el0) * 2 + sid0) * NT + q];
-        n1[v] = a.mu[pvE + el1] + (double)tr1[((tb + el1) * 2 + sid1) * NT + q];
+        n0[v] = cload(a.mu, (size_t)pv[v] * E + el0) + (double)nb.v0[v];
+        n1[v] = cload(a.mu, (size_t)pv[v] * E + el1) + (double)nb.v1[v];
     }
     if (flip0) n0[1] = -n0[1];
     if (flip1) n1[1] = -n1[1];
@@ -384,7 +433,7 @@ __device__ __forceinline__ void pencil(const MArgs& a, const float* Dsl, float* 
         for (int f = 0; f < M; f++) {
             float x = 0.f;
 #pragma unroll
-            for (int l = 0; l < N; l++) x += p[l] * a.S2F[f * N + l];
+            for (int l = 0; l < N; l++) x += p[l] * cload(a.S2F, f * N + l);
             uf[f][v] = x;
         }
     }
@@ -453,6 +502,18 @@ __device__ __forceinline__ double pencil_weight(const MArgs& a, int q) {
     return pick(a.wq, q / N) * pick(a.wq, q % N);
 }
 
+// Barrier between phases that touch only the element's own LDS area. An
+// element lies in one wave, so the wave's own order is enough: a wave's LDS
+// operations execute in order, and the wavefront-scope fences keep the
+// compiler from moving its LDS accesses across the point. The waves of a
+// block then run their phases independently (a block barrier makes each wait
+// for the slowest).
+__device__ __forceinline__ void elem_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // New state at the control volumes and the element's dt candidate (FP64):
 // compute_primitives, sp->cv sweeps x, y, z (src/transforms.cpp:99-117) and
 // src/hydro.cpp:226-256. `area` is the element's LDS (>= 2 planes of FP64).
@@ -471,7 +532,7 @@ __device__ __forceinline__ double cv_and_dt(const double* un, double* area, bool
 #pragma unroll
         for (int v = 0; v < NVP; v++) wa[v * TPE + s] = wv[v];
     }
-    __syncthreads();
+    elem_sync();
     double* src = wa;
     double* dst = wb;
 #pragma unroll
@@ -484,12 +545,12 @@ __device__ __forceinline__ double cv_and_dt(const double* un, double* area, bool
 #pragma unroll
                 for (int l = 0; l < N; l++) {
                     int sl = d == 0 ? s - ii + l : (d == 1 ? s + (l - jj) * N : s + (l - kk) * N * N);
-                    x += src[v * TPE + sl] * S2C[id * N + l];
+                    x += src[v * TPE + sl] * cload(S2C, id * N + l);
                 }
                 dst[v * TPE + s] = x;
             }
         }
-        __syncthreads();
+        elem_sync();
         double* tmp = src;
         src = dst;
         dst = tmp;
@@ -518,44 +579,54 @@ __device__ __forceinline__ double cv_and_dt(const double* un, double* area, bool
     return r;
 }
 
-// Block minimum of r into part[blockIdx.x]; `red` holds BLOCK doubles.
+// Block minimum of r into part[blockIdx.x]: each wave's over its lanes, the
+// waves' through LDS (red, one double per wave, any area of the block).
 template <int BLOCK>
 __device__ __forceinline__ void block_min(double r, double* red, double* part) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) r = nan_min(r, __shfl_xor(r, off, 64));
     __syncthreads();
-    red[threadIdx.x] = r;
+    if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = r;
     __syncthreads();
-    for (int w = BLOCK / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] = nan_min(red[threadIdx.x], red[threadIdx.x + w]);
-        __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int w = 1; w < BLOCK / 64; w++) r = nan_min(r, red[w]);
+        part[blockIdx.x] = r;
     }
-    if (threadIdx.x == 0) part[blockIdx.x] = red[0];
 }
 
-// Conservative shift of the point updates du (see the header): red holds
-// 2 * NVP * TPE doubles of the element's LDS, X_shift NVP doubles.
+// Conservative shift of the point updates du (see the header): I - J is the
+// sum over the element's points of bal - wsp du. One element per wave: over
+// the lanes; otherwise through red (NVP * TPE doubles of the element's LDS)
+// and X_shift (NVP doubles), four partial sums per variable.
 template <int N, int DIM>
 __device__ __forceinline__ void cons_shift(double* du, const double* bal, double wsp, double wtot, double* red,
                                            double* X_shift, bool live, int s) {
     constexpr int TPE = MT<N, DIM>::TPE;
-    if (live)
+    if constexpr (TPE == 64) {
 #pragma unroll
         for (int v = 0; v < NVP; v++) {
-            red[v * TPE + s] = bal[v];
-            red[(NVP + v) * TPE + s] = wsp * du[v];
-        }
-    __syncthreads();
-    if (live)
-        for (int v = s; v < NVP; v += TPE) {  // an element may have fewer points than variables
-            double I = 0.0, J = 0.0;
-            for (int j = 0; j < TPE; j++) {
-                I += red[v * TPE + j];
-                J += red[(NVP + v) * TPE + j];
-            }
-            X_shift[v] = (I - J) / wtot;
-        }
-    __syncthreads();
+            double x = bal[v] - wsp * du[v];
 #pragma unroll
-    for (int v = 0; v < NVP; v++) du[v] += X_shift[v];
+            for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+            du[v] += x / wtot;
+        }
+    } else {
+        if (live)
+#pragma unroll
+            for (int v = 0; v < NVP; v++) red[v * TPE + s] = bal[v] - wsp * du[v];
+        elem_sync();
+        if (live)
+            for (int v = s; v < NVP; v += TPE) {  // an element may have fewer points than variables
+                double x[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                for (int j = 0; j < TPE; j++) x[j % 4] += red[v * TPE + j];
+                X_shift[v] = ((x[0] + x[1]) + (x[2] + x[3])) / wtot;
+            }
+        elem_sync();
+#pragma unroll
+        for (int v = 0; v < NVP; v++) du[v] += live ? X_shift[v] : 0.0;
+    }
 }
 
 // face_integral (src/transforms.cpp:378-481) of the round's axis d for every
@@ -614,7 +685,7 @@ __device__ __forceinline__ void mfv_faces(const MArgs& a, const float* Fs, const
         const int li = lane & 15, lk = lane >> 4;
         float av[4];
 #pragma unroll
-        for (int ks = 0; ks < 4; ks++) av[ks] = a.SS[li * 16 + 4 * ks + lk];  // A[row li][k = 4 ks + lk]
+        for (int ks = 0; ks < 4; ks++) av[ks] = cload(a.SS, li * 16 + 4 * ks + lk);  // A[row li][k = 4 ks + lk]
         double* base[T];
 #pragma unroll
         for (int t = 0; t < T; t++) base[t] = d == 0 ? a.Ffv[t][0] : (d == 1 ? a.Ffv[t][1] : a.Ffv[t][2]);
@@ -723,7 +794,7 @@ __device__ __forceinline__ void mfv_faces_staged(const MArgs& a, unsigned char* 
         const int lane = s, li = lane & 15, lk = lane >> 4;
         float av[4];
 #pragma unroll
-        for (int ks = 0; ks < 4; ks++) av[ks] = a.SS[li * 16 + 4 * ks + lk];
+        for (int ks = 0; ks < 4; ks++) av[ks] = cload(a.SS, li * 16 + 4 * ks + lk);
 #pragma unroll
         for (int ct = 0; ct < NCOL / 16; ct++) {
             const int col = ct * 16 + li;
@@ -796,45 +867,72 @@ __device__ __forceinline__ void mfv_faces_staged(const MArgs& a, unsigned char* 
     }
 }
 
-// Barrier between sweep phases that touch only the element's own LDS area.
-// With one element per wave (TPE = 64) the wave's own order is enough: a
-// wave's LDS operations execute in order, and the wavefront-scope fences keep
-// the compiler from moving its LDS accesses across the point. The waves of a
-// block then run their phases independently (a block barrier makes each wait
-// for the slowest). Otherwise, and in the face sweep (MODE 2, whose staged
-// writes cross elements), the block barrier.
-template <int TPE, int MODE>
-__device__ __forceinline__ void elem_sync() {
-    if constexpr (TPE == 64 && MODE != 2) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    } else {
-        __syncthreads();
+// Kinds of sweep, compiled apart.
+enum {
+    M_START = 0,  // the first predictor sweep from the zero-order guess (one slice, all axes in one round)
+    M_PRED = 1,   // a predictor sweep from the state in D
+    M_CORR = 2,   // the corrector: face balance, conservative update, cv state and dt
+    M_FACES = 3,  // flux evaluation of the predictor's slices with their face integrals written for the FV update
+    M_STAGED = 4  // the same with the writes staged through LDS (mfv_faces_staged; 3-D p=3)
+};
+
+// Flux divergence along axis d at point (ii, jj, kk), added to dudt, from the
+// flux slots: slot t holds slice t, or (ALL_AXES, one slice) slot d axis d.
+template <int N, int DIM, int TS, bool ALL_AXES>
+__device__ __forceinline__ void divergence(const MArgs& a, const float* Fs, int d, int ii, int jj, int kk,
+                                           float (&dudt)[N][NVP]) {
+    constexpr int M = N + 1, FSZ = MT<N, DIM>::FSZ;
+    // pencil through this point and the point's position along it
+    const int q = d == 0 ? (DIM == 3 ? kk * N + jj : jj) : (d == 1 ? (DIM == 3 ? kk * N + ii : ii) : jj * N + ii);
+    const int id = d == 0 ? ii : (d == 1 ? jj : kk);
+    const Geo g = geo<N, DIM>(d, q);
+    float Dr[M];
+#pragma unroll
+    for (int l = 0; l < M; l++) Dr[l] = cload(a.Dh, (d * N + id) * M + l);
+#pragma unroll
+    for (int t = 0; t < TS; t++) {
+        const float* Ft = Fs + (ALL_AXES ? d : t) * NVP * FSZ;
+#pragma unroll
+        for (int v = 0; v < NVP; v++) {
+            float acc = 0.f;
+#pragma unroll
+            for (int l = 0; l < M; l++) acc += Ft[v * FSZ + g.fb + l * g.fs] * Dr[l];
+            dudt[t][v] += acc;
+        }
     }
 }
 
-// MODE 0: a predictor sweep (out_pred set); MODE 1: the corrector (face
-// balance, conservative update, cv state and dt); MODE 2: the flux
-// evaluation of the predictor's slices with their face integrals written
-// for the FV update (mfv_faces), nothing else. Compiled apart, the predictor
-// needs fewer VGPRs (3 waves per SIMD at 3-D p=3 instead of 2).
+// One sweep. At 98^3 elements, p=3, M_PRED moves 25.4 GB (state and traces read
+// and written, d_old read) in 6.6 ms, 3.8 TB/s where a copy reaches 4.4; M_START
+// 15.7 GB in 4.4 ms; M_CORR 20 GB in 6.5 ms, 62% of it issuing FP64 and FP32
+// vector instructions; M_STAGED 40 GB, of them 32 written, in 12.0 ms (7.5, 7.5,
+// 10.6 and 14.7 ms before the following, same values):
+//   - the matrices, means and versions come through the constant address
+//     space (cload): the compiler cannot show that the kernel's stores leave
+//     them alone, and otherwise loads them per lane again after each fence
+//     (a third of the time of M_PRED);
+//   - the element index is wave-uniform at 64 points per element, so its
+//     neighbours' addresses are scalar;
+//   - the axes are unrolled, apart from the first sweep's single round;
+//   - no block barrier between the phases of an element, in M_CORR too: the
+//     conservative shift and the dt minimum go across the wave's lanes.
 template <int N, int DIM, int MODE>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE == 0 && N == 4 && DIM == 3 ? 3 : SPDK_MSWEEP_WAVES))) k_msweep(MArgs a) {
-    constexpr bool CONS = MODE == 1;
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE >= M_FACES ? 1 : MT<N, DIM>::WAVES))) k_msweep(MArgs a) {
+    constexpr bool CONS = MODE == M_CORR, PRED = MODE == M_START || MODE == M_PRED;
     using G = MT<N, DIM>;
     constexpr int M = G::M, NT = G::NT, TPE = G::TPE, EPB = G::EPB, T = G::T, FSZ = G::FSZ;
+    constexpr int TS = MODE == M_START ? 1 : T;  // distinct slices of the input state
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const int tid = threadIdx.x;
-    const int el = tid / TPE, s = tid % TPE;
-    // MODE 2: workgroups go to the 8 XCDs in turn; XCD x takes the x-th
+    const int el = G::el_of(tid), s = G::pt_of(tid);
+    // Face integrals: workgroups go to the 8 XCDs in turn; XCD x takes the x-th
     // contiguous eighth of the element blocks, so the face rows that
     // neighbouring blocks share (rows are not line-aligned) are written
     // through one L2. The grid is a multiple of 8; blocks past the end exit.
     int blk;
     if (a.blist) {
         blk = a.blist[blockIdx.x];
-    } else if (MODE == 2) {
+    } else if (MODE == M_FACES || MODE == M_STAGED) {
         blk = (int)((blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8);
         if (blk * EPB >= a.E) return;  // uniform per block
     } else {
@@ -859,43 +957,60 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE =
         ek = e / (a.Ne[0] * a.Ne[1]);
     }
     const int ii = s % N, jj = DIM >= 2 ? (s / N) % N : 0, kk = DIM == 3 ? s / (N * N) : 0;
-    // pencil through this point and the point's position along it, per axis
-    const int qx = DIM == 3 ? kk * N + jj : jj, qy = DIM == 3 ? kk * N + ii : ii, qz = jj * N + ii;
-    const double wsp = pick(a.wq, ii) * (DIM >= 2 ? pick(a.wq, jj) : 1.0) * (DIM == 3 ? pick(a.wq, kk) : 1.0);
-
-    if (live)
-        for (int v = s; v < NVP; v += TPE) X[v] = a.mu[(size_t)v * E + e];
-    if (live && s == 0) {  // active: own residual or a trace source's was >= tol last sweep
-        bool act = true;
-        if (a.big_in) {
-            act = a.big_in[e] != 0;
+    // active: own residual or a trace source's was >= tol last sweep
+    bool act_e = live;
+    if (PRED && a.big_in) {
+        if (live) {
+            act_e = a.big_in[e] != 0;
 #pragma unroll
             for (int d = 0; d < DIM; d++) {
                 size_t el0, el1;
                 face_sources(a, d, ei, ej, ek, (size_t)e, el0, el1);
-                act = act || a.big_in[el0] || a.big_in[el1];
+                act_e = act_e || a.big_in[el0] || a.big_in[el1];
             }
         }
-        X[G::XACT] = act ? 1.0 : 0.0;
-    }
-    elem_sync<TPE, MODE>();
-    const bool act_e = live && X[G::XACT] != 0.0;
-    if (!__syncthreads_or(act_e)) {  // nothing to do in this block
-        if (live && s == 0 && a.big_out) a.big_out[e] = 0;
-        if (tid == 0) {
-            if (a.res_part) a.res_part[blockIdx.x] = 0.0;
-            if (a.cnt_part) a.cnt_part[blockIdx.x] = 0.0;
+        if (!__syncthreads_or(act_e)) {  // nothing to do in this block
+            if (live && s == 0 && a.big_out) a.big_out[e] = 0;
+            if (tid == 0) {
+                if (a.res_part) a.res_part[blockIdx.x] = 0.0;
+                if (a.cnt_part) a.cnt_part[blockIdx.x] = 0.0;
+            }
+            return;
         }
-        return;
     }
-    if (act_e && s < DIM) {  // F(mu) along axis s
-        double um[NVP], fb[NVP];
+
+    // The loads of the element's state and of the first axis' traces go out
+    // together; the mean state is prepared while they are in flight.
+    float dold[NVP], din[TS][NVP];
 #pragma unroll
-        for (int v = 0; v < NVP; v++) um[v] = X[vperm(v, s)];
-        mflux(um, fb, a.gm - 1.0);
+    for (int v = 0; v < NVP; v++) dold[v] = act_e && PRED ? a.d_old[(size_t)v * slabE + eo] : 0.f;
+    if (MODE != M_START && act_e)
 #pragma unroll
-        for (int v = 0; v < NVP; v++) X[NVP + s * NVP + vperm(v, s)] = fb[v];
-    }
+        for (int t = 0; t < TS; t++)
+#pragma unroll
+            for (int v = 0; v < NVP; v++) din[t][v] = a.D[((size_t)t * NVP + v) * slabE + eo];
+    // this thread's pencil of every round (M_START: task s = d * NT + q instead)
+    const int tq = s / NT, q = s % NT;
+    const int ts = a.tin_slices > 1 ? tq : 0;
+    // the face integrals read faces 0..M-2 only, unless the x flux points are written as well
+    const bool lower = MODE == M_STAGED || (MODE == M_FACES && !a.F_x);
+    Nbr nb;
+    if (MODE != M_START && act_e) nb = load_traces<N, DIM>(a, 0, a.tin_slices, ts, q, ei, ej, ek, (size_t)e, lower);
+    if (MODE == M_START && act_e && s < DIM * NT) nb = load_traces<N, DIM>(a, s / NT, 1, 0, q, ei, ej, ek, (size_t)e);
+
+    if (live)
+        for (int v = s; v < NVP; v += TPE) X[v] = cload(a.mu, (size_t)v * E + e);
+    if (live && s == 0) X[G::XACT] = act_e ? 1.0 : 0.0;
+    elem_sync();
+    if (act_e)
+        for (int d = s; d < DIM; d += TPE) {  // F(mu) along axis d
+            double um[NVP], fb[NVP];
+#pragma unroll
+            for (int v = 0; v < NVP; v++) um[v] = X[vperm(v, d)];
+            mflux(um, fb, a.gm - 1.0);
+#pragma unroll
+            for (int v = 0; v < NVP; v++) X[NVP + d * NVP + vperm(v, d)] = fb[v];
+        }
     if (act_e && s == 0) {  // the mean state in FP32 for the difference-form fluxes
         float* XF = (float*)(X + G::XMF);
         const double ri = 1.0 / X[0];
@@ -910,106 +1025,78 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE =
         XF[6] = (float)X[3];
         XF[7] = (float)(X[4] + pm);
     }
-    float dold[NVP];
-#pragma unroll
-    for (int v = 0; v < NVP; v++) dold[v] = act_e && MODE != 2 ? a.d_old[(size_t)v * slabE + eo] : 0.f;
     if (act_e) {
-        if (a.path) {
 #pragma unroll
-            for (int t = 0; t < T; t++)
+        for (int t = 0; t < TS; t++)
 #pragma unroll
-                for (int v = 0; v < NVP; v++) Ds[(t * NVP + v) * PSZ + so] = a.D[((size_t)t * NVP + v) * slabE + eo];
-        } else {
-#pragma unroll
-            for (int v = 0; v < NVP; v++) Ds[v * PSZ + so] = dold[v];
-        }
+            for (int v = 0; v < NVP; v++) Ds[(t * NVP + v) * PSZ + so] = MODE == M_START ? dold[v] : din[t][v];
     }
-    elem_sync<TPE, MODE>();
+    elem_sync();
 
     float dudt[T][NVP];
 #pragma unroll
     for (int t = 0; t < T; t++)
 #pragma unroll
         for (int v = 0; v < NVP; v++) dudt[t][v] = 0.f;
-    // the corrector conserves: accumulate the face balance
-    const bool cons = CONS;
-    double bal[NVP] = {0.0, 0.0, 0.0, 0.0, 0.0};
-
-    // Rounds of pencil tasks, then the flux divergence of the round's fluxes.
-    // Zero-order guess (path 0): one round, one slice, task s = d * NT + q in
-    // flux slot d. Otherwise DIM rounds, round d: task s = t * NT + q in flux
-    // slot t. The round loop is not unrolled: one copy of its code.
-    const int nrounds = a.path ? DIM : 1;
-    double wsum = 0.0;
-#pragma unroll
-    for (int t = 0; t < T; t++) wsum += a.wdt[t];
+    double bal[NVP] = {0.0, 0.0, 0.0, 0.0, 0.0};  // the corrector's face balance
+    if constexpr (MODE == M_START) {
+        // one round, one slice: task s = d * NT + q in flux slot d
+        if (act_e)
+            for (int task = s; task < DIM * NT; task += TPE) {  // more than TPE only for p = 1 in 3-D
+                const int d = task / NT, qq = task % NT;
+                if (task != s) nb = load_traces<N, DIM>(a, d, 1, 0, qq, ei, ej, ek, (size_t)e);
+                pencil<N, DIM>(a, nb, Ds, Fs + d * NVP * FSZ, X, d, qq, ei, ej, ek, (size_t)e, false, bal, 0.0);
+            }
+        elem_sync();
+        if (act_e)
 #pragma unroll 1
-    for (int r = 0; r < nrounds; r++) {
-        // tasks of the round: TPE (= T * NT) or DIM * NT (more than TPE only for p = 1 in 3-D)
-        const int ntask = a.path ? TPE : DIM * NT;
-        for (int task = s; act_e && task < ntask; task += TPE) {
-            const int d = a.path ? r : task / NT, t = a.path ? task / NT : 0, q = task % NT;
-            const int slot = a.path ? t : d;
-            const int ts = a.tin_slices > 1 ? t : 0;
-            const double bw = (a.path ? pick(a.wdt, t) : wsum) * pencil_weight<N, DIM>(a, q) * pick(a.ih, d);
-            // the face integrals (MODE 2) read faces 0..M-2 only, unless the
-            // x flux points are written as well
-            pencil<N, DIM>(a, Ds + t * NVP * PSZ, Fs + slot * NVP * FSZ, X, d, q, ts, ei, ej, ek, (size_t)e, cons,
-                           bal, bw, MODE == 2 && !a.F_x);
-        }
-        elem_sync<TPE, MODE>();
-        if (MODE == 2) {
-            if constexpr (N == 4 && DIM == 3) {
-                if (!a.F_x && !a.fv_valu) mfv_faces_staged<N, DIM>(a, lds_raw, blk, r, s, el, act_e);
-                else mfv_faces<N, DIM>(a, Fs, X, r, s, act_e, ei, ej, ek);
+            for (int d = 0; d < DIM; d++) divergence<N, DIM, TS, MODE == M_START>(a, Fs, d, ii, jj, kk, dudt);
+        elem_sync();
+#pragma unroll
+        for (int t = 1; t < T; t++)  // the zero-order guess has identical slices
+#pragma unroll
+            for (int v = 0; v < NVP; v++) dudt[t][v] = dudt[0][v];
+    } else {
+        // Round d: the pencil (slice tq, line q) of axis d into flux slot tq,
+        // then the divergence along d. The next axis' traces are loaded
+        // during the divergence. Unrolled (but for the unstaged 3-D face
+        // integrals, whose code is long): the axis' variable order, strides and
+        // addresses are then constants of the code.
+        constexpr int UN = MODE == M_FACES && DIM == 3 ? 1 : DIM;
+        const double bt = CONS ? pick(a.wdt, tq) * pencil_weight<N, DIM>(a, q) : 0.0;
+#pragma unroll UN
+        for (int d = 0; d < DIM; d++) {
+            if (act_e) {
+                pencil<N, DIM>(a, nb, Ds + tq * NVP * PSZ, Fs + tq * NVP * FSZ, X, d, q, ei, ej, ek, (size_t)e, CONS,
+                               bal, CONS ? bt * a.ih[d] : 0.0, lower);
+                if (d + 1 < DIM) nb = load_traces<N, DIM>(a, d + 1, a.tin_slices, ts, q, ei, ej, ek, (size_t)e, lower);
+            }
+            elem_sync();
+            if constexpr (MODE == M_STAGED) {
+                mfv_faces_staged<N, DIM>(a, lds_raw, blk, d, s, el, act_e);
+                __syncthreads();  // read the block's other elements
+                continue;
+            } else if constexpr (MODE == M_FACES) {
+                mfv_faces<N, DIM>(a, Fs, X, d, s, act_e, ei, ej, ek);
             } else {
-                mfv_faces<N, DIM>(a, Fs, X, r, s, act_e, ei, ej, ek);
+                if (act_e) divergence<N, DIM, TS, MODE == M_START>(a, Fs, d, ii, jj, kk, dudt);
             }
-        }
-        if (act_e) {
-            const int d0 = a.path ? r : 0, d1 = MODE == 2 ? d0 : (a.path ? r + 1 : DIM);
-#pragma unroll 1
-            for (int d = d0; d < d1; d++) {
-                const int qdd = d == 0 ? qx : (d == 1 ? qy : qz), idd = d == 0 ? ii : (d == 1 ? jj : kk);
-                const Geo gd = geo<N, DIM>(d, qdd);
-                float Dr[M];
-#pragma unroll
-                for (int l = 0; l < M; l++) Dr[l] = a.Dh[(d * N + idd) * M + l];
-#pragma unroll
-                for (int t = 0; t < T; t++) {
-                    if (!a.path && t > 0) break;
-                    const float* Ft = Fs + (a.path ? t : d) * NVP * FSZ;
-#pragma unroll
-                    for (int v = 0; v < NVP; v++) {
-                        const float* F = Ft + v * FSZ;
-                        float acc = 0.f;
-#pragma unroll
-                        for (int l = 0; l < M; l++) acc += F[gd.fb + l * gd.fs] * Dr[l];
-                        dudt[t][v] += acc;
-                    }
-                }
-            }
-            if (a.F_x && (a.path ? r == 0 : true)) {  // x fluxes at the flux points (outputs)
+            if ((CONS || MODE == M_FACES) && a.F_x && act_e && d == 0) {  // x fluxes at the flux points (outputs)
                 for (int idx = s; idx < FSZ; idx += TPE)
                     for (int t = 0; t < T; t++) {
                         size_t o = (((size_t)t * NV) * E + e) * FSZ + idx;
-                        const float* Ft = Fs + (a.path ? t : 0) * NVP * FSZ;  // path 0: slot 0 is x
+                        const float* Ft = Fs + t * NVP * FSZ;
 #pragma unroll
                         for (int v = 0; v < NVP; v++) a.F_x[o + (size_t)v * E * FSZ] = X[NVP + v] + (double)Ft[v * FSZ + idx];
                         a.F_x[o + (size_t)NVP * E * FSZ] = 0.0;
                     }
             }
+            elem_sync();
         }
-        elem_sync<TPE, MODE>();
     }
-    if (MODE == 2) return;
-    if (!a.path)  // the zero-order guess has identical slices
-#pragma unroll
-        for (int t = 1; t < T; t++)
-#pragma unroll
-            for (int v = 0; v < NVP; v++) dudt[t][v] = dudt[0][v];
+    if constexpr (!PRED && !CONS) return;
 
-    if (!CONS && a.grav && act_e) {
+    if (PRED && a.grav && act_e) {
         // update_prediction's gravity source (src/transforms.cpp:17-27,
         // :309-313), dudt -= S, in the reference's in-place order: the
         // momenta's source takes the density just written, the energy's the
@@ -1042,7 +1129,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE =
 #pragma unroll
         for (int t = 0; t < T; t++) dudt[t][4] -= smu4 + (mn[t][0] * g0 + mn[t][1] * g1 + mn[t][2] * g2);
     }
-    if (!CONS) {
+    if constexpr (PRED) {
         // ---- predictor: d_new(t) = d_old - sum_l cdt(t,l) dudt(l); residual vs the input state
         float res = 0.f;
         if (act_e) {
@@ -1054,36 +1141,34 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE =
 #pragma unroll
                     for (int l = 0; l < T; l++) acc += a.cdt[t * kMaxTm + l] * dudt[l][v];
                     float dn = dold[v] - acc;
-                    // input state at this point: its own LDS slot (path 1) or d_old
-                    float din = a.path ? Ds[(t * NVP + v) * PSZ + so] : dold[v];
-                    const float df = fabsf(dn - din);
+                    // input state at this point: its own LDS slot, or d_old
+                    float di = MODE == M_START ? dold[v] : Ds[(t * NVP + v) * PSZ + so];
+                    const float df = fabsf(dn - di);
                     if (!(df <= res)) res = (df == df) ? df : __builtin_inff();  // a NaN never passes
                     a.D[((size_t)t * NVP + v) * slabE + eo] = dn;
                     Ds[(t * NVP + v) * PSZ + so] = dn;
                 }
         }
-        elem_sync<TPE, MODE>();
-        // traces of the new state into this element's older buffer: task =
-        // (d, t, q), q fastest: at 3-D p=3 each 64-lane pass is one axis
-        const int wb = act_e ? (a.ver[(size_t)a.E + e] < a.ver[e] ? 1 : 0) : 0;
+        elem_sync();
+        // traces of the new state into this element's older buffer, one
+        // pencil (slice tq, line q) per thread and axis
+        const int wb = act_e ? (cload(a.ver, E + e) < cload(a.ver, (size_t)e) ? 1 : 0) : 0;
         if (act_e) {
-            for (int task = s; task < T * DIM * NT; task += TPE) {
-                const int d = task / (T * NT), t = (task / NT) % T, q = task % NT;
+#pragma unroll
+            for (int d = 0; d < DIM; d++) {
                 const Geo gt = geo<N, DIM>(d, q);
+                float* to = wb ? a.trb[1][d] : a.trb[0][d];
 #pragma unroll
                 for (int v = 0; v < NVP; v++) {
                     float x0 = 0.f, x1 = 0.f;
 #pragma unroll
                     for (int l = 0; l < N; l++) {
-                        float p = Ds[(t * NVP + v) * PSZ + gt.sb + l * gt.ss];
-                        x0 += p * a.S2F[l];
-                        x1 += p * a.S2F[(M - 1) * N + l];
+                        float p = Ds[(tq * NVP + v) * PSZ + gt.sb + l * gt.ss];
+                        x0 += p * cload(a.S2F, l);
+                        x1 += p * cload(a.S2F, (M - 1) * N + l);
                     }
-                    float* tb = wb ? (d == 0 ? a.trb[1][0] : (d == 1 ? a.trb[1][1] : a.trb[1][2]))
-                                   : (d == 0 ? a.trb[0][0] : (d == 1 ? a.trb[0][1] : a.trb[0][2]));
-                    float* to = tb + ((((size_t)t * NVP + v) * E + e) * 2) * NT + q;
-                    to[0] = x0;
-                    to[NT] = x1;
+                    to[trace_at<NT>(E, T, v, 0, e, tq, q)] = x0;
+                    to[trace_at<NT>(E, T, v, 1, e, tq, q)] = x1;
                 }
             }
         }
@@ -1094,10 +1179,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE =
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) re = nan_maxf(re, __shfl_xor(re, off, 64));
         } else {
-            __syncthreads();
             if (act_e) Fs[s] = res;
-            __syncthreads();
+            elem_sync();
             if (act_e && s == 0)
+#pragma unroll
                 for (int j = 0; j < TPE; j++) re = nan_maxf(re, Fs[j]);
         }
         if (act_e && s == 0) {
@@ -1136,42 +1221,47 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE =
     }
 
     // ---- corrector (src/transforms.cpp:354-372), FP64 accumulation, conservative shift
-    double un[NVP], du[NVP];
+    if constexpr (CONS) {
+        const double wsp = pick(a.wq, ii) * (DIM >= 2 ? pick(a.wq, jj) : 1.0) * (DIM == 3 ? pick(a.wq, kk) : 1.0);
+        double un[NVP], du[NVP];
 #pragma unroll
-    for (int v = 0; v < NVP; v++) {
-        du[v] = 0.0;
+        for (int v = 0; v < NVP; v++) un[v] = act_e ? a.U_sp[(size_t)v * slabE + eo] : 1.0;
 #pragma unroll
-        for (int t = 0; t < T; t++) du[v] += a.wdt[t] * (double)dudt[t][v];
-    }
-    // update_solution's gravity source (src/transforms.cpp:364-367) from the
-    // final predictor slices, in FP64: sum_t w_t dt S_t, added after the
-    // conservative shift (which balances the fluxes only)
-    double sg[NVP] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    if (a.grav && act_e) {
+        for (int v = 0; v < NVP; v++) {
+            du[v] = 0.0;
 #pragma unroll
-        for (int t = 0; t < T; t++) {
-            const float* Dt = Ds + (a.path ? t : 0) * NVP * PSZ + so;  // path 0: one slice, d_old
-            const double rho = X[0] + (double)Dt[0];
-            const double m1 = X[1] + (double)Dt[PSZ], m2 = X[2] + (double)Dt[2 * PSZ], m3 = X[3] + (double)Dt[3 * PSZ];
-            sg[1] += a.wdt[t] * (rho * a.g[0]);
-            sg[2] += a.wdt[t] * (rho * a.g[1]);
-            sg[3] += a.wdt[t] * (rho * a.g[2]);
-            sg[4] += a.wdt[t] * (m1 * a.g[0] + m2 * a.g[1] + m3 * a.g[2]);
+            for (int t = 0; t < T; t++) du[v] += a.wdt[t] * (double)dudt[t][v];
         }
+        // update_solution's gravity source (src/transforms.cpp:364-367) from the
+        // final predictor slices, in FP64: sum_t w_t dt S_t, added after the
+        // conservative shift (which balances the fluxes only)
+        double sg[NVP] = {0.0, 0.0, 0.0, 0.0, 0.0};
+        if (a.grav && act_e) {
+#pragma unroll
+            for (int t = 0; t < T; t++) {
+                const float* Dt = Ds + t * NVP * PSZ + so;
+                const double rho = X[0] + (double)Dt[0];
+                const double m1 = X[1] + (double)Dt[PSZ], m2 = X[2] + (double)Dt[2 * PSZ], m3 = X[3] + (double)Dt[3 * PSZ];
+                sg[1] += a.wdt[t] * (rho * a.g[0]);
+                sg[2] += a.wdt[t] * (rho * a.g[1]);
+                sg[3] += a.wdt[t] * (rho * a.g[2]);
+                sg[4] += a.wdt[t] * (m1 * a.g[0] + m2 * a.g[1] + m3 * a.g[2]);
+            }
+            elem_sync();
+        }
+        cons_shift<N, DIM>(du, bal, wsp, a.wtot, (double*)Ds, X + G::XSHIFT, act_e, s);
+#pragma unroll
+        for (int v = 1; v < NVP; v++) du[v] -= sg[v];
+#pragma unroll
+        for (int v = 0; v < NVP; v++) un[v] = act_e ? un[v] - du[v] : 1.0;
+        if (act_e)
+#pragma unroll
+            for (int v = 0; v < NVP; v++) a.U_new[(size_t)v * slabE + eo] = un[v];
+        elem_sync();
+        double r = cv_and_dt<N, DIM>(un, (double*)Ds, act_e, s, ii, jj, kk, ei, ej, ek, (size_t)e, a.W_cv, slabE, a.S2C,
+                                     a.Ne, a.act, a.h, a.gm, a.cfl);
+        block_min<G::BLOCK>(r, (double*)lds_raw, a.part);
     }
-    __syncthreads();
-    cons_shift<N, DIM>(du, bal, wsp, a.wtot, (double*)Ds, X + G::XSHIFT, act_e, s);
-#pragma unroll
-    for (int v = 1; v < NVP; v++) du[v] -= sg[v];
-#pragma unroll
-    for (int v = 0; v < NVP; v++) un[v] = act_e ? a.U_sp[(size_t)v * slabE + eo] - du[v] : 1.0;
-    if (act_e)
-#pragma unroll
-        for (int v = 0; v < NVP; v++) a.U_new[(size_t)v * slabE + eo] = un[v];
-    __syncthreads();
-    double r = cv_and_dt<N, DIM>(un, (double*)Ds, act_e, s, ii, jj, kk, ei, ej, ek, (size_t)e, a.W_cv, slabE, a.S2C,
-                                 a.Ne, a.act, a.h, a.gm, a.cfl);
-    block_min<G::BLOCK>(r, (double*)lds_raw, a.part);
 }
 
 // Step start: element means, deviations and their face traces (one slice);
@@ -1184,7 +1274,7 @@ __global__ void __launch_bounds__(256) k_mstart(const double* __restrict__ U_sp,
     using G = MT<N, DIM>;
     constexpr int M = G::M, NT = G::NT, TPE = G::TPE, EPB = G::EPB;
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    const int tid = threadIdx.x, el = tid / TPE, s = tid % TPE;
+    const int tid = threadIdx.x, el = G::el_of(tid), s = G::pt_of(tid);
     const int e = blockIdx.x * EPB + el;
     const bool live = el < EPB && e < Eint;
     unsigned char* base = lds_raw + (size_t)(el < EPB ? el : 0) * G::ELEM_BYTES;
@@ -1235,9 +1325,8 @@ __global__ void __launch_bounds__(256) k_mstart(const double* __restrict__ U_sp,
                 x0 += p * S2F[l];
                 x1 += p * S2F[(M - 1) * N + l];
             }
-            float* to = trd + (((size_t)v * E + e) * 2) * NT + q;
-            to[0] = x0;
-            to[NT] = x1;
+            trd[trace_at<NT>(E, 1, v, 0, e, 0, q)] = x0;
+            trd[trace_at<NT>(E, 1, v, 1, e, 0, q)] = x1;
         }
     }
 }
@@ -1249,7 +1338,7 @@ __global__ void __launch_bounds__(256) k_mtrace(const float* __restrict__ D, flo
     using G = MT<N, DIM>;
     constexpr int M = G::M, NT = G::NT, TPE = G::TPE, EPB = G::EPB, T = G::T;
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    const int tid = threadIdx.x, el = tid / TPE, s = tid % TPE;
+    const int tid = threadIdx.x, el = G::el_of(tid), s = G::pt_of(tid);
     const int e = blockIdx.x * EPB + el;
     const bool live = el < EPB && e < Eint;
     float* Ds = (float*)(lds_raw + (size_t)(el < EPB ? el : 0) * G::ELEM_BYTES);
@@ -1265,7 +1354,7 @@ __global__ void __launch_bounds__(256) k_mtrace(const float* __restrict__ D, flo
         ver[(size_t)Eint + e] = -1;
     }
     for (int task = s; task < T * DIM * NT; task += TPE) {
-        const int t = task / (DIM * NT), r = task % (DIM * NT), d = r / NT, q = r % NT;
+        const int d = task / TPE, t = task % TPE / NT, q = task % NT;
         float* trd = d == 0 ? tr0 : (d == 1 ? tr1 : tr2);
 #pragma unroll
         for (int v = 0; v < NVP; v++) {
@@ -1276,9 +1365,8 @@ __global__ void __launch_bounds__(256) k_mtrace(const float* __restrict__ D, flo
                 x0 += p * S2F[l];
                 x1 += p * S2F[(M - 1) * N + l];
             }
-            float* to = trd + ((((size_t)t * NVP + v) * E + e) * 2) * NT + q;
-            to[0] = x0;
-            to[NT] = x1;
+            trd[trace_at<NT>(E, T, v, 0, e, t, q)] = x0;
+            trd[trace_at<NT>(E, T, v, 1, e, t, q)] = x1;
         }
     }
 }
@@ -1297,7 +1385,7 @@ __global__ void __launch_bounds__(256) k_mrestart(const float* __restrict__ d_ol
     using G = MT<N, DIM>;
     constexpr int M = G::M, NT = G::NT, TPE = G::TPE, EPB = G::EPB, T = G::T;
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    const int tid = threadIdx.x, el = tid / TPE, s = tid % TPE;
+    const int tid = threadIdx.x, el = G::el_of(tid), s = G::pt_of(tid);
     const int e = blockIdx.x * EPB + el;
     const bool live = el < EPB && e < Eint;
     const bool go = live && flags[e] != 0;
@@ -1330,9 +1418,8 @@ __global__ void __launch_bounds__(256) k_mrestart(const float* __restrict__ d_ol
             }
 #pragma unroll
             for (int t = 0; t < T; t++) {
-                float* to = tb + ((((size_t)t * NVP + v) * E + e) * 2) * NT + q;
-                to[0] = x0;
-                to[NT] = x1;
+                tb[trace_at<NT>(E, T, v, 0, e, t, q)] = x0;
+                tb[trace_at<NT>(E, T, v, 1, e, t, q)] = x1;
             }
         }
     }
@@ -1827,13 +1914,20 @@ int run_mixed(spdk_ctx* c, double* U_sp, const int Ne[3], void* ws, double dt, d
     auto sweep = [&](const MArgs& args, unsigned nb) -> int {
         bool rec = c->timing && c->ev_used < spdk_ctx::kEvPool && !args.Ffv[0][0];
         if (rec) SPDK_CHECK(hipEventRecord(c->evs[c->ev_used][0], c->stream));
-        if (args.Ffv[0][0])
-            hipLaunchKernelGGL((k_msweep<N, DIM, 2>), dim3(args.blist ? nb : (nb + 7) / 8 * 8), block, lds, c->stream,
-                               args);
+        if (args.Ffv[0][0]) {
+            constexpr int MF = N == 4 && DIM == 3 ? M_STAGED : M_FACES;
+            const dim3 g8((nb + 7) / 8 * 8);
+            if (MF == M_FACES || args.F_x || args.fv_valu)
+                hipLaunchKernelGGL((k_msweep<N, DIM, M_FACES>), g8, block, lds, c->stream, args);
+            else
+                hipLaunchKernelGGL((k_msweep<N, DIM, MF>), g8, block, lds, c->stream, args);
+        }
         else if (!args.out_pred || args.U_new)
-            hipLaunchKernelGGL((k_msweep<N, DIM, 1>), dim3(nb), block, lds, c->stream, args);
+            hipLaunchKernelGGL((k_msweep<N, DIM, M_CORR>), dim3(nb), block, lds, c->stream, args);
+        else if (args.path)
+            hipLaunchKernelGGL((k_msweep<N, DIM, M_PRED>), dim3(nb), block, lds, c->stream, args);
         else
-            hipLaunchKernelGGL((k_msweep<N, DIM, 0>), dim3(nb), block, lds, c->stream, args);
+            hipLaunchKernelGGL((k_msweep<N, DIM, M_START>), dim3(nb), block, lds, c->stream, args);
         SPDK_LAUNCH_CHECK("k_msweep");
         if (rec) SPDK_CHECK(hipEventRecord(c->evs[c->ev_used++][1], c->stream));
         return SPDK_OK;
@@ -2096,7 +2190,10 @@ int run_iterate(spdk_ctx* c, double* U_sp, const int Ne[3], void* ws, double dt,
         s.tin_slices = k == 0 ? 1 : G::T;
         s.out_pred = 1;
         s.sweep = k;
-        hipLaunchKernelGGL((k_msweep<N, DIM, 0>), dim3(L.blocks), dim3(G::BLOCK), G::LDS_BYTES, c->stream, s);
+        if (s.path)
+            hipLaunchKernelGGL((k_msweep<N, DIM, M_PRED>), dim3(L.blocks), dim3(G::BLOCK), G::LDS_BYTES, c->stream, s);
+        else
+            hipLaunchKernelGGL((k_msweep<N, DIM, M_START>), dim3(L.blocks), dim3(G::BLOCK), G::LDS_BYTES, c->stream, s);
         SPDK_LAUNCH_CHECK("k_msweep");
     }
     return SPDK_OK;
