@@ -181,7 +181,7 @@ __device__ __forceinline__ void fv_faces(const SweepArgs& a, double* scr, const 
 #pragma unroll
                         for (int ll = 0; ll < N; ll++) {
                             const int q = d == 1 ? ll * N + nn : nn * N + ll;
-                            u += Fs[(d * NVP + v) * FSZ + fidx(d, f1, q, N, NT, M)] * S[o1 * N + ll];
+                            u += Fs[(d * NVP + v) * FSZ + fidx(d, f1, q, N, NT, M)] * cload(S, o1 * N + ll);
                         }
                         scr[v * TPE + s] = u;
                     }
@@ -194,7 +194,7 @@ __device__ __forceinline__ void fv_faces(const SweepArgs& a, double* scr, const 
                 for (int v = 0; v < NVP; v++) {
                     double acc = 0;
 #pragma unroll
-                    for (int nn = 0; nn < N; nn++) acc += scr[v * TPE + (f * N + o1) * N + nn] * S[o2 * N + nn];
+                    for (int nn = 0; nn < N; nn++) acc += scr[v * TPE + (f * N + o1) * N + nn] * cload(S, o2 * N + nn);
                     accv[v] = acc;
                 }
             }
@@ -240,14 +240,14 @@ __device__ __forceinline__ void fv_faces(const SweepArgs& a, double* scr, const 
 #pragma unroll
                     for (int ll = 0; ll < N; ll++) {
                         double x = Fs[v * FSZ + fidx(0, f, ll, N, NT, M)];
-                        x *= S[o[1] * N + ll];
+                        x *= cload(S, o[1] * N + ll);
                         acc += x;
                     }
                 } else {  // d = 1: dim1 = z inactive, dim2 = x active
 #pragma unroll
                     for (int nn = 0; nn < N; nn++) {
                         double x = Fs[(NVP + v) * FSZ + fidx(1, f, nn, N, NT, M)];
-                        x *= S[o[0] * N + nn];
+                        x *= cload(S, o[0] * N + nn);
                         acc += x;
                     }
                 }
@@ -300,7 +300,7 @@ __device__ __forceinline__ void pencil(const SweepArgs& a, const double* U, size
         for (int v = 0; v < NVP; v++) {
             double x = 0;
 #pragma unroll
-            for (int l = 0; l < N; l++) x += p[v][l] * a.S2F[f * N + l];
+            for (int l = 0; l < N; l++) x += p[v][l] * cload(a.S2F, f * N + l);
             u[v] = x;
         }
     };
@@ -376,14 +376,16 @@ __global__ void __launch_bounds__(256, MODE == FACES ? 2 : SPDK_SWEEP_WAVES) k_s
     const int tid = threadIdx.x;
     const int bx = MODE == FACES ? face_sweep_block() : (int)blockIdx.x;
     if (MODE == FACES && bx * EL >= a.E) return;  // padding of the XCD-ordered grid (uniform per block)
-    const int unit = tid / TPE, s = tid % TPE;    // (element, slice) and solution point of this thread
+    // (element, slice) and solution point of this thread; the former is the
+    // wave's where a slice fills it, and its addresses are then scalar
+    const int unit = TPE == 64 ? __builtin_amdgcn_readfirstlane(tid / 64) : tid / TPE, s = tid % TPE;
     const int el = unit / S, ut = unit % S;
     const int e = bx * EL + el;
     const bool live = unit < X::UNITS && e < a.E;
     const size_t E = (size_t)a.E;
     const size_t slabE = E * TPE;  // one (t,v) plane of a state array
     double* const Fs = lds + (unit < X::UNITS ? unit : 0) * X::AREA + X::SCR;
-    for (int i = tid; i < N * M; i += G::BLOCK) sD[i] = a.Dm[i];
+    for (int i = tid; i < N * M; i += G::BLOCK) sD[i] = cload(a.Dm, i);
 
     int ei = 0, ej = 0, ek = 0;
     if (live) {
@@ -508,7 +510,7 @@ __global__ void __launch_bounds__(256, MODE == FACES ? 2 : SPDK_SWEEP_WAVES) k_s
                     for (int v = 0; v < NVP; v++) {
                         double du = 0;
 #pragma unroll
-                        for (int l = 0; l < T; l++) du += rate(l, v) * a.inv[t * T + l] * a.w[l] * a.dt;
+                        for (int l = 0; l < T; l++) du += rate(l, v) * cload(a.inv, t * T + l) * cload(a.w, l) * a.dt;
                         const double un = u_old[v] - du;
                         a.U_out[((size_t)t * NVP + v) * slabE + (size_t)e * TPE + s] = un;
                         slice_at(t)[v * TPE + s] = un;
@@ -536,7 +538,7 @@ __global__ void __launch_bounds__(256, MODE == FACES ? 2 : SPDK_SWEEP_WAVES) k_s
                                 double r = rate(l, v);
                                 if (v >= 1 && v <= 3) r -= n[0] * a.g[v - 1];
                                 if (v == 4) r -= n[TPE] * a.g[0] + n[2 * TPE] * a.g[1] + n[3 * TPE] * a.g[2];
-                                du += r * a.inv[t * T + l] * a.w[l] * a.dt;
+                                du += r * cload(a.inv, t * T + l) * cload(a.w, l) * a.dt;
                             }
                             const double un = u_old[v] - du;
                             a.U_out[((size_t)t * NVP + v) * slabE + (size_t)e * TPE + s] = un;
@@ -563,9 +565,9 @@ __global__ void __launch_bounds__(256, MODE == FACES ? 2 : SPDK_SWEEP_WAVES) k_s
                 for (int l = 0; l < N; l++) p[l] = un[v * TPE + l0 + l * ls];
                 double x0 = 0, x1 = 0;
 #pragma unroll
-                for (int l = 0; l < N; l++) x0 += p[l] * a.S2F[l];
+                for (int l = 0; l < N; l++) x0 += p[l] * cload(a.S2F, l);
 #pragma unroll
-                for (int l = 0; l < N; l++) x1 += p[l] * a.S2F[(M - 1) * N + l];
+                for (int l = 0; l < N; l++) x1 += p[l] * cload(a.S2F, (M - 1) * N + l);
                 double* to = tr + (((size_t)t * NVP + v) * E + pe) * 2 * NT + q;
                 to[0] = x0;
                 to[NT] = x1;
@@ -583,7 +585,7 @@ __global__ void __launch_bounds__(256, MODE == FACES ? 2 : SPDK_SWEEP_WAVES) k_s
         for (int v = 0; v < NVP; v++) {
             double du = 0;
 #pragma unroll
-            for (int t = 0; t < T; t++) du += rate(t, v) * a.w[t] * a.dt;
+            for (int t = 0; t < T; t++) du += rate(t, v) * cload(a.w, t) * a.dt;
             un[v] = u_old[v] - du;
         }
         if (a.rk_a != 0.0) {  // combine_solution (src/transforms.cpp:252-261)
@@ -620,7 +622,7 @@ __global__ void __launch_bounds__(256, MODE == FACES ? 2 : SPDK_SWEEP_WAVES) k_s
 #pragma unroll
                 for (int l = 0; l < N; l++) {
                     int sl = d == 0 ? s - ii + l : (d == 1 ? s + (l - jj) * N : s + (l - kk) * N * N);
-                    x += src[v * TPE + sl] * a.S2C[id * N + l];
+                    x += src[v * TPE + sl] * cload(a.S2C, id * N + l);
                 }
                 dst[v * TPE + s] = x;
             }

@@ -125,7 +125,11 @@ struct MArgs {
     const float* d_old;     // (5,E,TPE) U_sp - mu
     float* D;               // (T,5,E,TPE) predictor state, read and rewritten in place
     float* trb[2][3];       // two trace buffers per axis, (5,2,E,slices,NT) (see trace_at)
-    int* ver;               // (2,E): sweep number of each element's last write to each buffer
+    // (2,E): sweep number of each element's last write to each buffer. Read with
+    // cload although the sweep writes it: the value that replaces an entry, the
+    // current sweep's number, leads every reader to the same buffer as the
+    // entry it replaces
+    int* ver;
     int cur;                // this sweep's number
     const unsigned char* big_in;  // per element: r_e >= tol in the previous sweep (null: every element active)
     const int* blist;       // blocks to run (grid = its length; null: every block)
@@ -164,16 +168,6 @@ struct MArgs {
     const float* SS;
     int fv_valu;
 };
-
-// p[i] of an array that the kernel's own writes cannot change: through the
-// constant address space, so that wave-uniform elements come by scalar loads
-// and the others may be loaded ahead of fences and stores. (a.ver is written
-// by the sweep, but the value that replaces an entry, the current sweep's
-// number, leads every reader to the same buffer as the entry it replaces.)
-template <typename V>
-__device__ __forceinline__ V cload(const V* p, size_t i) {
-    return ((const __attribute__((address_space(4))) V*)p)[i];
-}
 
 // ---- FP64 physics in the frame of the face normal: slot 1 is the normal
 // momentum, slots 2 and 3 the transverse ones (cyclic, as V1, V2, V3 of

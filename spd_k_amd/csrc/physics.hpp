@@ -48,6 +48,16 @@ __device__ __forceinline__ double sound_speed(double rho, double p, double gm) {
     return sqrt(c2);
 }
 
+// p[i] of an array that the kernel's own writes cannot change: through the
+// constant address space, so that wave-uniform elements come by scalar loads
+// and the others may be loaded ahead of barriers, fences and stores. A plain
+// load of a matrix is repeated per lane after each of them, because the
+// compiler cannot show that the kernel's stores leave the matrix alone.
+template <typename V>
+__device__ __forceinline__ V cload(const V* p, size_t i) {
+    return ((const __attribute__((address_space(4))) V*)p)[i];
+}
+
 // Primitive variables of one state (src/hydro.cpp:95-106). E_kin starts at
 // +0.0 and accumulates in x, y, z order.
 __device__ __forceinline__ void prim(const double* u, double* w, double gm) {
