@@ -46,6 +46,8 @@ struct Geo {  // FV sub-grid coordinates per axis (device pointers)
     const double* c[3];
     // widths with their divisions: c[l+1] - c[l], c[l+1] - c[l-1], f[l+1] - f[l] at index l
     const ConstDiv *dc1[3], *dc2[3], *df[3];
+    // width of cell l, loaded once however many stores lie between its uses
+    __device__ __forceinline__ double h(int d, int l) const { return cload(f[d], l + 1) - cload(f[d], l); }
 };
 
 // ---------------------------------------------------------------------------
@@ -186,9 +188,9 @@ __device__ __forceinline__ void fv_cell(double* __restrict__ Un, double* __restr
         double h, F = 0;
         double uo = Ucv[v * slab + o];
         if (write_old) Uo[sc.off(v, K, J, I)] = uo;
-        if (a.act[0]) { h = geo.f[0][I + 1] - geo.f[0][I]; F += (Fx[sx.off(v, K, J, I + 1)] - Fx[sx.off(v, K, J, I)]) / h; }
-        if (a.act[1]) { h = geo.f[1][J + 1] - geo.f[1][J]; F += (Fy[sy.off(v, K, J + 1, I)] - Fy[sy.off(v, K, J, I)]) / h; }
-        if (a.act[2]) { h = geo.f[2][K + 1] - geo.f[2][K]; F += (Fz[sz.off(v, K + 1, J, I)] - Fz[sz.off(v, K, J, I)]) / h; }
+        if (a.act[0]) { h = geo.h(0, I); F += (Fx[sx.off(v, K, J, I + 1)] - Fx[sx.off(v, K, J, I)]) / h; }
+        if (a.act[1]) { h = geo.h(1, J); F += (Fy[sy.off(v, K, J + 1, I)] - Fy[sy.off(v, K, J, I)]) / h; }
+        if (a.act[2]) { h = geo.h(2, K); F += (Fz[sz.off(v, K + 1, J, I)] - Fz[sz.off(v, K, J, I)]) / h; }
         if (a.grav) {
             double S = 0.0;
             if (v == 1) S = Ucv[o] * a.g[0];
@@ -254,9 +256,9 @@ __global__ void __launch_bounds__(BS) k_fv_update_prims(double* __restrict__ Un,
     for (int v = 0; v < NV; v++) {
         double h, F = 0;
         uo[v] = Ucv[v * slab + o];
-        if (a.act[0]) { h = geo.f[0][I + 1] - geo.f[0][I]; F += (Fx[sx.off(v, K, J, I + 1)] - Fx[sx.off(v, K, J, I)]) / h; }
-        if (a.act[1]) { h = geo.f[1][J + 1] - geo.f[1][J]; F += (Fy[sy.off(v, K, J + 1, I)] - Fy[sy.off(v, K, J, I)]) / h; }
-        if (a.act[2]) { h = geo.f[2][K + 1] - geo.f[2][K]; F += (Fz[sz.off(v, K + 1, J, I)] - Fz[sz.off(v, K, J, I)]) / h; }
+        if (a.act[0]) { h = geo.h(0, I); F += (Fx[sx.off(v, K, J, I + 1)] - Fx[sx.off(v, K, J, I)]) / h; }
+        if (a.act[1]) { h = geo.h(1, J); F += (Fy[sy.off(v, K, J + 1, I)] - Fy[sy.off(v, K, J, I)]) / h; }
+        if (a.act[2]) { h = geo.h(2, K); F += (Fz[sz.off(v, K + 1, J, I)] - Fz[sz.off(v, K, J, I)]) / h; }
         if (a.grav) {
             double S = 0.0;
             if (v == 1) S = Ucv[o] * a.g[0];
@@ -328,42 +330,40 @@ template <int Q, int D>
 struct ElTile {
     static constexpr int TPE = D == 1 ? Q : (D == 2 ? Q * Q : Q * Q * Q);
     static constexpr int EPB = TPE >= BS ? 1 : BS / TPE;
+    static constexpr int PLANE = EPB * TPE;  // LDS plane of one variable
 };
 
-// transform_a_to_b of one element (src/transforms.cpp:81-118 per axis, x then
-// y then z): point s of the element enters as `in`, its transformed value is
-// returned. b0/b1 are the element's two LDS planes; every thread of the block
-// calls it (it holds barriers).
+// transform_a_to_b of the physical variables of one element
+// (src/transforms.cpp:81-118 per axis, x then y then z): point s of the
+// element enters with u and leaves with its transformed values. b0/b1 are the
+// element's LDS planes, a variable ElTile::PLANE after the one before; every
+// thread of the block calls it (it holds barriers: one set for all variables).
 template <int Q, int D>
-__device__ __forceinline__ double el_transform(double in, double* b0, double* b1, const double* sM, int s, bool live) {
-    const int ii = s % Q, jj = (s / Q) % Q, kk = s / (Q * Q);
+__device__ __forceinline__ void el_transform(double (&u)[NVP], double* b0, double* b1, const double* sM, int s, bool live) {
+    constexpr int PL = ElTile<Q, D>::PLANE;
+    const int x[3] = {s % Q, (s / Q) % Q, s / (Q * Q)};
+    constexpr int st[3] = {1, Q, Q * Q};
     __syncthreads();
-    if (live) b0[s] = in;
-    __syncthreads();
-    double u = 0;
-    if (live) {
 #pragma unroll
-        for (int l = 0; l < Q; l++) u += b0[s - ii + l] * sM[ii * Q + l];
-    }
-    if (D >= 2) {
-        if (live) b1[s] = u;
+    for (int d = 0; d < D; d++) {
+        double* b = d == 1 ? b1 : b0;
+        if (live)
+#pragma unroll
+            for (int v = 0; v < NVP; v++) b[v * PL + s] = u[v];
         __syncthreads();
-        u = 0;
         if (live) {
+            double m[Q];
 #pragma unroll
-            for (int l = 0; l < Q; l++) u += b1[s + (l - jj) * Q] * sM[jj * Q + l];
-        }
-        if (D == 3) {
-            if (live) b0[s] = u;
-            __syncthreads();
-            u = 0;
-            if (live) {
+            for (int l = 0; l < Q; l++) m[l] = sM[x[d] * Q + l];
+            const double* p = b + s - x[d] * st[d];
 #pragma unroll
-                for (int l = 0; l < Q; l++) u += b0[s + (l - kk) * Q * Q] * sM[kk * Q + l];
+            for (int v = 0; v < NVP; v++) {
+                u[v] = 0;
+#pragma unroll
+                for (int l = 0; l < Q; l++) u[v] += p[v * PL + l * st[d]] * m[l];
             }
         }
     }
-    return u;
 }
 
 // Slot q of a workgroup's FV rows: the row (jj, kk) of the EPB elements, x
@@ -388,7 +388,7 @@ __global__ void __launch_bounds__(BS) k_fv_state_in(const double* __restrict__ U
                                                     int fx, int fy, int fz, int ex, int ey, int gpr, uint32_t groups) {
     using TL = ElTile<Q, D>;
     constexpr int TPE = TL::TPE, EPB = TL::EPB;
-    __shared__ double b0[EPB * TPE], b1[EPB * TPE], sM[Q * Q];
+    __shared__ double b0[NVP * TL::PLANE], b1[NVP * TL::PLANE], sM[Q * Q];
     const uint32_t g = xcd_block();  // neighbouring groups share FV row lines: one L2
     if (g >= groups) return;
     const int tid = threadIdx.x, el = tid / TPE, sp = tid % TPE;
@@ -401,20 +401,24 @@ __global__ void __launch_bounds__(BS) k_fv_state_in(const double* __restrict__ U
     const size_t eo = ((((size_t)(k + gz) * s.Ny + (j + gy)) * s.Nx) + (i + gx)) * TPE + sp;
     double* e0 = b0 + (live ? el : 0) * TPE;
     double* e1 = b1 + (live ? el : 0) * TPE;
-    for (int v = 0; v < NVP; v++) {
-        const double u = el_transform<Q, D>(live ? Usp[v * slab + eo] : 0.0, e0, e1, sM, sp, live);
-        __syncthreads();
-        if (live) b1[el * TPE + sp] = u;
-        __syncthreads();
-        if (tid < EPB * TPE) {
-            int e, pt, ii, jj, kk;
-            fv_slot<Q, D>(tid, e, pt, ii, jj, kk);
-            if (i0 + e < ex) {
-                const int I = fx + (i0 + e) * Q + ii;
-                const int J = D >= 2 ? fy + j * Q + jj : fy + j;
-                const int K = D == 3 ? fz + k * Q + kk : fz + k;
-                Ufv[sc.off(v, K, J, I)] = b1[e * TPE + pt];
-            }
+    double u[NVP];
+#pragma unroll
+    for (int v = 0; v < NVP; v++) u[v] = live ? Usp[v * slab + eo] : 0.0;
+    el_transform<Q, D>(u, e0, e1, sM, sp, live);
+    __syncthreads();
+    if (live)
+#pragma unroll
+        for (int v = 0; v < NVP; v++) e1[v * TL::PLANE + sp] = u[v];
+    __syncthreads();
+    if (tid < EPB * TPE) {
+        int e, pt, ii, jj, kk;
+        fv_slot<Q, D>(tid, e, pt, ii, jj, kk);
+        if (i0 + e < ex) {
+            const int I = fx + (i0 + e) * Q + ii;
+            const int J = D >= 2 ? fy + j * Q + jj : fy + j;
+            const int K = D == 3 ? fz + k * Q + kk : fz + k;
+#pragma unroll
+            for (int v = 0; v < NVP; v++) Ufv[sc.off(v, K, J, I)] = b1[v * TL::PLANE + e * TPE + pt];
         }
     }
 }
@@ -440,9 +444,9 @@ __global__ void __launch_bounds__(BS) k_fv_state_update_prims(double* __restrict
     for (int v = 0; v < NVP; v++) {
         double h, F = 0;
         uo[v] = Ucv[v * pl + o];
-        if (a.act[0]) { h = geo.f[0][I + 1] - geo.f[0][I]; F += (Fx[sx.off(v, K, J, I + 1)] - Fx[sx.off(v, K, J, I)]) / h; }
-        if (a.act[1]) { h = geo.f[1][J + 1] - geo.f[1][J]; F += (Fy[sy.off(v, K, J + 1, I)] - Fy[sy.off(v, K, J, I)]) / h; }
-        if (a.act[2]) { h = geo.f[2][K + 1] - geo.f[2][K]; F += (Fz[sz.off(v, K + 1, J, I)] - Fz[sz.off(v, K, J, I)]) / h; }
+        if (a.act[0]) { h = geo.h(0, I); F += (Fx[sx.off(v, K, J, I + 1)] - Fx[sx.off(v, K, J, I)]) / h; }
+        if (a.act[1]) { h = geo.h(1, J); F += (Fy[sy.off(v, K, J + 1, I)] - Fy[sy.off(v, K, J, I)]) / h; }
+        if (a.act[2]) { h = geo.h(2, K); F += (Fz[sz.off(v, K + 1, J, I)] - Fz[sz.off(v, K, J, I)]) / h; }
         if (a.grav) {
             double S = 0.0;
             if (v == 1) S = uo[0] * a.g[0];
@@ -494,10 +498,10 @@ __global__ void __launch_bounds__(BS) k_fv_state_update_prims_z(double* __restri
         for (int v = 0; v < NVP; v++) {
             double h, F = 0;
             uo[v] = Ucv[v * pl + o];
-            if (a.act[0]) { h = geo.f[0][I + 1] - geo.f[0][I]; F += (Fx[sx.off(v, K, J, I + 1)] - Fx[sx.off(v, K, J, I)]) / h; }
-            if (a.act[1]) { h = geo.f[1][J + 1] - geo.f[1][J]; F += (Fy[sy.off(v, K, J + 1, I)] - Fy[sy.off(v, K, J, I)]) / h; }
+            if (a.act[0]) { h = geo.h(0, I); F += (Fx[sx.off(v, K, J, I + 1)] - Fx[sx.off(v, K, J, I)]) / h; }
+            if (a.act[1]) { h = geo.h(1, J); F += (Fy[sy.off(v, K, J + 1, I)] - Fy[sy.off(v, K, J, I)]) / h; }
             const double fup = Fz[sz.off(v, K + 1, J, I)];
-            h = geo.f[2][K + 1] - geo.f[2][K];
+            h = geo.h(2, K);
             F += (fup - flo[v]) / h;
             flo[v] = fup;
             if (a.grav) {
@@ -550,9 +554,9 @@ __global__ void __launch_bounds__(BS) k_fv_state_update_blended(double* __restri
     for (int v = 0; v < NVP; v++) {
         double h, F = 0;
         const double uo = Ucv[v * pl + o];
-        if (a.act[0]) { h = geo.f[0][I + 1] - geo.f[0][I]; F += (Fx[sx.off(v, K, J, I + 1)] - Fx[sx.off(v, K, J, I)]) / h; }
-        if (a.act[1]) { h = geo.f[1][J + 1] - geo.f[1][J]; F += (Fy[sy.off(v, K, J + 1, I)] - Fy[sy.off(v, K, J, I)]) / h; }
-        if (a.act[2]) { h = geo.f[2][K + 1] - geo.f[2][K]; F += (Fz[sz.off(v, K + 1, J, I)] - Fz[sz.off(v, K, J, I)]) / h; }
+        if (a.act[0]) { h = geo.h(0, I); F += (Fx[sx.off(v, K, J, I + 1)] - Fx[sx.off(v, K, J, I)]) / h; }
+        if (a.act[1]) { h = geo.h(1, J); F += (Fy[sy.off(v, K, J + 1, I)] - Fy[sy.off(v, K, J, I)]) / h; }
+        if (a.act[2]) { h = geo.h(2, K); F += (Fz[sz.off(v, K + 1, J, I)] - Fz[sz.off(v, K, J, I)]) / h; }
         if (a.grav) {
             double S = 0.0;
             if (v == 1) S = un[0] * a.g[0];
@@ -584,7 +588,7 @@ __global__ void __launch_bounds__(BS) k_fv_state_out(const double* __restrict__ 
                                                      double* __restrict__ part) {
     using TL = ElTile<Q, D>;
     constexpr int TPE = TL::TPE, EPB = TL::EPB;
-    __shared__ double b0[EPB * TPE], b1[EPB * TPE], sI[EPB * TPE], sMc[Q * Q], sMs[Q * Q];
+    __shared__ double b0[NVP * TL::PLANE], b1[NVP * TL::PLANE], sMc[Q * Q], sMs[Q * Q];
     __shared__ double red[BS];
     const int tid = threadIdx.x, el = tid / TPE, sp = tid % TPE;
     if (tid < Q * Q) {
@@ -603,38 +607,54 @@ __global__ void __launch_bounds__(BS) k_fv_state_out(const double* __restrict__ 
         const size_t eo = (((size_t)k * s.Ny + j) * s.Nx + i) * TPE + sp;
         double* e0 = b0 + (live ? el : 0) * TPE;
         double* e1 = b1 + (live ? el : 0) * TPE;
-        double u[NVP];
-        for (int v = 0; v < NVP; v++) {
-            // the cell values: FV rows for active elements, the forward
-            // transform of U_sp for ghost elements
-            __syncthreads();
-            if (act_row && tid < EPB * TPE) {
-                int e, pt, ii, jj, kk;
-                fv_slot<Q, D>(tid, e, pt, ii, jj, kk);
-                const int ie = i0 + e;
-                if (ie >= gx && ie < s.Nx - gx) {
-                    const int I = fx + (ie - gx) * Q + ii;
-                    const int J = D >= 2 ? fy + (j - gy) * Q + jj : fy + (j - gy);
-                    const int K = D == 3 ? fz + (k - gz) * Q + kk : fz + (k - gz);
-                    sI[e * TPE + pt] = Ufv[sc.off(v, K, J, I)];
-                }
+        // the cell values: FV rows for active elements, the forward transform
+        // of U_sp for ghost elements (in the groups that hold any)
+        const bool ghosts = !act_row || i0 < gx || i0 + EPB > s.Nx - gx;  // uniform per block
+        double u[NVP], gs[NVP], x[NVP];
+        int slot = -1;
+        if (act_row && tid < EPB * TPE) {
+            int e, pt, ii, jj, kk;
+            fv_slot<Q, D>(tid, e, pt, ii, jj, kk);
+            const int ie = i0 + e;
+            if (ie >= gx && ie < s.Nx - gx) {
+                slot = e * TPE + pt;
+                const int I = fx + (ie - gx) * Q + ii;
+                const int J = D >= 2 ? fy + (j - gy) * Q + jj : fy + (j - gy);
+                const int K = D == 3 ? fz + (k - gz) * Q + kk : fz + (k - gz);
+#pragma unroll
+                for (int v = 0; v < NVP; v++) x[v] = Ufv[sc.off(v, K, J, I)];
             }
-            const double cg = el_transform<Q, D>(live && !active ? Usp[v * slab + eo] : 0.0, e0, e1, sMs, sp,
-                                                 live && !active);
-            const double cv = active ? sI[el * TPE + sp] : cg;
-            u[v] = el_transform<Q, D>(cv, e0, e1, sMc, sp, live);
-            if (live) Usp[v * slab + eo] = u[v];
         }
+        if (ghosts)
+#pragma unroll
+            for (int v = 0; v < NVP; v++) gs[v] = live && !active ? Usp[v * slab + eo] : 0.0;
+        __syncthreads();
+        if (slot >= 0)
+#pragma unroll
+            for (int v = 0; v < NVP; v++) b1[v * TL::PLANE + slot] = x[v];
+        __syncthreads();
+#pragma unroll
+        for (int v = 0; v < NVP; v++) u[v] = active ? e1[v * TL::PLANE + sp] : 0.0;
+        if (ghosts) {
+            el_transform<Q, D>(gs, e0, e1, sMs, sp, live && !active);
+            if (!active)
+#pragma unroll
+                for (int v = 0; v < NVP; v++) u[v] = gs[v];
+        }
+        el_transform<Q, D>(u, e0, e1, sMc, sp, live);
+        if (live)
+#pragma unroll
+            for (int v = 0; v < NVP; v++) Usp[v * slab + eo] = u[v];
         if (!want_w && !want_dt) continue;
         double w[NVP];
         if (live) prim(u, w, dta.gm);
         else
             for (int v = 0; v < NVP; v++) w[v] = 0.0;
-        double wc[NVP];
-        for (int v = 0; v < NVP; v++) {
-            wc[v] = el_transform<Q, D>(w[v], e0, e1, sMs, sp, live);
-            if (live && want_w) Wcv[v * slab + eo] = wc[v];
-        }
+        el_transform<Q, D>(w, e0, e1, sMs, sp, live);
+        const double (&wc)[NVP] = w;
+        if (live && want_w)
+#pragma unroll
+            for (int v = 0; v < NVP; v++) Wcv[v * slab + eo] = wc[v];
         if (active && want_dt) {
             const double c_s = sound_speed(wc[0], wc[4], dta.gm);
             double c_max = 0, dx_min = 1, dt_min;
@@ -738,12 +758,19 @@ __global__ void __launch_bounds__(BS) k_fv_bc_all(double* __restrict__ U, FV s, 
     const int si = b.act[0] ? bc_src(i, s.Nx, b.type[0], fx) : i;
     const int sj = b.act[1] ? bc_src(j, s.Ny, b.type[1], fy) : j;
     const int sk = b.act[2] ? bc_src(k, s.Nz, b.type[2], fz) : k;
-    for (int v = 0; v < s.nv; v++) {
-        double u = U[s.off(v, sk, sj, si)];
-        if (fx && v == 1) u = -1.0 * u;
-        if (fy && v == 2) u = -1.0 * u;
-        if (fz && v == 3) u = -1.0 * u;
-        U[s.off(v, k, j, i)] = u;
+    // all of a cell's loads, then its stores: one round trip instead of one
+    // per variable (64^2 elements p=3: 3.9 -> 3.4 us)
+    for (int v0 = 0; v0 < s.nv; v0 += NV) {
+        double u[NV];
+#pragma unroll
+        for (int v = 0; v < NV; v++)
+            if (v0 + v < s.nv) u[v] = U[s.off(v0 + v, sk, sj, si)];
+#pragma unroll
+        for (int v = 0; v < NV; v++) {
+            if (v0 + v >= s.nv) continue;
+            if (v0 == 0 && ((fx && v == 1) || (fy && v == 2) || (fz && v == 3))) u[v] = -1.0 * u[v];
+            U[s.off(v0 + v, k, j, i)] = u[v];
+        }
     }
 }
 
@@ -1038,32 +1065,43 @@ __global__ void __launch_bounds__(BS) k_relax_pad(const double* __restrict__ Wn,
         if (AZ) az = (uint32_t)abits[c0 - sz] & m0 & (uint32_t)abits[c0 + sz] & kZ;
         all_ge1 = ax | ay | az;
     }
-    for (int v = 0; v < nvar; v++) {
-        if (!((a.mask >> v) & 1)) continue;
-        const size_t o = v * pl + c0;
-        bool small;  // the smallest alpha around the cell is below 1
-        if (BITS) {
-            const uint32_t need = (AX ? 1u << (v * 3) : 0u) | (AY ? 1u << (v * 3 + 1) : 0u) | (AZ ? 1u << (v * 3 + 2) : 0u);
-            small = (all_ge1 & need) != need;
-        } else {
-            double alpha = 1;
-            if (AX) alpha = smin(smin(alx[o - 1], alx[o]), alx[o + 1]);
-            if (AY) alpha = smin(alpha, smin(smin(aly[o - sy], aly[o]), aly[o + sy]));
-            if (AZ) alpha = smin(alpha, smin(smin(alz[o - sz], alz[o]), alz[o + sz]));
-            small = alpha < 1;
+    // the troubles are loaded before the first is stored (the same array), five variables at a time
+    constexpr int V = 5;
+    double tmax = 0;
+    for (int v0 = 0; v0 < nvar; v0 += V) {
+        double t[V];
+#pragma unroll
+        for (int w = 0; w < V; w++)
+            if (v0 + w < nvar && ((a.mask >> (v0 + w)) & 1)) t[w] = tr[(v0 + w) * pl + c0];
+#pragma unroll
+        for (int w = 0; w < V; w++) {
+            const int v = v0 + w;
+            if (v >= nvar || !((a.mask >> v) & 1)) continue;
+            const size_t o = v * pl + c0;
+            if (a.use_sed) {
+                bool small;  // the smallest alpha around the cell is below 1
+                if (BITS) {
+                    const uint32_t need = (AX ? 1u << (v * 3) : 0u) | (AY ? 1u << (v * 3 + 1) : 0u) | (AZ ? 1u << (v * 3 + 2) : 0u);
+                    small = (all_ge1 & need) != need;
+                } else {
+                    double alpha = 1;
+                    if (AX) alpha = smin(smin(alx[o - 1], alx[o]), alx[o + 1]);
+                    if (AY) alpha = smin(alpha, smin(smin(aly[o - sy], aly[o]), aly[o + sy]));
+                    if (AZ) alpha = smin(alpha, smin(smin(alz[o - sz], alz[o]), alz[o + sz]));
+                    small = alpha < 1;
+                }
+                if (!small) t[w] = 0;
+                tr[o] = t[w];
+            }
+            tmax = smax(tmax, t[w]);
         }
-        double t = tr[o];
-        if (a.use_sed) tr[o] = small ? t : 0;
     }
-    double t = 0;
-    for (int v = 0; v < nvar; v++)
-        if ((a.mask >> v) & 1) t = smax(t, tr[v * pl + c0]);
-    tr[nvar * pl + c0] = t;
     if (a.pad) {
-        double d = Wn[c0], p = Wn[4 * pl + c0];
-        if (d < kRhoMin || d > kRhoMax) tr[nvar * pl + c0] = 1;
-        if (p < kPMin || p > kPMax) tr[nvar * pl + c0] = 1;
+        const double d = Wn[c0], p = Wn[4 * pl + c0];
+        if (d < kRhoMin || d > kRhoMax) tmax = 1;
+        if (p < kPMin || p > kPMax) tmax = 1;
     }
+    tr[nvar * pl + c0] = tmax;
 }
 
 // apply_blending (src/trouble_detection.cpp:191-210), cells 1..N-2
