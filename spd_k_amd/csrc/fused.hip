@@ -27,7 +27,7 @@ namespace {
 
 constexpr int kMaxT = 8;
 
-// Waves per SIMD the sweeps are compiled for (FACES: 2). At 4 (128 registers)
+// Waves per SIMD the sweeps are compiled for (FACES: 3). At 4 (128 registers)
 // the 3-D p=3 sweeps spill 2 to 10 registers and still gain over 3: predictor
 // 5.58 -> 5.25 ms, corrector 4.61 -> 4.41 ms at 64^3, 2-D p=3 predictor
 // 0.295 -> 0.239 ms at 256^2.
@@ -129,6 +129,14 @@ __device__ __forceinline__ int spidx(int d, int ll, int q) {
     return ll * N * N + q;                                  // q = jj*N + ii
 }
 
+// Element block of a face-integral sweep workgroup: workgroups go to the 8
+// XCDs in turn and XCD x takes the x-th contiguous eighth of the blocks, so
+// the face rows that neighbouring blocks share (rows are not line-aligned)
+// are written through one L2. The grid is padded to a multiple of 8.
+__device__ __forceinline__ int face_sweep_block() {
+    return (int)((blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8);
+}
+
 // face_integral of slice t for every active axis (src/transforms.cpp:378-481)
 // from the element's flux-point fluxes in LDS (Fs, the fidx layout of each
 // axis): each element writes the sub-cell faces of its cells' lower sides
@@ -139,21 +147,19 @@ __device__ __forceinline__ int spidx(int d, int ll, int q) {
 // after the pencils) and the dim2 sum over nn of u S(o2, nn) is written;
 // otherwise the single contraction of face_integral_ref. Sums in the
 // reference's order, so the faces equal the stage kernels' bit for bit.
-__device__ __forceinline__ int el_of(int tid, int tpe) { return tid / tpe; }
-
-// Element block of a face-integral sweep workgroup: workgroups go to the 8
-// XCDs in turn and XCD x takes the x-th contiguous eighth of the blocks, so
-// the face rows that neighbouring blocks share (rows are not line-aligned)
-// are written through one L2. The grid is padded to a multiple of 8.
-__device__ __forceinline__ int face_sweep_block() {
-    return (int)((blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8);
-}
-
 template <int N, int DIM, int AREA>
-__device__ __forceinline__ void fv_faces(const SweepArgs& a, double* scr, const double* Fs, int t, int s, bool live,
-                                         int ei, int ej, int ek) {
+__device__ __forceinline__ void fv_faces(const SweepArgs& a, double* scr, double* Fs, int t, int s, bool live, int ei,
+                                         int ej, int ek) {
     using G = Tile<N, DIM>;
     constexpr int M = G::M, NT = G::NT, TPE = G::TPE, FSZ = G::FSZ;
+    // 3-D p=3: an element is a wave, so its two contractions need no block
+    // barrier. An axis' faces then replace its fluxes (read for the last time by
+    // its first contraction), and after one barrier per slice the block's four
+    // elements (consecutive along x) write 16 consecutive faces per row, whole
+    // 128-byte rows. With four barriers per axis instead, the waves waited 52%
+    // of their time: 62 x 66 x 61 elements 5.92 -> 5.20 ms.
+    constexpr bool WAVE = TPE == 64 && DIM == 3;
+    static_assert(!WAVE || TPE <= FSZ, "the faces fit over the fluxes");
     const double* S = a.S2C;
     const int ec[3] = {ei, ej, ek};
     const int o[3] = {s % N, DIM >= 2 ? (s / N) % N : 0, DIM == 3 ? s / (N * N) : 0};  // x fastest
@@ -186,8 +192,8 @@ __device__ __forceinline__ void fv_faces(const SweepArgs& a, double* scr, const 
                         scr[v * TPE + s] = u;
                     }
             }
-            __syncthreads();
-            double accv[NVP];
+            if (WAVE) elem_sync();
+            else __syncthreads();
             if (own) {
                 const int o1 = o[dim1], o2 = o[dim2];
 #pragma unroll
@@ -195,41 +201,12 @@ __device__ __forceinline__ void fv_faces(const SweepArgs& a, double* scr, const 
                     double acc = 0;
 #pragma unroll
                     for (int nn = 0; nn < N; nn++) acc += scr[v * TPE + (f * N + o1) * N + nn] * cload(S, o2 * N + nn);
-                    accv[v] = acc;
+                    if (WAVE) Fs[(d * NVP + v) * FSZ + s] = acc;
+                    else if (put) out[(size_t)v * vstride] = acc;
                 }
             }
-            if (G::EPB == 4 && N == 4) {
-                // staged: the block's four elements (consecutive along x) write
-                // 16 consecutive faces per row, whole 128-byte rows
-                __syncthreads();
-                if (own)
-#pragma unroll
-                    for (int v = 0; v < NVP; v++) scr[v * TPE + s] = accv[v];
-                __syncthreads();
-                const int tid = threadIdx.x, xx = tid % 16, row = tid / 16;
-                const int e2l = xx / N, ox = xx % N, oy = row % N, oz = row / N;
-                const int e2 = face_sweep_block() * G::EPB + e2l;
-                if (e2 < a.E) {
-                    const int ec2[3] = {e2 % a.Ne[0], (e2 / a.Ne[0]) % a.Ne[1], e2 / (a.Ne[0] * a.Ne[1])};
-                    bool own2 = true;
-#pragma unroll
-                    for (int x = 0; x < DIM; x++)
-                        own2 = own2 && ec2[x] >= 1 && ec2[x] <= (x == d ? a.Ne[x] - 1 : a.Ne[x] - 2);
-                    const int o2v[3] = {ox, oy, oz};
-                    if (own2 && (ec2[d] < a.Ne[d] - 1 || o2v[d] == 0)) {
-                        const int I2 = ox + a.fgh[0] + (ec2[0] - 1) * N, J2 = oy + a.fgh[1] + (ec2[1] - 1) * N;
-                        const int K2 = oz + a.fgh[2] + (ec2[2] - 1) * N;
-                        double* out2 = a.Ffv[t][d] + ((size_t)K2 * ny + J2) * nx + I2;
-                        const double* sc2 = scr + (long)(e2l - el_of(threadIdx.x, TPE)) * AREA;
-#pragma unroll
-                        for (int v = 0; v < NVP; v++) out2[(size_t)v * vstride] = sc2[v * TPE + ox + N * (oy + N * oz)];
-                    }
-                }
-            } else if (put) {
-#pragma unroll
-                for (int v = 0; v < NVP; v++) out[(size_t)v * vstride] = accv[v];
-            }
-            __syncthreads();
+            if (WAVE) elem_sync();
+            else __syncthreads();
         } else if (put) {  // at most one transverse axis active: face_integral_ref
 #pragma unroll
             for (int v = 0; v < NVP; v++) {
@@ -253,6 +230,32 @@ __device__ __forceinline__ void fv_faces(const SweepArgs& a, double* scr, const 
                 }
                 out[(size_t)v * vstride] = acc;
             }
+        }
+    }
+    if constexpr (WAVE) {
+        static_assert(G::EPB == 4, "four elements per workgroup");
+        __syncthreads();
+        const int tid = threadIdx.x, xx = tid % 16, row = tid / 16;
+        const int e2l = xx / N, ox = xx % N, oy = row % N, oz = row / N;
+        const int e2 = face_sweep_block() * G::EPB + e2l;
+        if (e2 >= a.E) return;
+        const int ec2[3] = {e2 % a.Ne[0], (e2 / a.Ne[0]) % a.Ne[1], e2 / (a.Ne[0] * a.Ne[1])};
+        const int o2[3] = {ox, oy, oz};
+        const int I2 = ox + a.fgh[0] + (ec2[0] - 1) * N, J2 = oy + a.fgh[1] + (ec2[1] - 1) * N;
+        const int K2 = oz + a.fgh[2] + (ec2[2] - 1) * N;
+        const double* F2 = Fs + (long)(e2l - tid / TPE) * AREA + ox + N * (oy + N * oz);
+#pragma unroll
+        for (int d = 0; d < DIM; d++) {
+            bool own2 = ec2[d] < a.Ne[d] - 1 || o2[d] == 0;
+#pragma unroll
+            for (int x = 0; x < DIM; x++)
+                own2 = own2 && ec2[x] >= 1 && ec2[x] <= (x == d ? a.Ne[x] - 1 : a.Ne[x] - 2);
+            if (!own2) continue;
+            const int nx = a.fvn[0] + (d == 0), ny = a.fvn[1] + (d == 1), nz = a.fvn[2] + (d == 2);
+            double* out = a.Ffv[t][d] + ((size_t)K2 * ny + J2) * nx + I2;
+            const size_t vstride = (size_t)nz * ny * nx;
+#pragma unroll
+            for (int v = 0; v < NVP; v++) out[(size_t)v * vstride] = F2[(d * NVP + v) * FSZ];
         }
     }
 }
@@ -367,7 +370,7 @@ __device__ __forceinline__ double divergence_slow(const SweepArgs& a, const doub
 // memory by the pencils and one slice per thread the predictor needs 38.5 KB
 // LDS and fits 4 workgroups per CU.
 template <int N, int DIM, int T, int S, int MODE>
-__global__ void __launch_bounds__(256, MODE == FACES ? 2 : SPDK_SWEEP_WAVES) k_sweep(SweepArgs a) {
+__global__ void __launch_bounds__(256, MODE == FACES ? 3 : SPDK_SWEEP_WAVES) k_sweep(SweepArgs a) {
     using G = Tile<N, DIM>;
     using X = Unit<N, DIM, T, S, MODE>;
     constexpr int M = G::M, NT = G::NT, TPE = G::TPE, EL = X::EL;
@@ -419,7 +422,6 @@ __global__ void __launch_bounds__(256, MODE == FACES ? 2 : SPDK_SWEEP_WAVES) k_s
         __syncthreads();
         if (MODE == FACES || MODE == FLUXES) {  // the stage flux-point layout (src/hydro_ader.hpp:278-289)
             const int t = MODE == FACES ? tl : ut;
-            if (MODE == FACES) fv_faces<N, DIM, X::AREA>(a, Fs - X::SCR, Fs, t, s, live, ei, ej, ek);
             if (live) {
 #pragma unroll
                 for (int d = 0; d < DIM; d++)
@@ -430,7 +432,10 @@ __global__ void __launch_bounds__(256, MODE == FACES ? 2 : SPDK_SWEEP_WAVES) k_s
                         for (int v = NVP; v < a.out_nv; v++) o[(size_t)v * E * G::FSZ] = 0.0;
                     }
             }
-            if (MODE == FACES) __syncthreads();
+            if (MODE == FACES) {  // last: its faces replace the fluxes
+                fv_faces<N, DIM, X::AREA>(a, Fs - X::SCR, Fs, t, s, live, ei, ej, ek);
+                __syncthreads();
+            }
         }
     }
     if (MODE == FACES || MODE == FLUXES) return;

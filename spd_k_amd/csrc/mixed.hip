@@ -496,18 +496,6 @@ __device__ __forceinline__ double pencil_weight(const MArgs& a, int q) {
     return pick(a.wq, q / N) * pick(a.wq, q % N);
 }
 
-// Barrier between phases that touch only the element's own LDS area. An
-// element lies in one wave, so the wave's own order is enough: a wave's LDS
-// operations execute in order, and the wavefront-scope fences keep the
-// compiler from moving its LDS accesses across the point. The waves of a
-// block then run their phases independently (a block barrier makes each wait
-// for the slowest).
-__device__ __forceinline__ void elem_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // New state at the control volumes and the element's dt candidate (FP64):
 // compute_primitives, sp->cv sweeps x, y, z (src/transforms.cpp:99-117) and
 // src/hydro.cpp:226-256. `area` is the element's LDS (>= 2 planes of FP64).

@@ -41,6 +41,18 @@ __device__ __forceinline__ double div_fast(double x, const ConstDiv& c) {
 }
 __device__ __forceinline__ bool div_recheck(double s) { return s != 0.0 && !(fabs(s) >= 0x1p-900); }
 
+// Barrier between phases that touch only an element's own LDS area, where an
+// element lies in one wave, so the wave's own order is enough: a wave's LDS
+// operations execute in order, and the wavefront-scope fences keep the
+// compiler from moving its LDS accesses across the point. The waves of a
+// block then run their phases independently (a block barrier makes each wait
+// for the slowest).
+__device__ __forceinline__ void elem_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // src/hydro.cpp:27-32
 __device__ __forceinline__ double sound_speed(double rho, double p, double gm) {
     double c2 = gm * p / rho;
