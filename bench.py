@@ -185,7 +185,8 @@ def hbm_traffic(n, steps=1):
                 if c not in acc:
                     continue
                 k = row["Kernel_Name"]
-                slot = 0 if "copyBuffer" in k else (1 if "k_msweep<4, 3, 0>" in k else None)
+                # the predictor sweeps: the first from the zero-order guess, the others
+                slot = 0 if "copyBuffer" in k else (1 if re.search(r"k_msweep<4, 3, [01]>", k) else None)
                 if slot is not None:
                     dd = acc[c][slot]
                     dd[row["Dispatch_Id"]] = dd.get(row["Dispatch_Id"], 0.0) + float(row["Counter_Value"])
