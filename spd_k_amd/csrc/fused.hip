@@ -29,7 +29,7 @@ constexpr int kMaxT = 8;
 
 // Waves per SIMD the sweeps are compiled for (FACES: 3). At 4 (128 registers)
 // the 3-D p=3 sweeps spill 2 to 10 registers and still gain over 3: predictor
-// 5.58 -> 5.25 ms, corrector 4.61 -> 4.41 ms at 64^3 (4.3 and 4.2 since the
+// 5.58 -> 5.25 ms, corrector 4.61 -> 4.41 ms at 64^3 (4.6 and 4.4 since the
 // matrices come by scalar loads), 2-D p=3 predictor
 // 0.295 -> 0.239 ms at 256^2.
 #ifndef SPDK_SWEEP_WAVES
