@@ -988,6 +988,8 @@ const Variant* find_variant(spdk_ctx* c) {
     int dim = c->prm.active[0] + c->prm.active[1] + c->prm.active[2];
     // the fused tile assumes active axes are x, x-y or x-y-z
     if (!c->prm.active[0] || (c->prm.active[2] && !c->prm.active[1])) return nullptr;
+    // the kernels are compiled for p+1 slices (ADER) or one (SSP-RK); grid and workspace follow c->T
+    if (c->T != c->n && c->T != 1) return nullptr;
     for (const Variant& v : kVariants)
         if (v.n == c->n && v.dim == dim) return &v;
     return nullptr;
@@ -1029,7 +1031,7 @@ extern "C" {
 size_t spdk_fused_workspace_bytes(spdk_ctx* c, const int N[3]) {
     const Variant* v = c ? find_variant(c) : nullptr;
     if (!v) {
-        set_error("fused path: no tile variant for this degree/dimensionality");
+        set_error("fused path: no tile variant for this degree, dimensionality and slice count");
         return 0;
     }
     if (c->T > kMaxT || c->prm.nu != 0.0) {
@@ -1047,7 +1049,7 @@ static int check_step_fused(spdk_ctx* c, const spdk_sd_shape& s, const Variant**
         return SPDK_E_CONFIG;
     }
     const Variant* v = find_variant(c);
-    if (!v) { set_error("fused path: no tile variant for this degree/dimensionality"); return SPDK_E_CONFIG; }
+    if (!v) { set_error("fused path: no tile variant for this degree, dimensionality and slice count"); return SPDK_E_CONFIG; }
     if (s.nv != NV || s.nt != 1 || s.nx != c->n || s.ny != (c->prm.active[1] ? c->n : 1) ||
         s.nz != (c->prm.active[2] ? c->n : 1)) {
         set_error("fused: U_sp shape");
@@ -1102,7 +1104,7 @@ int spdk_fused_predict(spdk_ctx* c, double* U_sp, spdk_sd_shape s, void* ws, dou
         return SPDK_E_CONFIG;
     }
     const Variant* v = find_variant(c);
-    if (!v) { set_error("fused path: no tile variant for this degree/dimensionality"); return SPDK_E_CONFIG; }
+    if (!v) { set_error("fused path: no tile variant for this degree, dimensionality and slice count"); return SPDK_E_CONFIG; }
     if (s.nv != NV || s.nt != 1 || s.nx != c->n || s.ny != (c->prm.active[1] ? c->n : 1) ||
         s.nz != (c->prm.active[2] ? c->n : 1) || s_ader.nt != c->T || s_ader.nv < NVP || s_ader.Nx != s.Nx ||
         s_ader.Ny != s.Ny || s_ader.Nz != s.Nz || s_ader.nx != s.nx || s_ader.ny != s.ny || s_ader.nz != s.nz) {
@@ -1131,7 +1133,7 @@ static int check_flux_args(spdk_ctx* c, spdk_sd_shape s_ader, double* const F[3]
         return SPDK_E_CONFIG;
     }
     const Variant* v = find_variant(c);
-    if (!v) { set_error("fused path: no tile variant for this degree/dimensionality"); return SPDK_E_CONFIG; }
+    if (!v) { set_error("fused path: no tile variant for this degree, dimensionality and slice count"); return SPDK_E_CONFIG; }
     if (s_ader.nt != c->T || s_ader.nv < NVP || s_ader.nx != c->n || s_ader.ny != (c->prm.active[1] ? c->n : 1) ||
         s_ader.nz != (c->prm.active[2] ? c->n : 1)) {
         set_error("fused fluxes: slice shape");
@@ -1207,7 +1209,7 @@ int spdk_fused_predict_fv_fluxes(spdk_ctx* c, double* U_sp, spdk_sd_shape s, voi
 size_t spdk_fused_fluxes_workspace_bytes(spdk_ctx* c, const int N[3]) {
     const Variant* v = c ? find_variant(c) : nullptr;
     if (!v || c->T < 2) {
-        set_error("fused fluxes: no tile variant for this degree/dimensionality, or not ADER");
+        set_error("fused fluxes: no tile variant for this degree, dimensionality and slice count, or not ADER");
         return 0;
     }
     return v->slice_traces((size_t)N[0] * N[1] * N[2], c->T) * sizeof(double);

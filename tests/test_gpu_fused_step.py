@@ -84,3 +84,33 @@ def test_step(act, N, p, rk, bc, g):
         assert np.array_equal(host(Wa), host(Wb))
         assert dta == dtb
         c.close()
+
+
+@pytest.mark.parametrize("T", [2, 3, 5, 8, 10])
+def test_other_slice_counts_are_refused(T):
+    """The kernels are compiled for p+1 slices or one: every fused entry of a
+    context with another count returns its error before any launch."""
+    p, act, N = 3, (1, 1, 1), (2, 3, 2)
+    m = op.matrices(p)
+    ops = {k: m[k] for k in sk.Context.MATS}
+    ops["wt"], ops["invader"] = np.ones(T), np.ones((T, T))
+    c = sk.Context(p, act, (0, 0, 0), T, ops, h=[0.5, 0.5, 0.5])
+    L, E_CONFIG = sk.lib(), -5
+    s, sa = sd_shape(1, 6, N, p + 1, act), sd_shape(T, 6, N, p + 1, act)
+    Ne = (ctypes.c_int * 3)(s[4], s[3], s[2])
+    assert L.spdk_fused_workspace_bytes(c.ctx, Ne) == 0
+    assert L.spdk_fused_fluxes_workspace_bytes(c.ctx, Ne) == 0
+    U = torch.ones(s, dtype=torch.float64, device="cuda")
+    b = torch.zeros(64, dtype=torch.float64, device="cuda")  # any non-null address: nothing may touch it
+    u, q, ss, ssa, dt = ctypes.c_void_p(U.data_ptr()), ctypes.c_void_p(b.data_ptr()), sk.SDShape.of(s), sk.SDShape.of(sa), \
+        ctypes.c_double(1e-3)
+    fv = sk.FVShape.of((6,) + tuple(N[d] * (p + 1) + 4 for d in (2, 1, 0)))
+    faces = (ctypes.c_void_p * (3 * T))(*[b.data_ptr()] * (3 * T))
+    assert L.spdk_hydro_step_fused(c.ctx, u, ss, q, dt, None, None, None) == E_CONFIG
+    assert L.spdk_hydro_step_fused_noalloc(c.ctx, u, ss, dt, None, None, None) == E_CONFIG
+    assert L.spdk_fused_predict(c.ctx, u, ss, q, dt, q, ssa) == E_CONFIG
+    assert L.spdk_fused_predict_fluxes(c.ctx, u, ss, q, dt, q, q, q, ssa) == E_CONFIG
+    assert L.spdk_fused_predict_fv_fluxes(c.ctx, u, ss, q, dt, faces, fv, None, ssa) == E_CONFIG
+    assert L.spdk_fused_fluxes(c.ctx, q, ssa, q, q, q, q) == E_CONFIG
+    assert (host(U) == 1).all() and (host(b) == 0).all()
+    c.close()
