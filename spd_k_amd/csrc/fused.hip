@@ -750,8 +750,11 @@ Layout layout_for(size_t E, int T) {
     L.off_trA = o; o += DIM * L.tr_axis;
     L.off_trB = o; o += DIM * L.tr_axis;
     L.off_u0 = o; o += (size_t)NVP * E * G::TPE;
-    L.off_part = o; o += L.blocks + kMinBlocks;
     L.total = o;
+    // the dt minima lie over the trace buffer that the last sweep (number
+    // T - 1; even ones read buffer A) neither reads nor writes: at least 10 E
+    // doubles, where at most E minima go, and 256 more above 16384 (kMinBlocks)
+    L.off_part = T % 2 ? L.off_trB : L.off_trA;
     return L;
 }
 
