@@ -344,18 +344,39 @@ __device__ __forceinline__ void pencil(const SweepArgs& a, const double* U, size
 }
 
 // Flux divergence of variable v at solution point s (src/transforms.cpp:301-307),
-// with exact divisions: where a fast one may have been inexact.
+// whose sum `acc` of fast quotients is zero, small or NaN: formed again with
+// divisions, unless it is a zero without inexact terms.
 template <int N, int DIM>
-__device__ __forceinline__ double divergence_slow(const SweepArgs& a, const double* Fs, const double* sD, int v, int ii,
-                                                  int jj, int kk) {
+__device__ __forceinline__ double divergence_recheck(const SweepArgs& a, const double* Fs, const double* sD, int v,
+                                                     int ii, int jj, int kk, double acc) {
     using G = Tile<N, DIM>;
     constexpr int M = G::M, NT = G::NT;
-    double acc = 0;
+    auto fx = [&](int l) { return Fs[v * G::FSZ + fidx(0, l, DIM == 3 ? kk * N + jj : jj, N, NT, M)]; };
+    auto fy = [&](int l) { return Fs[(NVP + v) * G::FSZ + fidx(1, l, DIM == 3 ? kk * N + ii : ii, N, NT, M)]; };
+    auto fz = [&](int l) { return Fs[(2 * NVP + v) * G::FSZ + fidx(2, l, jj * N + ii, N, NT, M)]; };
+    bool redo = acc != 0.0;  // NaN: true
+    if (!redo) {
+        AnyBits any;
+#pragma unroll
+        for (int l = 0; l < M; l++) {
+            any.add(fx(l));
+            if (DIM >= 2) any.add(fy(l));
+            if (DIM == 3) any.add(fz(l));
+        }
+#pragma unroll 1
+        for (int l = 0; l < M && any.b; l++) {
+            redo |= div_small(fx(l) * sD[ii * M + l]);
+            if (DIM >= 2) redo |= div_small(fy(l) * sD[jj * M + l]);
+            if (DIM == 3) redo |= div_small(fz(l) * sD[kk * M + l]);
+        }
+    }
+    if (!redo) return acc;
+    acc = 0;
 #pragma unroll 1
     for (int l = 0; l < M; l++) {
-        acc += Fs[v * G::FSZ + fidx(0, l, DIM == 3 ? kk * N + jj : jj, N, NT, M)] * sD[ii * M + l] / a.h[0];
-        if (DIM >= 2) acc += Fs[(NVP + v) * G::FSZ + fidx(1, l, DIM == 3 ? kk * N + ii : ii, N, NT, M)] * sD[jj * M + l] / a.h[1];
-        if (DIM == 3) acc += Fs[(2 * NVP + v) * G::FSZ + fidx(2, l, jj * N + ii, N, NT, M)] * sD[kk * M + l] / a.h[2];
+        acc += fx(l) * sD[ii * M + l] / a.h[0];
+        if (DIM >= 2) acc += fy(l) * sD[jj * M + l] / a.h[1];
+        if (DIM == 3) acc += fz(l) * sD[kk * M + l] / a.h[2];
     }
     return acc;
 }
@@ -450,21 +471,28 @@ __global__ void __launch_bounds__(256, MODE == FACES ? 3 : SPDK_SWEEP_WAVES) k_s
 #pragma unroll
         for (int v = 0; v < NVP; v++) {
             double acc = 0;
+            AnyBits any;
             const double* Fx = Fs + v * G::FSZ;
             const double* Fy = Fs + (NVP + v) * G::FSZ;
             const double* Fz = Fs + (2 * NVP + v) * G::FSZ;
+            auto flux = [&](double f) {
+                if (v > DIM && v < 4) any.add(f);  // momentum along an inactive axis: zero in most flows
+                return f;
+            };
 #pragma unroll
             for (int l = 0; l < M; l++) {
-                acc += div_fast(Fx[fidx(0, l, qx, N, NT, M)] * sD[ii * M + l], a.dh[0]);
-                if (DIM >= 2) acc += div_fast(Fy[fidx(1, l, qy, N, NT, M)] * sD[jj * M + l], a.dh[1]);
-                if (DIM == 3) acc += div_fast(Fz[fidx(2, l, qz, N, NT, M)] * sD[kk * M + l], a.dh[2]);
+                acc += div_fast(flux(Fx[fidx(0, l, qx, N, NT, M)]) * sD[ii * M + l], a.dh[0]);
+                if (DIM >= 2) acc += div_fast(flux(Fy[fidx(1, l, qy, N, NT, M)]) * sD[jj * M + l], a.dh[1]);
+                if (DIM == 3) acc += div_fast(flux(Fz[fidx(2, l, qz, N, NT, M)]) * sD[kk * M + l], a.dh[2]);
             }
             dudt[v] = acc;
-            recheck = recheck || div_recheck(acc);
+            if (v > DIM && v < 4) recheck = recheck || (sum_recheck(acc) && (any.b || acc != 0.0));
+            else recheck = recheck || sum_recheck(acc);
         }
         if (recheck)
 #pragma unroll
-            for (int v = 0; v < NVP; v++) dudt[v] = divergence_slow<N, DIM>(a, Fs, sD, v, ii, jj, kk);
+            for (int v = 0; v < NVP; v++)
+                if (sum_recheck(dudt[v])) dudt[v] = divergence_recheck<N, DIM>(a, Fs, sD, v, ii, jj, kk, dudt[v]);
         if (a.grav && MODE == CORRECT) {
             // update_solution's gravity source (src/transforms.cpp:17-27,
             // :364-367) from the ADER slice: rho g and m . g

@@ -829,7 +829,7 @@ __device__ __forceinline__ Sed sed_slopes(double wm2, double wm1, double u, doub
     auto div = [&](double x, const ConstDiv& c) -> double {
         if (EXACT) return x / c.h;
         const double q = div_fast(x, c);
-        recheck = recheck || div_recheck(q);
+        recheck = recheck || div_recheck(x, q);
         return q;
     };
     Sed r;
@@ -1366,8 +1366,9 @@ __device__ __forceinline__ void recon(P W, size_t pl, const int (&st)[3], const 
         bool recheck = false;
 #pragma unroll
         for (int v = 0; v < NVP; v++) {
-            const double SL = div_fast(W[v * pl + st[d]] - r.w[v], cu), SR = div_fast(r.w[v] - W[(long)(v * pl) - st[d]], cd);
-            recheck = recheck || div_recheck(SL) || div_recheck(SR);
+            const double xL = W[v * pl + st[d]] - r.w[v], xR = r.w[v] - W[(long)(v * pl) - st[d]];
+            const double SL = div_fast(xL, cu), SR = div_fast(xR, cd);
+            recheck = recheck || div_recheck(xL, SL) || div_recheck(xR, SR);
             r.dw[d][v] = minmod(SL, SR, df);
         }
         if (recheck)
@@ -1389,8 +1390,9 @@ __device__ __forceinline__ void hancock(const Recon& r, const Geo& g, int k, int
     bool recheck = false;
 #pragma unroll
     for (int v = 0; v < NVP; v++) {
-        hs[v] = div_fast(r.dwt[v] * dt, h);
-        recheck = recheck || div_recheck(hs[v]);
+        const double x = r.dwt[v] * dt;
+        hs[v] = div_fast(x, h);
+        recheck = recheck || div_recheck(x, hs[v]);
     }
     if (recheck)
 #pragma unroll

@@ -37,6 +37,7 @@
 // carries never reach B.
 #include <hip/hip_runtime.h>
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <type_traits>
 #include "ctx.hpp"
@@ -260,6 +261,7 @@ __global__ void __launch_bounds__((Tile<N, D, T, R>::THREADS)) k_isweep(IArgs a)
     __shared__ R sE[EPB * T * G::EP];  // face-solved E (element, slice, point), then the predictor slices
     __shared__ R sS2F[M * N];
     __shared__ double sDm[N * M], sInv[T * T], sW[T];
+    __shared__ int sLow[TH / 64];
     __shared__ Acc sDmH[PLAIN ? 1 : D][PLAIN ? 1 : N * M];  // dfp_to_sp / h_axis
     __shared__ float sP[PLAIN ? 1 : T * T];                  // invader * w * dt
     // workgroups go to the 8 XCDs in turn; XCD x takes the x-th contiguous
@@ -288,6 +290,7 @@ __global__ void __launch_bounds__((Tile<N, D, T, R>::THREADS)) k_isweep(IArgs a)
     for (int c = 0; c < D; c++) any_mean = any_mean || dir[c] == 0;
 
     // A. face-solved E of every slice
+    int low = 0;  // smallest binary exponent of a nonzero value
     for_each_component([&](auto comp) {
         constexpr int e = comp.value, EPT = G::epts(e);
         if (tid >= ne * EPT) return;
@@ -321,9 +324,17 @@ __global__ void __launch_bounds__((Tile<N, D, T, R>::THREADS)) k_isweep(IArgs a)
                                         : edge_solved<e, D, false, Slices<R, T>>(lo, hi, dir, face, raw);
 #pragma unroll
         for (int t = 0; t < T; t++)
-            if (t < tin) sE[(q * T + t) * G::EP + G::eoff(e) + p] = v.v[t];
+            if (t < tin) {
+                sE[(q * T + t) * G::EP + G::eoff(e) + p] = v.v[t];
+                if (PLAIN) low = min(low, __builtin_amdgcn_frexp_exp((double)v.v[t]));
+            }
     });
+    // a zero sum may hold inexact quotients (div_small) only with such an edge value: matrix entries are zero or at
+    // least 2^-200 (step())
+    if (PLAIN) sLow[tid / 64] = __ballot(low <= -700) != 0;
     __syncthreads();
+
+    const bool small = PLAIN && (sLow[0] | sLow[1] | sLow[2] | sLow[3] | sLow[TH / 64 - 1]);
 
     // B. dB/dt of every slice at the thread's face-B points
     Acc dBdt[3][T];
@@ -366,7 +377,7 @@ __global__ void __launch_bounds__((Tile<N, D, T, R>::THREADS)) k_isweep(IArgs a)
                     dB -= PLAIN ? (Acc)div_fast((double)x, a.dh[a1]) : x;
                 }
             }
-            if (PLAIN && div_recheck((double)dB)) {
+            if (PLAIN && sum_recheck((double)dB) && (dB != 0 || small)) {
                 dB = 0;
 #pragma unroll 1
                 for (int l = 0; l < M; l++) {
@@ -552,6 +563,10 @@ int step(spdk_ctx* c, double* Bx, spdk_sd_shape sx, double* By, spdk_sd_shape sy
         if (a.n[d] < 1) { set_error("fused induction: axis needs ghost elements"); return SPDK_E_SHAPE; }
         nel *= (size_t)a.n[d];
     }
+    // see k_isweep: with smaller matrix entries every quotient is formed by division
+    for (double x : c->mat_host[SPDK_M_DFP_TO_SP])
+        if (x != 0.0 && std::fabs(x) < 0x1p-200)
+            for (int d = 0; d < 3; d++) a.dh[d].z = __builtin_nan("");
     if (nel >= (1ull << 31)) { set_error("fused induction: too many elements"); return SPDK_E_SHAPE; }
     a.nel = (int)nel;
     std::strncpy(c->kernel_name, "k_isweep", sizeof(c->kernel_name) - 1);

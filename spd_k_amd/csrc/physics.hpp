@@ -6,6 +6,7 @@
 // reference arithmetic.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <cstdint>
 
 namespace spdk {
 
@@ -23,23 +24,41 @@ __host__ __device__ __forceinline__ double smin(double a, double b) { return (b 
 // fused multiply-adds, is x / h rounded to nearest, the bits of the division
 // (Markstein 1990; Brisebarre, Muller, Raina 2004), in 3 instructions instead
 // of the 11 of the general division. It holds while no step leaves the normal
-// range: div_recheck(s) is true for a sum s of such quotients that may hold an
-// inexact one (a term below 2^-969 can only matter to a sum that small; an
-// infinite or NaN term makes the sum NaN), which the caller then forms again
-// with divisions. h must be positive, finite and well inside the normal
-// range; otherwise z is NaN and every sum is formed again.
+// range, which is sure for numerators of at least 2^-900 (h is within 2^-64 and
+// 2^64; otherwise z is NaN, and so is every quotient), for zero, and for
+// quotients of at least 2^-900. The others are formed again by division:
+//   - div_recheck(x, q): the quotient q of x may be inexact;
+//   - sum_recheck(s): the sum s of quotients may hold an inexact one. Where s is
+//     zero, div_small(x) of its numerators tells; in a flow's zero sums they are
+//     mostly zeros all, which AnyBits of their factors shows first. An inexact
+//     quotient is less than 2^-905 and off by less than 2^-957: a sum of at
+//     least 2^-800 could show that only if partial sums lay that close to a tie,
+//     one after the other.
+// An infinite or NaN numerator makes the quotient and every sum of it NaN.
 struct ConstDiv {
     double h, z;
 };
 __host__ inline ConstDiv const_div(double h) {
-    const bool ok = h > 0x1p-100 && h < 0x1p100;
+    const bool ok = h > 0x1p-64 && h < 0x1p64;
     return {h, ok ? 1.0 / h : __builtin_nan("")};
 }
 __device__ __forceinline__ double div_fast(double x, const ConstDiv& c) {
     const double q = x * c.z;
     return __builtin_fma(-__builtin_fma(q, c.h, -x), c.z, q);
 }
-__device__ __forceinline__ bool div_recheck(double s) { return s != 0.0 && !(fabs(s) >= 0x1p-900); }
+__device__ __forceinline__ bool div_recheck(double x, double q) {
+    return !(fabs(q) >= 0x1p-900) && fabs(x) + fabs(q) != 0.0;
+}
+__device__ __forceinline__ bool sum_recheck(double s) { return !(fabs(s) >= 0x1p-800); }
+__device__ __forceinline__ bool div_small(double x) { return x != 0.0 && fabs(x) < 0x1p-900; }
+// OR of values' bits but the signs: zero while all were zeros
+struct AnyBits {
+    uint32_t b = 0;
+    __device__ __forceinline__ void add(double x) {
+        const uint64_t u = __builtin_bit_cast(uint64_t, x);
+        b |= (uint32_t)u | (uint32_t)(u >> 32) << 1;
+    }
+};
 
 // Barrier between phases that touch only an element's own LDS area, where an
 // element lies in one wave, so the wave's own order is enough: a wave's LDS

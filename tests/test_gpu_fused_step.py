@@ -86,6 +86,36 @@ def test_step(act, N, p, rk, bc, g):
         c.close()
 
 
+@pytest.mark.parametrize("act,N,p", [((1, 0, 0), (23, 1, 1), 3), ((1, 1, 0), (6, 7, 1), 2), ((1, 1, 1), (3, 2, 2), 3)])
+@pytest.mark.parametrize("rk", [0, 1])
+def test_step_subnormal_on_wide_elements(act, N, p, rk):
+    """A momentum of a few units of 2^-1074 on elements wider than 1, and a state that is constant elsewhere: sums that
+    are zero, with and without terms whose quotients are inexact."""
+    rng = np.random.default_rng(70 + p + sum(act))
+    m = op.matrices(p)
+    ops = {k: m[k] for k in sk.Context.MATS}
+    ops["wt"] = m["wt"] if rk == 0 else np.ones(1)
+    if rk:
+        ops["invader"] = np.ones((1, 1))
+    T = p + 1 if rk == 0 else 1
+    c = sk.Context(p, act, (0, 0, 0), T, ops, h=[1.9, 1.3, 1.7], rk_order=rk)
+    U = np.zeros(sd_shape(1, 6, N, p + 1, act))
+    U[0, 0], U[0, 4], U[0, 1] = 1.0, 2.5, 1.0
+    U[0, 3] = rng.integers(-8, 9, size=U[0, 3].shape) * 5e-324
+    U[0, 2, ..., : U.shape[4] // 2, :, :, :] = 0.25  # and velocity along y in half of the elements along x
+    a, b = dev(U), dev(U)
+    Wb = torch.full(U.shape, float("nan"), dtype=torch.float64, device="cuda")
+    shapes = [sd_shape(T, 6, N, p + 1, act, stag=d) for d in range(3)]
+    Wa, dta = stages(c, a, p, T, act, shapes, 1.0, rk)
+    dtb = c.hydro_step_fused(b, 1.0, Wb)
+    x, y = host(a), host(b)
+    assert np.isfinite(x).all() and (x[0, 3] != U[0, 3]).any()
+    assert np.array_equal(x, y), f"U: {int((x != y).sum())} of {x.size} differ"
+    assert np.array_equal(host(Wa), host(Wb))
+    assert dta == dtb
+    c.close()
+
+
 @pytest.mark.parametrize("T", [2, 3, 5, 8, 10])
 def test_other_slice_counts_are_refused(T):
     """The kernels are compiled for p+1 slices or one: every fused entry of a

@@ -118,3 +118,65 @@ def test_fallback(act, N, nonfinite):
             ok = (got == Fo[d]) | (np.isnan(got) & np.isnan(Fo[d])) | skip
             assert ok.all(), (d, int((~ok).sum()))
     c.close()
+
+
+def wide(act, N, seed):
+    """As setup, on cells 1.9 wide, with a field that grows by 4 or no units of 2^-1074 from cell to cell."""
+    p, faces, centers = 3, [], []
+    for d in range(3):
+        f = 1.9 * np.arange(4 * N[d] + 5) if act[d] else np.array([-1.0, 0.0])
+        faces.append(f)
+        centers.append(0.5 * (f[1:] + f[:-1]) if act[d] else np.array([-1.0]))
+    m = op.matrices(p)
+    ops = {k: m[k] for k in sk.Context.MATS}
+    ops["wt"], ops["fv_faces"], ops["fv_centers"] = m["wt"], faces, centers
+    c = sk.Context(p, act, (0, 0, 0), p + 1, ops, h=[7.6] * 3)
+    geo = ((ctypes.POINTER(ctypes.c_double) * 3)(*[op.dp(x) for x in centers]),
+           (ctypes.POINTER(ctypes.c_double) * 3)(*[op.dp(x) for x in faces]),
+           (ctypes.c_int * 3)(*[len(x) for x in centers]))
+    rng, s_fv = np.random.default_rng(seed), fv_shape(6, N, 4, act)
+    W = np.zeros(s_fv)
+    W[0], W[4], W[1] = 1.0, 2.5, 1.0
+    for d in range(3):
+        if act[d]:
+            step = 4 * rng.integers(0, 2, size=s_fv[3 - d])
+            W[3] += np.cumsum(step).reshape([-1 if a == 2 - d else 1 for a in range(3)]) * 5e-324
+    return c, op.OrcCfg.make(act=act, p=p), geo, (faces, centers), s_fv, W, rng
+
+
+@pytest.mark.parametrize("act,N", MESHES)
+def test_detection_subnormal_on_wide_cells(act, N):
+    c, cfg, geo, _keep, s_fv, Wn, rng = wide(act, N, 23)
+    Wo = Wn.copy()
+    Wo[3] = rng.integers(0, 7, size=s_fv[1:]) * 5e-324
+    tr_o, al = np.zeros(s_fv), [np.zeros(s_fv) for _ in range(3)]
+    op.orc().orc_detect(ctypes.byref(cfg), op.dp(Wn), op.dp(Wo), op.dp(tr_o), *[op.dp(a) for a in al], op.ip(s_fv),
+                        *geo, 1, 0b01000)
+    z = lambda: torch.zeros(s_fv, dtype=torch.float64, device="cuda")
+    tr, ga = z(), [z() for _ in range(3)]
+    c.detect_troubles(dev(Wn), dev(Wo), tr, *ga, 1, 0b01000)
+    for d in range(3):
+        if act[d]:
+            assert same(host(ga[d]), al[d]), d
+    assert same(host(tr), tr_o)
+    tr, bits = z(), torch.zeros(s_fv[1:], dtype=torch.int16, device="cuda")
+    c.detect_troubles_bits(dev(Wn), dev(Wo), tr, bits, 1, 0b01000)
+    assert same(host(tr), tr_o)
+    c.close()
+
+
+@pytest.mark.parametrize("act,N", MESHES + [((1, 0, 1), (9, 1, 5))])  # the last: one thread per cell
+def test_fallback_subnormal_on_wide_cells(act, N):
+    c, cfg, geo, _keep, s_fv, W, rng = wide(act, N, 29)
+    th = np.ones((1,) + s_fv[1:])
+    Fs = [np.zeros(fv_shape(6, N, 4, act, stag=d)) for d in range(3)]
+    Fo = [f.copy() for f in Fs]
+    op.orc().orc_fallback(ctypes.byref(cfg), op.dp(W), op.dp(th), *[op.dp(f) for f in Fo], op.ip(s_fv), *geo,
+                          ctypes.c_double(0.5))
+    Fg = [dev(f) for f in Fs]
+    c.fallback_fluxes(dev(W), dev(th), Fg[0], Fg[1] if act[1] else None, Fg[2] if act[2] else None, 0.5)
+    assert (Fo[0][3] != 0).any()
+    for d in range(3):
+        if act[d]:
+            assert same(host(Fg[d]), Fo[d]), d
+    c.close()

@@ -60,12 +60,12 @@ CASES = [(dim, p, N, v, bc)
 
 
 @pytest.mark.parametrize("dim,p,N,v,bc", CASES)
-def test_fused_step_equals_the_stages(dim, p, N, v, bc):
+def test_fused_step_equals_the_stages(dim, p, N, v, bc, wide=False):
     act = [d < dim for d in range(3)]
     m = op.matrices(p)
     ops = {k: m[k] for k in sk.Context.MATS}
     ops["wt"] = m["wt"]
-    h = [1.3 / (N[d] + 2) if act[d] else 1.0 for d in range(3)]
+    h = [1.9, 1.3, 1.7] if wide else [1.3 / (N[d] + 2) if act[d] else 1.0 for d in range(3)]
     stream = torch.cuda.Stream()
     with torch.cuda.stream(stream):
         c = sk.Context(p, act, bc, p + 1, ops, h=h, vel=v)
@@ -83,9 +83,11 @@ def test_fused_step_equals_the_stages(dim, p, N, v, bc):
         B0[0][..., 0] = 0.0  # exact zeros of either sign, and values near the smallest normal ones
         B0[1][..., 0] = -0.0
         B0[2][...] *= 1e-290
+        if wide:
+            B0 = [rng.integers(-2 ** (d + 1), 2 ** (d + 1) + 1, size=s) * 5e-324 for d, s in enumerate(sB)]
         a, b = [dev(x) for x in B0], [dev(x) for x in B0]
         E = [torch.zeros(s, dtype=torch.float64, device="cuda") for s in sE]
-        dt = 0.01
+        dt = 8.0 if wide else 0.01
         stage_step(c, p, a, sB, E, sE, dt, h, act)
         L = sk.lib()
         cnt = (ctypes.c_int * 3)(*Ne)
@@ -100,3 +102,10 @@ def test_fused_step_equals_the_stages(dim, p, N, v, bc):
             assert np.isfinite(x).all()
             assert np.array_equal(x, y), f"B{'xyz'[d]}: {int((x != y).sum())} of {x.size} differ"
         c.close()
+
+
+@pytest.mark.parametrize("dim,p,N", [(2, 3, (11, 3, 1)), (3, 3, (4, 3, 2))])
+@pytest.mark.parametrize("v", [(1.0, 0.5, 0.25), (0.0, -0.7, -1.0)])
+def test_subnormal_on_wide_elements(dim, p, N, v):
+    """A field of a few units of 2^-1074 on elements wider than 1: sums that are zero though their terms are not."""
+    test_fused_step_equals_the_stages(dim, p, N, v, (0, 0, 0), wide=True)

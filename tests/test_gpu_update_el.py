@@ -63,3 +63,41 @@ def test_update(act, N, p, g, values):
         c.update_solution(U_g, dev(Ua), Fg[0], Fg[1], Fg[2], p + 2, dt)
         assert np.array_equal(host(U_g), U_o, equal_nan=True)
     c.close()
+
+
+@pytest.mark.parametrize("act,N,p", [((1, 0, 0), (37, 1, 1), 3), ((1, 1, 0), (5, 3, 1), 3), ((1, 1, 1), (3, 2, 2), 3),
+                                     ((1, 1, 1), (2, 1, 1), 7)])
+def test_update_subnormal_on_wide_elements(act, N, p):
+    """Fluxes of a few units of 2^-1074 on elements wider than 1, where a quotient
+    formed without division can be zero though its numerator is not."""
+    rng = np.random.default_rng(40 + p + sum(act))
+    m = op.matrices(p)
+    ops = {k: m[k] for k in sk.Context.MATS}
+    ops["wt"] = m["wt"]
+    h = np.array([1.9, 1.3, 1.7])
+    c = sk.Context(p, act, (0, 0, 0), p + 1, ops, h=h)
+    n, T = p + 1, p + 1
+    s_a, s_u = sd_shape(T, 6, N, n, act), sd_shape(1, 6, N, n, act)
+    U, Ua = np.zeros(s_u), np.zeros(s_a)
+    F = [np.zeros(sd_shape(T, 6, N, n, act, stag=d)) for d in range(3)]
+    for d in range(3):
+        if act[d]:  # variable v: up to 2^v units
+            for v in range(6):
+                F[d][:, v] = rng.integers(-2 ** v, 2 ** v + 1, size=F[d][:, v].shape) * 5e-324
+    cfg = op.OrcCfg.make(act=act)
+    shapes, dt = [op.ip(f.shape) for f in F], 50.0
+    Fg = [dev(f) if act[d] else None for d, f in enumerate(F)]
+    Ua_o, U_o = Ua.copy(), U.copy()
+    op.orc().orc_predict(ctypes.byref(cfg), op.dp(U), op.ip(s_u), op.dp(Ua_o), op.ip(s_a), op.dp(F[0]), shapes[0],
+                         op.dp(F[1]), shapes[1], op.dp(F[2]), shapes[2], op.dp(m["dfp_to_sp"]), n, n + 1,
+                         op.dp(m["invader"]), op.dp(m["wt"]), op.dp(h), ctypes.c_double(dt))
+    op.orc().orc_correct(ctypes.byref(cfg), op.dp(U_o), op.ip(s_u), op.dp(Ua), op.ip(s_a), op.dp(F[0]), shapes[0],
+                         op.dp(F[1]), shapes[1], op.dp(F[2]), shapes[2], op.dp(m["dfp_to_sp"]), n, n + 1,
+                         op.dp(m["wt"]), op.dp(h), ctypes.c_double(dt))
+    assert (U_o != 0).mean() > 0.5
+    Ua_g, U_g = dev(Ua), dev(U)
+    c.update_prediction(dev(U), Ua_g, Fg[0], Fg[1], Fg[2], p + 2, dt)
+    c.update_solution(U_g, dev(Ua), Fg[0], Fg[1], Fg[2], p + 2, dt)
+    assert np.array_equal(host(Ua_g), Ua_o)
+    assert np.array_equal(host(U_g), U_o)
+    c.close()
