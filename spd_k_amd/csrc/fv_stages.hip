@@ -1659,14 +1659,16 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(SPDK_FB
 }
 
 // ===========================================================================
+// An axis without arrays of its own takes axis 0's.
 static Geo geo_of(spdk_ctx* c) {
     Geo g;
     for (int d = 0; d < 3; d++) {
-        g.f[d] = c->fvf[d] ? c->fvf[d] : c->fvf[0];
-        g.c[d] = c->fvc[d] ? c->fvc[d] : c->fvc[0];
-        g.dc1[d] = c->fvdc1[d];
-        g.dc2[d] = c->fvdc2[d];
-        g.df[d] = c->fvdf[d];
+        const int df = c->fvf[d] ? d : 0, dc = c->fvc[d] ? d : 0;
+        g.f[d] = c->fvf[df];
+        g.c[d] = c->fvc[dc];
+        g.dc1[d] = c->fvdc1[dc];
+        g.dc2[d] = c->fvdc2[dc];
+        g.df[d] = c->fvdf[df];
     }
     return g;
 }

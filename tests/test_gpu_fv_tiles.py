@@ -180,3 +180,34 @@ def test_fallback_subnormal_on_wide_cells(act, N):
         if act[d]:
             assert same(host(Fg[d]), Fo[d]), d
     c.close()
+
+
+@pytest.mark.parametrize("act", [(1, 1, 0), (1, 1, 1)])
+def test_axes_without_coordinates_take_those_of_x(act):
+    """A context given the FV coordinates of x alone, on a mesh of equal axes, against one given every axis'."""
+    N, p, m = [5 if a else 1 for a in act], 3, op.matrices(3)
+    xs = [op.fv_geometry(5, p) if a else (np.array([-1.0, 0.0]), np.array([-1.0])) for a in act]
+    s_fv, rng = fv_shape(6, N, 4, act), np.random.default_rng(31)
+    W = state((1,) + s_fv, rng)[0]
+    Wo = np.ascontiguousarray(W * (1 + 1e-2 * rng.normal(size=W.shape)))
+    th = rng.choice([0.0, 0.25, 1.0], size=(1,) + s_fv[1:])
+    Fs = [rng.normal(size=fv_shape(6, N, 4, act, stag=d)) for d in range(3)]
+    out = []
+    for own in (True, False):
+        ops = {k: m[k] for k in sk.Context.MATS}
+        ops["wt"] = m["wt"]
+        ops["fv_faces"], ops["fv_centers"] = [[x[q] if own or d == 0 else None for d, x in enumerate(xs)] for q in (0, 1)]
+        c = sk.Context(p, act, (0, 0, 0), p + 1, ops, h=[0.2] * 3)
+        z = lambda: torch.zeros(s_fv, dtype=torch.float64, device="cuda")
+        tr, al, tb = z(), [z() for _ in range(3)], z()
+        bits = torch.zeros(s_fv[1:], dtype=torch.int16, device="cuda")
+        F = [dev(f) if a else None for a, f in zip(act, Fs)]
+        torch.cuda.synchronize()
+        c.detect_troubles(dev(W), dev(Wo), tr, *al, 1, 0b10001)
+        c.detect_troubles_bits(dev(W), dev(Wo), tb, bits, 1, 0b10001)
+        c.fallback_fluxes(dev(W), dev(th), *F, 1e-3)
+        out.append([host(x) for x in [tr, tb, bits] + al + [f for f in F if f is not None]])
+        c.close()
+    assert out[0][0].any()
+    for a, b in zip(*out):
+        assert same(a, b)
