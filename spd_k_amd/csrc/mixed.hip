@@ -125,11 +125,7 @@ struct MArgs {
     const float* d_old;     // (5,E,TPE) U_sp - mu
     float* D;               // (T,5,E,TPE) predictor state, read and rewritten in place
     float* trb[2][3];       // two trace buffers per axis, (5,2,E,slices,NT) (see trace_at)
-    // (2,E): sweep number of each element's last write to each buffer. Read with
-    // cload although the sweep writes it: the value that replaces an entry, the
-    // current sweep's number, leads every reader to the same buffer as the
-    // entry it replaces
-    int* ver;
+    int* ver;               // (2,E): sweep number of each element's last write to each buffer (see versions_hold)
     int cur;                // this sweep's number
     const unsigned char* big_in;  // per element: r_e >= tol in the previous sweep (null: every element active)
     const int* blist;       // blocks to run (grid = its length; null: every block)
@@ -319,15 +315,23 @@ __device__ __forceinline__ size_t trace_at(size_t E, int ns, int v, int sd, size
     return (((size_t)(v * 2 + sd) * E + e) * ns + t) * NT + q;
 }
 
-// Trace buffer of axis d holding element el's newest traces written before
-// this sweep.
-__device__ __forceinline__ const float* read_buffer(const MArgs& a, int d, size_t el) {
-    const int v0 = cload(a.ver, el), v1 = cload(a.ver, (size_t)a.E + el);
-    const int b = (v1 < a.cur && (v1 > v0 || v0 >= a.cur)) ? 1 : 0;
-    const float* t0 = d == 0 ? a.trb[0][0] : (d == 1 ? a.trb[0][1] : a.trb[0][2]);
-    const float* t1 = d == 0 ? a.trb[1][0] : (d == 1 ? a.trb[1][1] : a.trb[1][2]);
-    return b ? t1 : t0;
+// The buffer holding an element's newest traces from before sweep cur, given
+// its two versions, and the one it writes in a sweep: the older.
+__host__ __device__ constexpr int newest(int v0, int v1, int cur) { return v1 < cur && (v1 > v0 || v0 >= cur) ? 1 : 0; }
+__host__ __device__ constexpr int older(int v0, int v1) { return v1 < v0 ? 1 : 0; }
+// An element writes its older buffer and then puts the current sweep's number
+// in place of that version. A reader must find the same buffer whether it sees
+// the version from before or after, and never the one that is being written.
+constexpr bool versions_hold() {
+    for (int cur = 1; cur < 8; cur++)
+        for (int v0 = -1; v0 < cur; v0++)
+            for (int v1 = -1; v1 < cur; v1++) {
+                const int b = newest(v0, v1, cur), w = older(v0, v1);
+                if (v0 != v1 && (b == w || newest(w ? v0 : cur, w ? cur : v1, cur) != b)) return false;
+            }
+    return true;
 }
+static_assert(versions_hold(), "readers and the writer of a sweep agree on the trace buffers");
 
 // Elements whose traces element e reads across its two faces along axis d
 // (ghost fills: periodic copies the opposite interior element, gradfree /
@@ -343,18 +347,48 @@ __device__ __forceinline__ void face_sources(const MArgs& a, int d, int ei, int 
     el1 = ebase + (size_t)(ed >= Nd - 2 ? (per ? 1 : Nd - 2) : ed + 1) * stride;
 }
 
+// Buffers of element e's traces in this sweep, one bit each: bit 2 d + i that
+// which holds the newest of its i-th source along axis d, bit 6 that which it
+// writes. The sweep that reads the versions also writes them (each workgroup
+// its own elements'), hence atomic accesses; all are loaded before the first
+// is looked at, and before the element's state (a wait for a load is a wait
+// for every earlier one, and for every earlier store). UNI: e is the same in
+// every lane, and the bits go to a scalar register.
+template <int DIM, bool UNI>
+__device__ __forceinline__ int trace_buffers(const MArgs& a, int ei, int ej, int ek, size_t e) {
+    int v[2 * DIM + 1][2];
+    auto load = [&](int i, size_t el) {
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+            v[i][b] = __hip_atomic_load(a.ver + b * (size_t)a.E + el, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+#pragma unroll
+    for (int d = 0; d < DIM; d++) {
+        size_t el0, el1;
+        face_sources(a, d, ei, ej, ek, e, el0, el1);
+        load(2 * d, el0);
+        load(2 * d + 1, el1);
+    }
+    load(2 * DIM, e);
+    int bits = older(v[2 * DIM][0], v[2 * DIM][1]) << 6;
+#pragma unroll
+    for (int i = 0; i < 2 * DIM; i++) bits |= newest(v[i][0], v[i][1], a.cur) << i;
+    return UNI ? __builtin_amdgcn_readfirstlane(bits) : bits;
+}
+
 // Traces a pencil reads across its two faces: v0 is the value left of face 0
 // (or the ghost fill that replaces the own value at face M-1 of the left
 // ghost), v1 the value right of face M-1 (or the ghost fill at face 0 of the
 // right ghost), normal frame, without the neighbours' means.
 struct Nbr { float v0[NVP], v1[NVP]; };
 
-// Loads the traces pencil (d, slice ts of ns, q) of element e reads. Ghost fills: periodic
+// Loads the traces pencil (d, slice ts of ns, q) of element e reads, from the
+// buffers bufs (trace_buffers). Ghost fills: periodic
 // copies the opposite interior element, gradfree / reflective the adjacent one
 // (src/boundary.cpp:48-113). lower_face_only: v1 only where the lower face
 // takes it (the right ghost).
 template <int N, int DIM>
-__device__ __forceinline__ Nbr load_traces(const MArgs& a, int d, int ns, int ts, int q, int ei, int ej, int ek,
+__device__ __forceinline__ Nbr load_traces(const MArgs& a, int bufs, int d, int ns, int ts, int q, int ei, int ej, int ek,
                                            size_t e, bool lower_face_only = false) {
     constexpr int NT = MT<N, DIM>::NT;
     const int ed = d == 0 ? ei : (d == 1 ? ej : ek);
@@ -364,8 +398,10 @@ __device__ __forceinline__ Nbr load_traces(const MArgs& a, int d, int ns, int ts
     face_sources(a, d, ei, ej, ek, e, el0, el1);
     const int sid0 = ed <= 1 ? (per ? 1 : 0) : 1;
     const int sid1 = ed >= Nd - 2 ? (per ? 0 : 1) : 0;
-    const float* t0 = read_buffer(a, d, el0);
-    const float* t1 = read_buffer(a, d, el1);
+    const float* bA = d == 0 ? a.trb[0][0] : (d == 1 ? a.trb[0][1] : a.trb[0][2]);
+    const float* bB = d == 0 ? a.trb[1][0] : (d == 1 ? a.trb[1][1] : a.trb[1][2]);
+    const float* t0 = (bufs >> (2 * d)) & 1 ? bB : bA;
+    const float* t1 = (bufs >> (2 * d + 1)) & 1 ? bB : bA;
     Nbr n;
 #pragma unroll
     for (int v = 0; v < NVP; v++) {
@@ -961,6 +997,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE >
         }
     }
 
+    // The first sweep reads the step start's traces (buffer A, version 0) and writes B.
+    int bufs = 1 << 6;
+    if (MODE != M_START && act_e) bufs = trace_buffers<DIM, TPE == 64>(a, ei, ej, ek, (size_t)e);
+
     // The loads of the element's state and of the first axis' traces go out
     // together; the mean state is prepared while they are in flight.
     float dold[NVP], din[TS][NVP];
@@ -977,8 +1017,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE >
     // the face integrals read faces 0..M-2 only, unless the x flux points are written as well
     const bool lower = MODE == M_STAGED || (MODE == M_FACES && !a.F_x);
     Nbr nb;
-    if (MODE != M_START && act_e) nb = load_traces<N, DIM>(a, 0, a.tin_slices, ts, q, ei, ej, ek, (size_t)e, lower);
-    if (MODE == M_START && act_e && s < DIM * NT) nb = load_traces<N, DIM>(a, s / NT, 1, 0, q, ei, ej, ek, (size_t)e);
+    if (MODE != M_START && act_e) nb = load_traces<N, DIM>(a, bufs, 0, a.tin_slices, ts, q, ei, ej, ek, (size_t)e, lower);
+    if (MODE == M_START && act_e && s < DIM * NT) nb = load_traces<N, DIM>(a, bufs, s / NT, 1, 0, q, ei, ej, ek, (size_t)e);
 
     if (live)
         for (int v = s; v < NVP; v += TPE) X[v] = cload(a.mu, (size_t)v * E + e);
@@ -1026,7 +1066,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE >
         if (act_e)
             for (int task = s; task < DIM * NT; task += TPE) {  // more than TPE only for p = 1 in 3-D
                 const int d = task / NT, qq = task % NT;
-                if (task != s) nb = load_traces<N, DIM>(a, d, 1, 0, qq, ei, ej, ek, (size_t)e);
+                if (task != s) nb = load_traces<N, DIM>(a, bufs, d, 1, 0, qq, ei, ej, ek, (size_t)e);
                 pencil<N, DIM>(a, nb, Ds, Fs + d * NVP * FSZ, X, d, qq, ei, ej, ek, (size_t)e, false, bal, 0.0);
             }
         elem_sync();
@@ -1051,7 +1091,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE >
             if (act_e) {
                 pencil<N, DIM>(a, nb, Ds + tq * NVP * PSZ, Fs + tq * NVP * FSZ, X, d, q, ei, ej, ek, (size_t)e, CONS,
                                bal, CONS ? bt * a.ih[d] : 0.0, lower);
-                if (d + 1 < DIM) nb = load_traces<N, DIM>(a, d + 1, a.tin_slices, ts, q, ei, ej, ek, (size_t)e, lower);
+                if (d + 1 < DIM) nb = load_traces<N, DIM>(a, bufs, d + 1, a.tin_slices, ts, q, ei, ej, ek, (size_t)e, lower);
             }
             elem_sync();
             if constexpr (MODE == M_STAGED) {
@@ -1134,7 +1174,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE >
         elem_sync();
         // traces of the new state into this element's older buffer, one
         // pencil (slice tq, line q) per thread and axis
-        const int wb = act_e ? (cload(a.ver, E + e) < cload(a.ver, (size_t)e) ? 1 : 0) : 0;
+        const int wb = bufs >> 6;
         if (act_e) {
 #pragma unroll
             for (int d = 0; d < DIM; d++) {
@@ -1181,7 +1221,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE >
             X[G::XRES] = rr;
             if (a.conv && rr < a.tol && a.conv[e] == 0xff) a.conv[e] = (unsigned char)a.sweep;
             if (a.big_out) a.big_out[e] = rr < a.tol ? 0 : 1;  // NaN: not converged
-            a.ver[(size_t)wb * E + e] = a.cur;
+            // the traces are read by the next launch on the stream
+            __hip_atomic_store(a.ver + (size_t)wb * E + e, a.cur, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         if (live && !act_e && s == 0) {  // kept state and traces
             X[G::XRES] = 0.0;
@@ -1382,7 +1423,7 @@ __global__ void __launch_bounds__(256) k_mrestart(const float* __restrict__ d_ol
 #pragma unroll
             for (int t = 0; t < T; t++) D[((size_t)t * NVP + v) * slabE + eo] = x;
         }
-        wb = ver[E + e] < ver[e] ? 1 : 0;
+        wb = older(ver[e], ver[E + e]);
     }
     __syncthreads();
     if (live && s == 0) next_flags[e] = go ? 1 : 0;
