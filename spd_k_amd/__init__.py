@@ -176,7 +176,9 @@ class Context:
                 o.fv_centers[d] = hold(c)
                 o.fv_ncells[d] = len(c)
         self.ctx = ctypes.c_void_p()
-        stream = torch.cuda.current_stream().cuda_stream
+        # the default stream's handle is 0, which spdk_ctx_create takes for a stream of the context's own, unordered
+        # with torch's work: hipStreamLegacy (1) names the default stream
+        stream = torch.cuda.current_stream().cuda_stream or 1
         check(lib().spdk_ctx_create(ctypes.byref(prm), ctypes.byref(o), ctypes.c_void_p(stream), ctypes.byref(self.ctx)),
               "spdk_ctx_create")
 

@@ -61,6 +61,23 @@ def state(shape, rng, positive=True):
     return np.ascontiguousarray(a)
 
 
+@pytest.mark.parametrize("default", [True, False])
+def test_context_runs_on_the_current_stream(default):
+    """A kernel entry sees what torch enqueued before it on the stream the context was created on, the default one included."""
+    act, N = (1, 1, 0), (5, 3, 1)
+    with torch.cuda.stream(torch.cuda.default_stream() if default else torch.cuda.Stream()):
+        c, _, _, _ = ctx_for(3, act, N=N)
+        U = dev(state(sd_shape(1, 6, N, 4, act), np.random.default_rng(3)))
+        A, W, V = torch.ones_like(U), torch.zeros_like(U), torch.zeros_like(U)
+        c.compute_primitives(U, V)
+        torch.cuda.synchronize()
+        torch.cuda._sleep(20_000_000)  # some 10 ms
+        A.copy_(U)
+        c.compute_primitives(A, W)
+        assert np.array_equal(host(W), host(V))
+        c.close()
+
+
 GEOMS = [((1, 1, 1), (3, 4, 2)), ((1, 1, 0), (5, 3, 1)), ((1, 0, 0), (6, 1, 1))]
 
 
