@@ -105,12 +105,6 @@ struct IArgs {
     ConstDiv dh[3];       // division by h
 };
 
-template <class R>
-__device__ __forceinline__ R upwind(R l, R r, double v) {
-    if (v == 0) return R(0.5) * (l + r);
-    return v > 0 ? l : r;
-}
-
 // Raw-E slab of component e (all slices): T x nel x epts(e), components
 // back to back.
 template <int N, int D, int T>

@@ -105,7 +105,7 @@ struct MT {
         return j < EPW ? tid / 64 * EPW + j : EPB;
     }
     static __device__ __forceinline__ int pt_of(int tid) { return (tid % 64) % TPE; }
-    static constexpr int LDS_BYTES = EPB * ELEM_BYTES > BLOCK * 8 ? EPB * ELEM_BYTES : BLOCK * 8;
+    static constexpr int LDS_BYTES = EPB * ELEM_BYTES;
     // waves per SIMD the sweeps are compiled for: as many as the blocks' LDS lets in, at most 3 (168 VGPRs)
     static constexpr int WAVES = 163840 / LDS_BYTES * BLOCK / 256 < 3 ? 163840 / LDS_BYTES * BLOCK / 256 : 3;
     static_assert(TPE <= 64 && EPB >= 1 && BLOCK <= 256, "tile does not fit a workgroup");
