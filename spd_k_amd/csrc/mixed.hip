@@ -347,13 +347,12 @@ __device__ __forceinline__ void face_sources(const MArgs& a, int d, int ei, int 
     el1 = ebase + (size_t)(ed >= Nd - 2 ? (per ? 1 : Nd - 2) : ed + 1) * stride;
 }
 
-// Buffers of element e's traces in this sweep, one bit each: bit 2 d + i that
-// which holds the newest of its i-th source along axis d, bit 6 that which it
-// writes. The sweep that reads the versions also writes them (each workgroup
-// its own elements'), hence atomic accesses; all are loaded before the first
-// is looked at, and before the element's state (a wait for a load is a wait
-// for every earlier one, and for every earlier store). UNI: e is the same in
-// every lane, and the bits go to a scalar register.
+// Buffers of element e's traces in a predictor sweep, one bit each: bit 2 d + i
+// that which holds the newest of its i-th source along axis d, bit 6 that which
+// it writes. The sweep also writes the versions (each workgroup its own
+// elements'), hence atomic accesses, and all of them before the element's state:
+// a wait for a vector load is one for every earlier load and store. UNI: e is
+// the same in every lane, and the bits go to a scalar register.
 template <int DIM, bool UNI>
 __device__ __forceinline__ int trace_buffers(const MArgs& a, int ei, int ej, int ek, size_t e) {
     int v[2 * DIM + 1][2];
@@ -383,11 +382,12 @@ __device__ __forceinline__ int trace_buffers(const MArgs& a, int ei, int ej, int
 struct Nbr { float v0[NVP], v1[NVP]; };
 
 // Loads the traces pencil (d, slice ts of ns, q) of element e reads, from the
-// buffers bufs (trace_buffers). Ghost fills: periodic
+// buffers bufs (trace_buffers), or (LOOKUP) by the versions, in a sweep that
+// leaves them as they are. Ghost fills: periodic
 // copies the opposite interior element, gradfree / reflective the adjacent one
 // (src/boundary.cpp:48-113). lower_face_only: v1 only where the lower face
 // takes it (the right ghost).
-template <int N, int DIM>
+template <int N, int DIM, bool LOOKUP>
 __device__ __forceinline__ Nbr load_traces(const MArgs& a, int bufs, int d, int ns, int ts, int q, int ei, int ej, int ek,
                                            size_t e, bool lower_face_only = false) {
     constexpr int NT = MT<N, DIM>::NT;
@@ -400,8 +400,11 @@ __device__ __forceinline__ Nbr load_traces(const MArgs& a, int bufs, int d, int 
     const int sid1 = ed >= Nd - 2 ? (per ? 0 : 1) : 0;
     const float* bA = d == 0 ? a.trb[0][0] : (d == 1 ? a.trb[0][1] : a.trb[0][2]);
     const float* bB = d == 0 ? a.trb[1][0] : (d == 1 ? a.trb[1][1] : a.trb[1][2]);
-    const float* t0 = (bufs >> (2 * d)) & 1 ? bB : bA;
-    const float* t1 = (bufs >> (2 * d + 1)) & 1 ? bB : bA;
+    auto in_b = [&](int i, size_t el) {
+        return LOOKUP ? newest(cload(a.ver, el), cload(a.ver, (size_t)a.E + el), a.cur) : (bufs >> (2 * d + i)) & 1;
+    };
+    const float* t0 = in_b(0, el0) ? bB : bA;
+    const float* t1 = in_b(1, el1) ? bB : bA;
     Nbr n;
 #pragma unroll
     for (int v = 0; v < NVP; v++) {
@@ -999,7 +1002,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE >
 
     // The first sweep reads the step start's traces (buffer A, version 0) and writes B.
     int bufs = 1 << 6;
-    if (MODE != M_START && act_e) bufs = trace_buffers<DIM, TPE == 64>(a, ei, ej, ek, (size_t)e);
+    if (MODE == M_PRED && act_e) bufs = trace_buffers<DIM, TPE == 64>(a, ei, ej, ek, (size_t)e);
 
     // The loads of the element's state and of the first axis' traces go out
     // together; the mean state is prepared while they are in flight.
@@ -1017,8 +1020,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE >
     // the face integrals read faces 0..M-2 only, unless the x flux points are written as well
     const bool lower = MODE == M_STAGED || (MODE == M_FACES && !a.F_x);
     Nbr nb;
-    if (MODE != M_START && act_e) nb = load_traces<N, DIM>(a, bufs, 0, a.tin_slices, ts, q, ei, ej, ek, (size_t)e, lower);
-    if (MODE == M_START && act_e && s < DIM * NT) nb = load_traces<N, DIM>(a, bufs, s / NT, 1, 0, q, ei, ej, ek, (size_t)e);
+    if (MODE != M_START && act_e) nb = load_traces<N, DIM, !PRED>(a, bufs, 0, a.tin_slices, ts, q, ei, ej, ek, (size_t)e, lower);
+    if (MODE == M_START && act_e && s < DIM * NT) nb = load_traces<N, DIM, !PRED>(a, bufs, s / NT, 1, 0, q, ei, ej, ek, (size_t)e);
 
     if (live)
         for (int v = s; v < NVP; v += TPE) X[v] = cload(a.mu, (size_t)v * E + e);
@@ -1066,7 +1069,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE >
         if (act_e)
             for (int task = s; task < DIM * NT; task += TPE) {  // more than TPE only for p = 1 in 3-D
                 const int d = task / NT, qq = task % NT;
-                if (task != s) nb = load_traces<N, DIM>(a, bufs, d, 1, 0, qq, ei, ej, ek, (size_t)e);
+                if (task != s) nb = load_traces<N, DIM, !PRED>(a, bufs, d, 1, 0, qq, ei, ej, ek, (size_t)e);
                 pencil<N, DIM>(a, nb, Ds, Fs + d * NVP * FSZ, X, d, qq, ei, ej, ek, (size_t)e, false, bal, 0.0);
             }
         elem_sync();
@@ -1091,7 +1094,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(MODE >
             if (act_e) {
                 pencil<N, DIM>(a, nb, Ds + tq * NVP * PSZ, Fs + tq * NVP * FSZ, X, d, q, ei, ej, ek, (size_t)e, CONS,
                                bal, CONS ? bt * a.ih[d] : 0.0, lower);
-                if (d + 1 < DIM) nb = load_traces<N, DIM>(a, bufs, d + 1, a.tin_slices, ts, q, ei, ej, ek, (size_t)e, lower);
+                if (d + 1 < DIM) nb = load_traces<N, DIM, !PRED>(a, bufs, d + 1, a.tin_slices, ts, q, ei, ej, ek, (size_t)e, lower);
             }
             elem_sync();
             if constexpr (MODE == M_STAGED) {
