@@ -29,7 +29,7 @@ constexpr int kMaxT = 8;
 
 // Waves per SIMD the sweeps are compiled for (FACES: 3). At 4 (128 registers)
 // the 3-D p=3 sweeps spill 2 to 10 registers and still gain over 3: predictor
-// 5.58 -> 5.25 ms, corrector 4.61 -> 4.41 ms at 64^3 (4.6 and 4.4 since the
+// 5.58 -> 5.25 ms, corrector 4.61 -> 4.41 ms at 64^3 (4.6 and 4.5 since the
 // matrices come by scalar loads), 2-D p=3 predictor
 // 0.295 -> 0.239 ms at 256^2.
 #ifndef SPDK_SWEEP_WAVES
@@ -158,7 +158,9 @@ __device__ __forceinline__ void fv_faces(const SweepArgs& a, double* scr, double
     // its first contraction), and after one barrier per slice the block's four
     // elements (consecutive along x) write 16 consecutive faces per row, whole
     // 128-byte rows. With four barriers per axis instead, the waves waited 52%
-    // of their time: 62 x 66 x 61 elements 5.92 -> 5.20 ms.
+    // of their time: 62 x 66 x 61 elements 5.92 -> 5.20 ms. At the other 3-D
+    // degrees an element is not a wave (8 points: 8 to a wave; 27: across waves),
+    // and two block barriers per axis stay.
     constexpr bool WAVE = TPE == 64 && DIM == 3;
     static_assert(!WAVE || TPE <= FSZ, "the faces fit over the fluxes");
     const double* S = a.S2C;

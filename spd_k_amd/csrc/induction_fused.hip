@@ -74,8 +74,11 @@ struct IG {
 // A workgroup's tile: as many whole elements as its threads cover with one
 // edge point of a component per thread, so that phases A and C run without a
 // loop over points and phase B keeps one face-B point per component and
-// thread (256 threads: 10 elements of 2-D p=3, 250 threads busy; the 100 edge
-// points of 3-D p=3 fit 3 times into 320).
+// thread (256 threads: 10 elements of 2-D p=3, 250 threads busy). The 100 edge
+// points of 3-D p=3 fit 3 times into 320 threads and twice, 200 busy, into 256;
+// a step with 320 and with 256, us: FP64 10 x 11 x 12 elements 65 and 70,
+// 20^3 204 and 200, 56^3 4589 and 4338; mixed 14 x 15 x 16 71 and 74,
+// 40 x 37 x 43 1096 and 992. So 320 is the better for meshes below some 20^3.
 template <int N, int D, int T, class R>
 struct Tile {
     using G = IG<N, D>;

@@ -925,13 +925,13 @@ __device__ __forceinline__ void divergence(const MArgs& a, const float* Fs, int 
 
 // One sweep. At 98^3 elements, p=3, M_PRED moves 25.4 GB (state and traces read
 // and written, d_old read) in 6.6 ms, 3.8 TB/s where a copy reaches 4.4; M_START
-// 15.7 GB in 4.4 ms; M_CORR 20 GB in 6.5 ms, 62% of it issuing FP64 and FP32
+// 15.7 GB in 4.6 ms; M_CORR 20 GB in 6.6 ms, 62% of it issuing FP64 and FP32
 // vector instructions; M_STAGED 40 GB, of them 32 written, in 12.0 ms (7.5, 7.5,
 // 10.6 and 14.7 ms before the following, same values):
-//   - the matrices, means and versions come through the constant address
-//     space (cload): the compiler cannot show that the kernel's stores leave
-//     them alone, and otherwise loads them per lane again after each fence
-//     (a third of the time of M_PRED);
+//   - the matrices and means come through the constant address space (cload):
+//     the compiler cannot show that the kernel's stores leave them alone, and
+//     otherwise loads them per lane again after each fence (a third of the time
+//     of M_PRED); the trace versions too, except in M_PRED, which writes them;
 //   - the element index is wave-uniform at 64 points per element, so its
 //     neighbours' addresses are scalar;
 //   - the axes are unrolled, apart from the first sweep's single round;

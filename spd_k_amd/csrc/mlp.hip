@@ -245,6 +245,8 @@ __global__ void __launch_bounds__(256) k_gemm_wgrad(WgradP p) {
 // bias gradient) added to gb. A thread owns one column and kMseRows rows, so a
 // column's sum and the workgroup's loss cost one atomic each (one atomic on
 // the loss per 256 values, from 20,480 workgroups, took 263 us at 4096 x 1280).
+// The atomics add in any order: bias gradients, like the weights', differ from
+// run to run in their last bits.
 constexpr int kMseRows = 32;
 __global__ void __launch_bounds__(256) k_mse(const float* Y, long ldy, const float* T, long ldt, int M, int dout,
                                              int dpad, float inv_count, bf16* dYb, float* gb, float* loss) {
